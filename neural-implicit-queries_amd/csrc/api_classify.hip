@@ -6,7 +6,7 @@ namespace {
 
 // Launch k_classify for (KIND, V) at template width W with tile T, compiled
 // for the activation set AS.
-template <int KIND, int V, int W, class T = TileCfg<W>, int AS = ACTS_ALL>
+template <int KIND, int V, int W, class T, int AS = ACTS_ALL>
 niq_status launch_classify_w(const niq_model* m, const ClassifyArgs& a, long long max_n, hipStream_t s) {
   constexpr int NB = T::NB, NW = T::NW;
   constexpr int OCC = T::OCC ? std::min(T::OCC, LdsOcc<Planes<KIND, V, 0>::R, NB, NW, W>::value) : 0;
@@ -32,11 +32,12 @@ niq_status launch_classify_w(const niq_model* m, const ClassifyArgs& a, long lon
     }
     return NIQ_OK;
   } else {
-    auto k = k_classify<KIND, V, NB, NW, W, false, OCC, AS>;
-    const long long tiles = (max_n + NB - 1) / NB;
-    if (tiles == 0) return NIQ_OK;
-    const unsigned g = tile_grid(tiles, persistent_blocks(k, NW * 64));
-    hipLaunchKernelGGL(k, dim3(g), dim3(NW * 64), 0, s, m->dev, a);
+    constexpr int TPW = T::TPW;
+    auto k = k_classify<KIND, V, NB, NW, W, false, OCC, AS, TPW>;
+    const long long wgs = (max_n + NB * TPW - 1) / (NB * TPW);
+    if (wgs == 0) return NIQ_OK;
+    const unsigned g = tile_grid(wgs, persistent_blocks(k, TPW * NW * 64));
+    hipLaunchKernelGGL(k, dim3(g), dim3(TPW * NW * 64), 0, s, m->dev, a);
     HIPCHK(hipGetLastError());
     if (a.recheck_tol > 0.f) {
       auto k64 = k_recheck_fp64<KIND, V, W>;
@@ -48,10 +49,23 @@ niq_status launch_classify_w(const niq_model* m, const ClassifyArgs& a, long lon
   }
 }
 
+// k_classify in the default tile, compiled for the activation set AS.
+template <int KIND, int V, int AS>
+niq_status launch_classify_acts(const niq_model* m, const ClassifyArgs& a, long long max_n, hipStream_t s) {
+  switch (m->wt) {
+    case 32: return launch_classify_w<KIND, V, 32, BoxTile<32>, AS>(m, a, max_n, s);
+    case 64: return launch_classify_w<KIND, V, 64, BoxTile<64>, AS>(m, a, max_n, s);
+    case 128: return launch_classify_w<KIND, V, 128, BoxTile<128>, AS>(m, a, max_n, s);
+    case 256: return launch_classify_w<KIND, V, 256, BoxTile<256>, AS>(m, a, max_n, s);
+    case 512: return launch_classify_w<KIND, V, 512, BoxTile<512>, AS>(m, a, max_n, s);
+  }
+  return fail(NIQ_ERR_UNSUPPORTED, "width");
+}
+
 // Tile variants for the forms trees use most (interval and affine_fixed over
-// 3 box vectors): 1 (and 0) TileCfg, 2 TileCfgAlt, 3 TileCfgRegs, 4
+// 3 box vectors): 1 (and 0) BoxTile, 2 TileCfgAlt, 3 TileCfgRegs, 4
 // TileCfgWide (16 boxes, the most waves: the narrowest width tile per wave);
-// the other forms always take TileCfg.  The waves of a tile split the layer's
+// the other forms always take BoxTile.  The waves of a tile split the layer's
 // feature tiles among them, so the wave count sets the width tile each wave
 // contracts (W / 16 / NW tiles of 16 features).
 template <int KIND, int V>
@@ -61,6 +75,7 @@ niq_status launch_classify(const niq_model* m, const ClassifyArgs& a, long long 
   // the same order, bit-identical results)
   if (variant == 0 && max_n <= 32LL * num_cus()) {
     switch (m->wt) {
+      case 32: return launch_classify_w<KIND, V, 32, TileCfgWide<32>>(m, a, max_n, s);
       case 64: return launch_classify_w<KIND, V, 64, TileCfgWide<64>>(m, a, max_n, s);
       case 128: return launch_classify_w<KIND, V, 128, TileCfgWide<128>>(m, a, max_n, s);
       case 256: return launch_classify_w<KIND, V, 256, TileCfgWide<256>>(m, a, max_n, s);
@@ -72,6 +87,7 @@ niq_status launch_classify(const niq_model* m, const ClassifyArgs& a, long long 
   if constexpr (has_alt) {
     if (variant == 2) {
       switch (m->wt) {
+        case 32: return launch_classify_w<KIND, V, 32, TileCfgAlt<32>>(m, a, max_n, s);
         case 64: return launch_classify_w<KIND, V, 64, TileCfgAlt<64>>(m, a, max_n, s);
         case 128: return launch_classify_w<KIND, V, 128, TileCfgAlt<128>>(m, a, max_n, s);
         case 256: return launch_classify_w<KIND, V, 256, TileCfgAlt<256>>(m, a, max_n, s);
@@ -81,6 +97,7 @@ niq_status launch_classify(const niq_model* m, const ClassifyArgs& a, long long 
     }
     if (variant == 3) {
       switch (m->wt) {
+        case 32: return launch_classify_w<KIND, V, 32, TileCfgRegs<32>>(m, a, max_n, s);
         case 64: return launch_classify_w<KIND, V, 64, TileCfgRegs<64>>(m, a, max_n, s);
         case 128: return launch_classify_w<KIND, V, 128, TileCfgRegs<128>>(m, a, max_n, s);
         case 256: return launch_classify_w<KIND, V, 256, TileCfgRegs<256>>(m, a, max_n, s);
@@ -90,6 +107,7 @@ niq_status launch_classify(const niq_model* m, const ClassifyArgs& a, long long 
     }
     if (variant == 4) {   // the narrowest width tile: one 16-feature tile per wave (at W <= 256)
       switch (m->wt) {
+        case 32: return launch_classify_w<KIND, V, 32, TileCfgWide<32>>(m, a, max_n, s);
         case 64: return launch_classify_w<KIND, V, 64, TileCfgWide<64>>(m, a, max_n, s);
         case 128: return launch_classify_w<KIND, V, 128, TileCfgWide<128>>(m, a, max_n, s);
         case 256: return launch_classify_w<KIND, V, 256, TileCfgWide<256>>(m, a, max_n, s);
@@ -99,26 +117,14 @@ niq_status launch_classify(const niq_model* m, const ClassifyArgs& a, long long 
     }
   }
   if constexpr (KIND == 0 && (V == 0 || V == 3)) {
-    // ReLU models, in the forms trees use (the default tile): a kernel
-    // compiled for ReLU alone, the same sums and rules (bit-identical), fewer
-    // registers
-    if (m->relu_only) {
-      switch (m->wt) {
-        case 64: return launch_classify_w<KIND, V, 64, TileCfg<64>, ACTS_RELU>(m, a, max_n, s);
-        case 128: return launch_classify_w<KIND, V, 128, TileCfg<128>, ACTS_RELU>(m, a, max_n, s);
-        case 256: return launch_classify_w<KIND, V, 256, TileCfg<256>, ACTS_RELU>(m, a, max_n, s);
-        case 512: return launch_classify_w<KIND, V, 512, TileCfg<512>, ACTS_RELU>(m, a, max_n, s);
-      }
-      return fail(NIQ_ERR_UNSUPPORTED, "width");
-    }
+    // Models of one activation, in the forms trees use (the default tile): a
+    // kernel compiled for it alone, the same sums and rules (bit-identical),
+    // fewer registers
+    if (m->relu_only) return launch_classify_acts<KIND, V, ACTS_RELU>(m, a, max_n, s);
+    if (m->tanh_only) return launch_classify_acts<KIND, V, ACTS_TANH>(m, a, max_n, s);
+    if (m->elu_only) return launch_classify_acts<KIND, V, ACTS_ELU>(m, a, max_n, s);
   }
-  switch (m->wt) {
-    case 64: return launch_classify_w<KIND, V, 64>(m, a, max_n, s);
-    case 128: return launch_classify_w<KIND, V, 128>(m, a, max_n, s);
-    case 256: return launch_classify_w<KIND, V, 256>(m, a, max_n, s);
-    case 512: return launch_classify_w<KIND, V, 512>(m, a, max_n, s);
-  }
-  return fail(NIQ_ERR_UNSUPPORTED, "width");
+  return launch_classify_acts<KIND, V, ACTS_ALL>(m, a, max_n, s);
 }
 
 // The weak-SDF test: one point plane, any number of box vectors.
@@ -139,6 +145,7 @@ niq_status launch_classify_sdf(const niq_model* m, const niq_eval_cfg* cfg, Clas
   if (a.recheck_tol > 0.f) return fail(NIQ_ERR_UNSUPPORTED, "the sdf mode has no FP64 re-test");
   a.lipschitz = cfg->sdf_lipschitz;
   switch (m->wt) {
+    case 32: return launch_classify_sdf_w<32>(m, a, max_n, s);
     case 64: return launch_classify_sdf_w<64>(m, a, max_n, s);
     case 128: return launch_classify_sdf_w<128>(m, a, max_n, s);
     case 256: return launch_classify_sdf_w<256>(m, a, max_n, s);
@@ -239,16 +246,16 @@ niq_status classify_with_recheck(const niq_model* m, const niq_eval_cfg* cfg, in
 namespace {
 template <class T, int W>
 void shape_of(int R, int* nb, int* nw, int* occ) {
-  *nb = T::NB; *nw = T::NW;
-  const int wgs = (int)((size_t)kLdsLimit / ((size_t)R * T::NB * W * 4));
-  const int lds = std::max(1, std::min(4, wgs * T::NW / 4));
+  *nb = T::NB * T::TPW; *nw = T::NW * T::TPW;
+  const int wgs = (int)((size_t)kLdsLimit / ((size_t)R * *nb * W * 4));
+  const int lds = std::max(1, std::min(4, wgs * *nw / 4));
   *occ = T::OCC ? std::min(T::OCC, lds) : lds;
 }
 template <int W>
 niq_status tile_shape_w(int which, int variant, int* nb, int* nw, int* occ) {
   if (which == 0) {   // plain FP32 classify, affine_fixed over 3 box vectors (5 planes)
     switch (variant) {
-      case 0: case 1: shape_of<TileCfg<W>, W>(5, nb, nw, occ); return NIQ_OK;
+      case 0: case 1: shape_of<BoxTile<W>, W>(5, nb, nw, occ); return NIQ_OK;
       case 2: shape_of<TileCfgAlt<W>, W>(5, nb, nw, occ); return NIQ_OK;
       case 3: shape_of<TileCfgRegs<W>, W>(5, nb, nw, occ); return NIQ_OK;
       case 4: shape_of<TileCfgWide<W>, W>(5, nb, nw, occ); return NIQ_OK;
@@ -271,6 +278,7 @@ extern "C" {
 niq_status niq_tile_shape(int which, int variant, int width, int* nb, int* nw, int* occ) {
   if (!nb || !nw || !occ) return fail(NIQ_ERR_INVALID, "null output");
   switch (template_width(width)) {
+    case 32: return tile_shape_w<32>(which, variant, nb, nw, occ);
     case 64: return tile_shape_w<64>(which, variant, nb, nw, occ);
     case 128: return tile_shape_w<128>(which, variant, nb, nw, occ);
     case 256: return tile_shape_w<256>(which, variant, nb, nw, occ);
@@ -308,6 +316,7 @@ niq_status niq_eval_points(const niq_model* m, const float* x, int64_t n, int d,
   if (n < 0 || (n > 0 && (!x || !out))) return fail(NIQ_ERR_INVALID, "bad buffers");
   hipStream_t s = (hipStream_t)stream;
   switch (m->wt) {
+    case 32: return launch_points_w<32>(m, x, d, n, out, s);
     case 64: return launch_points_w<64>(m, x, d, n, out, s);
     case 128: return launch_points_w<128>(m, x, d, n, out, s);
     case 256: return launch_points_w<256>(m, x, d, n, out, s);

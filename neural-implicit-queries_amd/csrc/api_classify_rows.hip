@@ -52,7 +52,7 @@ niq_status launch_rows(const niq_model* m, const niq_eval_cfg* cfg, const Classi
   const int variant = cfg ? cfg->variant : 0;
   if (variant == 2) {
     switch (m->wt) {
-      case 64: return launch_rows_w<64, MODE, RowsOcc<64>::value, RowsCfg<64>::CH / 2>(m, cfg, a, max_n, s);
+      case 32: case 64: return launch_rows_w<64, MODE, RowsOcc<64>::value, RowsCfg<64>::CH / 2>(m, cfg, a, max_n, s);
       case 128: return launch_rows_w<128, MODE, RowsOcc<128>::value, RowsCfg<128>::CH / 2>(m, cfg, a, max_n, s);
       case 256: return launch_rows_w<256, MODE, RowsOcc<256>::value, RowsCfg<256>::CH / 2>(m, cfg, a, max_n, s);
       case 512: return launch_rows_w<512, MODE, RowsOcc<512>::value, RowsCfg<512>::CH / 2>(m, cfg, a, max_n, s);
@@ -61,12 +61,12 @@ niq_status launch_rows(const niq_model* m, const niq_eval_cfg* cfg, const Classi
   }
   if (variant == 3) {
     switch (m->wt) {
-      case 64: return launch_rows_w<64, MODE, 2>(m, cfg, a, max_n, s);
+      case 32: case 64: return launch_rows_w<64, MODE, 2>(m, cfg, a, max_n, s);
       case 128: return launch_rows_w<128, MODE, 2>(m, cfg, a, max_n, s);
     }
   }
   switch (m->wt) {
-    case 64: return launch_rows_w<64, MODE>(m, cfg, a, max_n, s);
+    case 32: case 64: return launch_rows_w<64, MODE>(m, cfg, a, max_n, s);
     case 128: return launch_rows_w<128, MODE>(m, cfg, a, max_n, s);
     case 256: return launch_rows_w<256, MODE>(m, cfg, a, max_n, s);
     case 512: return launch_rows_w<512, MODE>(m, cfg, a, max_n, s);
@@ -101,7 +101,7 @@ static void rows_shape_w(int variant, int* ch, int* nw, int* occ) {
 niq_status rows_tile_shape(int variant, int wt, int* ch, int* nw, int* occ) {
   if (variant < 0 || variant > 4) return fail(NIQ_ERR_INVALID, "unknown variant");   // 4 runs the default
   switch (wt) {
-    case 64: rows_shape_w<64>(variant, ch, nw, occ); return NIQ_OK;
+    case 32: case 64: rows_shape_w<64>(variant, ch, nw, occ); return NIQ_OK;
     case 128: rows_shape_w<128>(variant, ch, nw, occ); return NIQ_OK;
     case 256: rows_shape_w<256>(variant, ch, nw, occ); return NIQ_OK;
     case 512: rows_shape_w<512>(variant, ch, nw, occ); return NIQ_OK;

@@ -33,6 +33,7 @@ niq_status launch_cp_round_kv(const niq_model* m, CpState* S, const CpArgs& a, h
     // (bit-identical; fewer registers, so more workgroups per CU)
     if (m->relu_only) {
       switch (m->wt) {
+        case 32: return launch_cp_round_w<KIND, V, 32, ACTS_RELU>(m, S, a, s);
         case 64: return launch_cp_round_w<KIND, V, 64, ACTS_RELU>(m, S, a, s);
         case 128: return launch_cp_round_w<KIND, V, 128, ACTS_RELU>(m, S, a, s);
         case 256: return launch_cp_round_w<KIND, V, 256, ACTS_RELU>(m, S, a, s);
@@ -42,6 +43,7 @@ niq_status launch_cp_round_kv(const niq_model* m, CpState* S, const CpArgs& a, h
     }
     if (m->tanh_only) {
       switch (m->wt) {
+        case 32: return launch_cp_round_w<KIND, V, 32, ACTS_TANH>(m, S, a, s);
         case 64: return launch_cp_round_w<KIND, V, 64, ACTS_TANH>(m, S, a, s);
         case 128: return launch_cp_round_w<KIND, V, 128, ACTS_TANH>(m, S, a, s);
         case 256: return launch_cp_round_w<KIND, V, 256, ACTS_TANH>(m, S, a, s);
@@ -51,6 +53,7 @@ niq_status launch_cp_round_kv(const niq_model* m, CpState* S, const CpArgs& a, h
     }
   }
   switch (m->wt) {
+    case 32: return launch_cp_round_w<KIND, V, 32>(m, S, a, s);
     case 64: return launch_cp_round_w<KIND, V, 64>(m, S, a, s);
     case 128: return launch_cp_round_w<KIND, V, 128>(m, S, a, s);
     case 256: return launch_cp_round_w<KIND, V, 256>(m, S, a, s);
@@ -187,6 +190,7 @@ extern "C" niq_status niq_closest_point(const niq_model* m, const niq_eval_cfg* 
       hipLaunchKernelGGL(k_cp_gather, dim3(gg), dim3(256), 0, s, S, a);
       if ((st = classify_dispatch(m, cfg, 3, ca, B, s))) break;
       switch (m->wt) {
+        case 32: st = launch_points_dev_w<32>(m, a.pts, &S->n, 7, 7LL * B, a.vals, s); break;
         case 64: st = launch_points_dev_w<64>(m, a.pts, &S->n, 7, 7LL * B, a.vals, s); break;
         case 128: st = launch_points_dev_w<128>(m, a.pts, &S->n, 7, 7LL * B, a.vals, s); break;
         case 256: st = launch_points_dev_w<256>(m, a.pts, &S->n, 7, 7LL * B, a.vals, s); break;
@@ -381,6 +385,7 @@ niq_status launch_points_dev_w(const niq_model* m, const float* x, const int* n_
 niq_status niqi::points_dev(const niq_model* m, const float* x, const int* n_dev, int mult, long long max_n,
                             float* out, hipStream_t s) {
   switch (m->wt) {
+    case 32: return launch_points_dev_w<32>(m, x, n_dev, mult, max_n, out, s);
     case 64: return launch_points_dev_w<64>(m, x, n_dev, mult, max_n, out, s);
     case 128: return launch_points_dev_w<128>(m, x, n_dev, mult, max_n, out, s);
     case 256: return launch_points_dev_w<256>(m, x, n_dev, mult, max_n, out, s);

@@ -77,9 +77,11 @@ niq_status niq_model_create(int n_layers, const int* dims, const int* acts, cons
   // hidden layers ReLU or the identity: the ReLU-only classify kernels apply
   m->relu_only = true;
   m->tanh_only = true;
+  m->elu_only = true;
   for (int i = 0; i + 1 < n_layers; ++i) {
     if (acts[i] != NIQ_ACT_RELU && acts[i] != NIQ_ACT_NONE) m->relu_only = false;
     if (acts[i] != NIQ_ACT_TANH && acts[i] != NIQ_ACT_NONE) m->tanh_only = false;
+    if (acts[i] != NIQ_ACT_ELU && acts[i] != NIQ_ACT_NONE) m->elu_only = false;
   }
   hipError_t e = hipMalloc(&m->weights, total);
   if (e == hipSuccess) e = hipMemcpy(m->weights, host.data(), total, hipMemcpyHostToDevice);
@@ -182,7 +184,7 @@ niq_status niq_model_create(int n_layers, const int* dims, const int* acts, cons
                           (1.0 + std::ldexp(1.0, -15)));
     }
     m->host16.wmax = wmax16;
-    m->wt16 = template_width(wmax16);
+    m->wt16 = std::max(template_width(wmax16), 64);   // its narrowest template
     e = hipMalloc(&m->weights16, t16);
     if (e == hipSuccess) e = hipMemcpy(m->weights16, h16.data(), t16, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&m->dev16), sizeof(DevModelBf16));

@@ -38,6 +38,7 @@ niq_status launch_rays_w(const DevModel* models, const RayArgs& a, long long n_r
 template <int KIND, int V, int VAR, int AS = ACTS_ALL>
 niq_status launch_rays_v(int wt, const DevModel* models, const RayArgs& a, long long n_rays, hipStream_t s) {
   switch (wt) {
+    case 32: return launch_rays_w<KIND, V, 32, VAR, AS>(models, a, n_rays, s);
     case 64: return launch_rays_w<KIND, V, 64, VAR, AS>(models, a, n_rays, s);
     case 128: return launch_rays_w<KIND, V, 128, VAR, AS>(models, a, n_rays, s);
     case 256: return launch_rays_w<KIND, V, 256, VAR, AS>(models, a, n_rays, s);

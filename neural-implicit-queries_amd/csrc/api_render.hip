@@ -129,6 +129,7 @@ extern "C" niq_status niq_outward_normals(const niq_model* const* models, int n_
   for (int f = 0; f < n_models && st == NIQ_OK && method == NIQ_NORMALS_AUTODIFF; ++f) {
     const int* list = lists + (size_t)f * n;
     switch (models[f]->wt) {
+      case 32: st = launch_grad_normals<32>(models[f], list, counts + f, n, hit_pos, out_normals, s); break;
       case 64: st = launch_grad_normals<64>(models[f], list, counts + f, n, hit_pos, out_normals, s); break;
       case 128: st = launch_grad_normals<128>(models[f], list, counts + f, n, hit_pos, out_normals, s); break;
       case 256: st = launch_grad_normals<256>(models[f], list, counts + f, n, hit_pos, out_normals, s); break;
@@ -139,6 +140,7 @@ extern "C" niq_status niq_outward_normals(const niq_model* const* models, int n_
   for (int f = 0; f < n_models && st == NIQ_OK && method == NIQ_NORMALS_FINITE_DIFFERENCES; ++f) {
     const int* list = lists + (size_t)f * n;
     switch (models[f]->wt) {
+      case 32: st = launch_normal_eval<32>(models[f], list, counts + f, n, hit_pos, eps, vals, s); break;
       case 64: st = launch_normal_eval<64>(models[f], list, counts + f, n, hit_pos, eps, vals, s); break;
       case 128: st = launch_normal_eval<128>(models[f], list, counts + f, n, hit_pos, eps, vals, s); break;
       case 256: st = launch_normal_eval<256>(models[f], list, counts + f, n, hit_pos, eps, vals, s); break;

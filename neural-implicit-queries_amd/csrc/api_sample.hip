@@ -48,6 +48,7 @@ template <bool MASS>
 niq_status sample_eval(const niq_model* m, const SampleSrc& S, long long n, float width, unsigned char* flags,
                        Sum4* partial, int max_blocks, int* blocks_used, hipStream_t s) {
   switch (m->wt) {
+    case 32: return launch_sample_eval<32, MASS>(m, S, n, width, flags, partial, max_blocks, blocks_used, s);
     case 64: return launch_sample_eval<64, MASS>(m, S, n, width, flags, partial, max_blocks, blocks_used, s);
     case 128: return launch_sample_eval<128, MASS>(m, S, n, width, flags, partial, max_blocks, blocks_used, s);
     case 256: return launch_sample_eval<256, MASS>(m, S, n, width, flags, partial, max_blocks, blocks_used, s);

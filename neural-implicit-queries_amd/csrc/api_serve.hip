@@ -60,8 +60,8 @@ struct Request {
 };
 
 // Template widths of a ray request's functions (FP32 and precision-mode
-// copies): requests merge into one cast only at equal widths, so no function
-// runs in a wider tile than its own cast would give it.
+// copies): requests merge into one cast only in one width class, so no
+// function runs in a tile more than one step wider than its own cast's.
 int req_wt(const Request& r, bool w16) {
   int w = 0;
   for (const niq_model* m : r.models) w = std::max(w, w16 ? m->wt16 : m->wt);
@@ -74,19 +74,21 @@ int req_wt(const Request& r, bool w16) {
 // functions, options, inputs and outputs.
 bool same_cast(const Request& a, const Request& b) {
   return a.kind == REQ_RAYS && b.kind == REQ_RAYS && std::memcmp(&a.cfg, &b.cfg, sizeof(niq_eval_cfg)) == 0 &&
-         req_wt(a, false) == req_wt(b, false) && req_wt(a, true) == req_wt(b, true);
+         merge_width(req_wt(a, false)) == merge_width(req_wt(b, false)) && req_wt(a, true) == req_wt(b, true);
 }
 
 // Tree requests that can share one batched build: the same eval config (its
 // tile variants aside: they change no result, and a batch runs the default
-// tile) and build params (root boxes aside), one template width, a batchable
+// tile) and build params (root boxes aside), one width class, a batchable
 // form.
 bool same_tree_batch(const Request& a, const Request& b) {
   if (a.kind != REQ_TREE || b.kind != REQ_TREE) return false;
   niq_eval_cfg ca = a.cfg, cb = b.cfg;
   ca.variant = cb.variant = 0;
   ca.ray_variant = cb.ray_variant = 0;
-  if (std::memcmp(&ca, &cb, sizeof(niq_eval_cfg)) != 0 || a.model->wt != b.model->wt) return false;
+  if (std::memcmp(&ca, &cb, sizeof(niq_eval_cfg)) != 0 ||
+      merge_width(a.model->wt) != merge_width(b.model->wt))
+    return false;
   const niq_tree_params &p = a.tp, &q = b.tp;
   return p.split_depth == q.split_depth && p.node_terminate_thresh == q.node_terminate_thresh &&
          p.batch_process_size == q.batch_process_size && p.with_interior_nodes == q.with_interior_nodes &&

@@ -547,10 +547,12 @@ niq_status tree_batch_build(const niq_model* const* models, int ng, const niq_ev
                             const niq_tree_params* p, const float* roots, void* ws, size_t ws_bytes,
                             niq_tree_result* const* res, niq_status* tree_status, hipStream_t s) {
   if (ng < 1 || ng > kMaxTreeBatch) return fail(NIQ_ERR_INVALID, "tree batch size out of range");
-  const int wt = models[0]->wt;
+  int wt = 0;
   for (int g = 0; g < ng; ++g) {
     if (niq_status st = check_model(models[g], 3)) return st;
-    if (models[g]->wt != wt) return fail(NIQ_ERR_INVALID, "a tree batch needs one template width");
+    wt = std::max(wt, models[g]->wt);
+    if (merge_width(models[g]->wt) != merge_width(models[0]->wt))
+      return fail(NIQ_ERR_INVALID, "a tree batch needs one width class");
     if (!tree_batchable(models[g], cfg, p)) return fail(NIQ_ERR_UNSUPPORTED, "tree not batchable");
     const niq_tree_result* r = res[g];
     if (!r->unknown_lower || !r->unknown_upper || r->unknown_capacity < 0)
@@ -602,6 +604,7 @@ niq_status tree_batch_build(const niq_model* const* models, int ng, const niq_ev
   auto classify = [&](int level, long long max_n) {
     if (st != NIQ_OK) return;
     switch (wt) {
+      case 32: st = launch_classify_items<32>(form, d_items, ng, o, level, p->offset, max_n, d_pref, s); break;
       case 64: st = launch_classify_items<64>(form, d_items, ng, o, level, p->offset, max_n, d_pref, s); break;
       case 128: st = launch_classify_items<128>(form, d_items, ng, o, level, p->offset, max_n, d_pref, s); break;
       case 256: st = launch_classify_items<256>(form, d_items, ng, o, level, p->offset, max_n, d_pref, s); break;

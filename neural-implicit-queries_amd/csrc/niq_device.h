@@ -56,6 +56,15 @@ __device__ __forceinline__ const __attribute__((address_space(1))) T* as_global(
   return (const __attribute__((address_space(1))) T*)p;
 }
 
+// Calls f(0), f(1), .. f(N - 1) with constant indices.
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, I + 1>(f);
+  }
+}
+
 template <class T> struct Fm;
 template <> struct Fm<float> {
   static __device__ __forceinline__ float exp(float x) { return expf(x); }
@@ -141,9 +150,11 @@ template <class T> __device__ __forceinline__ T act_deriv(int act, T x) {
 template <class T>
 __device__ __forceinline__ void relu_rule(T lo, T hi, T& a, T& b, T& d) {
   T al = (relu_t(hi) - relu_t(lo)) / (hi - lo);
-  if (lo >= T(0)) al = T(1);
-  if (hi < T(0)) al = T(0);
-  al = clip_t(nan_to_num_t(al), T(0), T(1));
+  al = lo >= T(0) ? T(1) : al;
+  al = hi < T(0) ? T(0) : al;
+  // nan_to_num and clip in one: max(NaN, 0) is 0, and an infinity clips as
+  // the largest finite value would
+  al = clip_t(al, T(0), T(1));
   T be = (relu_t(lo) - al * lo) / T(2);
   a = al; b = be; d = be;
 }
@@ -216,12 +227,17 @@ __device__ __forceinline__ void tanh_rule(T lo, T hi, T& a, T& b, T& d) {
   al = (hi > lo) ? al : dl;
   al = clip_t(nan_to_num_t(al), T(0), T(1));
   T xs = Fm<T>::atanh(Fm<T>::sqrt(T(1) - al));
-  T locs[4] = {lo, hi, xs, -xs};
+  // Each location clamps to itself, lo or hi, whose tanh is known (tanh is odd
+  // bit for bit), so the four values take one more tanh instead of four.
+  const T ts = Fm<T>::tanh(xs);
+  const T locs[4] = {lo, hi, xs, -xs};
+  const T tans[4] = {tl, tu, ts, -ts};
   T rl = T(INFINITY), ru = T(-INFINITY);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    T x = Fm<T>::min(Fm<T>::max(locs[i], lo), hi);
-    T v = Fm<T>::tanh(x) - al * x;
+    const T x = Fm<T>::min(Fm<T>::max(locs[i], lo), hi);
+    const T t = x == locs[i] ? tans[i] : (x == lo ? tl : tu);
+    const T v = t - al * x;
     rl = Fm<T>::min(rl, v); ru = Fm<T>::max(ru, v);
   }
   a = al; b = T(0.5) * (ru + rl); d = T(0.5) * (ru - rl);
@@ -362,19 +378,13 @@ __device__ __forceinline__ void final_bounds(const T* v, T& lo, T& hi, T& scale)
   }
 }
 
-// Activation sets a kernel is compiled for: every activation, or ReLU or TanH
-// alone (models whose hidden layers all use that one; the rules of the others
+// Activation sets a kernel is compiled for: every activation, or ReLU, TanH or
+// ELU alone (models whose hidden layers all use that one; the rules of the others
 // and their constants then take no registers).
-enum { ACTS_ALL = 0, ACTS_RELU = 1, ACTS_TANH = 2 };
+enum { ACTS_ALL = 0, ACTS_RELU = 1, ACTS_TANH = 2, ACTS_ELU = 3 };
 
-template <class PL, int KIND, int V, int AS = ACTS_ALL, class T>
+template <class PL, int KIND, int V, class T>
 __device__ __forceinline__ void apply_hidden(int act, T* v) {
-  if constexpr (AS == ACTS_RELU || AS == ACTS_TANH) {
-    // the same rule with the activation a constant (identity otherwise)
-    constexpr int A = AS == ACTS_RELU ? ACT_RELU : ACT_TANH;
-    if (act == A) apply_hidden<PL, KIND, V, ACTS_ALL>(A, v);
-    return;
-  }
   if constexpr (KIND == 0) affine_fixed_rule<V>(act, v);
   else if constexpr (KIND == 1) slope_rule<V>(act, v);
   else if constexpr (KIND == 3) {
@@ -399,6 +409,19 @@ __device__ __forceinline__ int xoff(int p, int b, int k) {
   return (p * NB + b) * WMAX + (k ^ ((b & 7) << 2));
 }
 
+// Barrier among the NW waves of a tile.  A tile of one wave needs none: its LDS
+// operations execute in order, so only the compiler must not reorder them (and
+// several such tiles may share a workgroup).
+template <int NW>
+__device__ __forceinline__ void tile_sync() {
+  if constexpr (NW == 1) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  } else {
+    __syncthreads();
+  }
+}
+
 template <class PL, int KIND, int V, int NB, int NW, int WMAX, int AS = ACTS_ALL, class Fin>
 __device__ __forceinline__ void mlp_forward(const DevModel& M, float* __restrict__ X, Fin&& fin) {
   constexpr int R = PL::R;
@@ -406,15 +429,33 @@ __device__ __forceinline__ void mlp_forward(const DevModel& M, float* __restrict
   constexpr int FTMAX = (WMAX / 16 + NW - 1) / NW;
   const int lane = threadIdx.x & 63;
   // wave-uniform, so the feature-tile tests below are scalar branches
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ln = lane & 15;
   const int lg = lane >> 4;
 
+  // The first k-block's weights of a layer: the narrow templates, which have
+  // the registers, load them before the epilogue of the layer before, so that
+  // their latency overlaps it; the others load them before the layer's first
+  // barrier.
+  constexpr bool PRE = WMAX <= 64;
+  floatx4 a_first[FTMAX];
+  auto load_first = [&](const DevLayer& Lx) {
+    const int nkb = Lx.in_pad >> 4, nft = Lx.out_pad >> 4;
+#pragma unroll
+    for (int f = 0; f < FTMAX; ++f) {
+      const int ft = wave + f * NW;
+      if (ft < nft) a_first[f] = as_global(Lx.Wp)[(size_t)(ft * nkb) * 64 + lane];
+    }
+  };
+  DevLayer Ly = M.L[0];
+  if constexpr (PRE) load_first(Ly);
+
   for (int l = 0; l < M.n_layers; ++l) {
-    const DevLayer Ly = M.L[l];
     const int nkb = Ly.in_pad >> 4;
     const int nft = Ly.out_pad >> 4;
     const bool last = (l == M.n_layers - 1);
+    if constexpr (!PRE) load_first(Ly);
+    const DevLayer Ln = M.L[last ? l : l + 1];
     floatx4 acc[FTMAX][R][BT];
 #pragma unroll
     for (int f = 0; f < FTMAX; ++f)
@@ -423,21 +464,18 @@ __device__ __forceinline__ void mlp_forward(const DevModel& M, float* __restrict
 #pragma unroll
         for (int t = 0; t < BT; ++t) acc[f][p][t] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    __syncthreads();  // layer input complete in X
+    tile_sync<NW>();  // layer input complete in X
 
     // Contraction over k-blocks of 16 inputs.  Each accumulator sums its
     // k-blocks in ascending order; the next k-block's weights (global) and
     // input fragments (LDS, unchanged until the barrier below) are loaded
     // while the current one's MFMAs run.  `FULL`: every feature tile of this
     // wave exists, so the loop carries no per-tile test.
-    auto contract = [&](auto full_tag) {
+    auto contract = [&](auto full_tag) __attribute__((always_inline)) {
       constexpr bool FULL = decltype(full_tag)::value;
       floatx4 a_nx[FTMAX];
 #pragma unroll
-      for (int f = 0; f < FTMAX; ++f) {
-        const int ft = wave + f * NW;
-        if (FULL || ft < nft) a_nx[f] = Ly.Wp[(size_t)(ft * nkb) * 64 + lane];
-      }
+      for (int f = 0; f < FTMAX; ++f) a_nx[f] = a_first[f];
       for (int kb = 0; kb < nkb; ++kb) {
         floatx4 a[FTMAX];
         floatx4 bx[R][BT];
@@ -480,7 +518,8 @@ __device__ __forceinline__ void mlp_forward(const DevModel& M, float* __restrict
     // chunking depends on the model only, not on the tile shape, so every
     // tile shape gives the same bits.
     constexpr int kKSplit = 4;
-    const bool ksplit = (nft == 1) && nkb >= 2 * kKSplit;
+    constexpr bool KSPLIT = WMAX / 16 >= 2 * kKSplit;   // whether a layer of this width can split
+    const bool ksplit = KSPLIT && (nft == 1) && nkb >= 2 * kKSplit;
     if (ksplit) {
       if (wave < kKSplit) {
         const int kb0 = wave * nkb / kKSplit, kb1 = (wave + 1) * nkb / kKSplit;
@@ -512,7 +551,18 @@ __device__ __forceinline__ void mlp_forward(const DevModel& M, float* __restrict
       contract(std::false_type{});
     }
 
-    __syncthreads();  // every wave has consumed X
+    // the epilogue's biases (and, narrow templates, the next layer's first
+    // weights, issued after them) load while the barrier is waited for
+    floatx4 bias4[FTMAX];
+#pragma unroll
+    for (int f = 0; f < FTMAX; ++f) {
+      const int ft = wave + f * NW;
+      if (ft < nft) bias4[f] = *reinterpret_cast<const __attribute__((address_space(1))) floatx4*>(
+                        as_global(Ly.bias) + ft * 16 + lg * 4);
+    }
+    if constexpr (PRE) load_first(Ln);
+
+    tile_sync<NW>();  // every wave has consumed X
 
     if (ksplit) {
       // partial sums through LDS (X is free now); wave 0 adds them in order
@@ -523,7 +573,7 @@ __device__ __forceinline__ void mlp_forward(const DevModel& M, float* __restrict
 #pragma unroll
           for (int t = 0; t < BT; ++t) Pp[(((wave - 1) * R + p) * BT + t) * 64 + lane] = acc[0][p][t];
       }
-      __syncthreads();
+      tile_sync<NW>();
       if (wave == 0) {
 #pragma unroll
         for (int w = 1; w < kKSplit; ++w)
@@ -532,37 +582,105 @@ __device__ __forceinline__ void mlp_forward(const DevModel& M, float* __restrict
 #pragma unroll
             for (int t = 0; t < BT; ++t) acc[0][p][t] += Pp[(((w - 1) * R + p) * BT + t) * 64 + lane];
       }
-      __syncthreads();  // partials read before the caller reuses X
+      tile_sync<NW>();  // partials read before the caller reuses X
     }
 
+    if (last) {
+      if (wave == 0 && lg == 0) {
 #pragma unroll
-    for (int f = 0; f < FTMAX; ++f) {
-      const int ft = wave + f * NW;
-      if (ft >= nft) continue;
-      const floatx4 bias4 = *reinterpret_cast<const floatx4*>(&Ly.bias[ft * 16 + lg * 4]);
-#pragma unroll
-      for (int t = 0; t < BT; ++t) {
-        const int b = t * 16 + ln;
-        floatx4 outv[R];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int t = 0; t < BT; ++t) {
           float v[R];
 #pragma unroll
-          for (int p = 0; p < R; ++p) v[p] = acc[f][p][t][j] + (PL::bias(p) ? bias4[j] : 0.f);
-          if (!last) {
-            apply_hidden<PL, KIND, V, AS>(Ly.act, v);
-          } else if (ft == 0 && lg == 0 && j == 0) {
-            fin(v, b);
-          }
-#pragma unroll
-          for (int p = 0; p < R; ++p) outv[p][j] = v[p];
+          for (int p = 0; p < R; ++p) v[p] = acc[0][p][t][0] + (PL::bias(p) ? bias4[0][0] : 0.f);
+          fin(v, t * 16 + ln);
         }
-        if (!last) {
+      }
+    } else {
+      // The layer's activation is chosen once per layer (uniform).  ReLU and the
+      // identity run on the accumulators, the 4 features of a lane together:
+      // their chains (a division each) have no branch between them and
+      // interleave.  (Unrolled by hand: past a size the compiler keeps
+      // `#pragma unroll` loops rolled, and the accumulators then live in
+      // scratch.)
+      auto epilogue = [&](auto act_tag) __attribute__((always_inline)) {
+        constexpr int ACT = decltype(act_tag)::value;
+        constexpr bool LIGHT = ACT == ACT_RELU || ACT == ACT_NONE;
+        static_for<FTMAX>([&](auto fc) __attribute__((always_inline)) {
+          constexpr int f = decltype(fc)::value;
+          const int ft = wave + f * NW;
+          if (ft >= nft) return;
+          static_for<BT>([&](auto tc) __attribute__((always_inline)) {
+            constexpr int t = decltype(tc)::value;
+            const int b = t * 16 + ln;
+            floatx4 outv[R];
+            static_for<4>([&](auto jc) __attribute__((always_inline)) {
+              constexpr int j = decltype(jc)::value;
+              float v[R];
 #pragma unroll
-          for (int p = 0; p < R; ++p)
-            *reinterpret_cast<floatx4*>(&X[xoff<NB, WMAX>(p, b, ft * 16 + lg * 4)]) = outv[p];
+              for (int p = 0; p < R; ++p) v[p] = acc[f][p][t][j] + (PL::bias(p) ? bias4[f][j] : 0.f);
+              if constexpr (LIGHT) apply_hidden<PL, KIND, V>(ACT, v);
+#pragma unroll
+              for (int p = 0; p < R; ++p) outv[p][j] = v[p];
+            });
+#pragma unroll
+            for (int p = 0; p < R; ++p)
+              *reinterpret_cast<floatx4*>(&X[xoff<NB, WMAX>(p, b, ft * 16 + lg * 4)]) = outv[p];
+          });
+        });
+        // The transcendental rules are hundreds of instructions per feature:
+        // unrolled over a wave's features they overflow the instruction cache
+        // and spill.  They run in a loop over the values just written (each
+        // lane reads its own back), one copy of the rule in all.
+        if constexpr (!LIGHT) {
+#pragma unroll 1
+          for (int i = 0; i < FTMAX * BT; ++i) {
+            const int ft = wave + (i / BT) * NW;
+            if (ft >= nft) break;
+            const int o = xoff<NB, WMAX>(0, (i % BT) * 16 + ln, ft * 16 + lg * 4);
+            floatx4 q[R];
+#pragma unroll
+            for (int p = 0; p < R; ++p) q[p] = *reinterpret_cast<const floatx4*>(&X[o + p * NB * WMAX]);
+            if constexpr (KIND == 2 && R == 1) {
+#pragma unroll
+              for (int j = 0; j < 4; ++j) q[0][j] = act_point(ACT, q[0][j]);
+            } else {
+              // two features at a time where the kernel has one rule only:
+              // their chains interleave (with every rule in it, they spill)
+              constexpr int JU = AS == ACTS_ALL ? 1 : 2;
+#pragma unroll 1
+              for (int j = 0; j < 4; j += JU) {
+                float v[JU][R];
+#pragma unroll
+                for (int u = 0; u < JU; ++u) {
+#pragma unroll
+                  for (int p = 0; p < R; ++p) v[u][p] = q[p][u];
+                  apply_hidden<PL, KIND, V>(ACT, v[u]);
+                }
+#pragma unroll
+                for (int p = 0; p < R; ++p)
+                  if constexpr (JU == 2) q[p] = floatx4{q[p][2], q[p][3], v[0][p], v[1][p]};
+                  else q[p] = floatx4{q[p][1], q[p][2], q[p][3], v[0][p]};
+              }
+            }
+#pragma unroll
+            for (int p = 0; p < R; ++p) *reinterpret_cast<floatx4*>(&X[o + p * NB * WMAX]) = q[p];
+          }
+        }
+      };
+      if constexpr (AS != ACTS_ALL) {
+        constexpr int A = AS == ACTS_RELU ? ACT_RELU : (AS == ACTS_TANH ? ACT_TANH : ACT_ELU);
+        if (Ly.act == A) epilogue(std::integral_constant<int, A>{});
+        else epilogue(std::integral_constant<int, ACT_NONE>{});
+      } else {
+        switch (Ly.act) {
+          case ACT_RELU: epilogue(std::integral_constant<int, ACT_RELU>{}); break;
+          case ACT_ELU: epilogue(std::integral_constant<int, ACT_ELU>{}); break;
+          case ACT_SIN: epilogue(std::integral_constant<int, ACT_SIN>{}); break;
+          case ACT_TANH: epilogue(std::integral_constant<int, ACT_TANH>{}); break;
+          default: epilogue(std::integral_constant<int, ACT_NONE>{}); break;
         }
       }
     }
+    Ly = Ln;
   }
 }

@@ -60,12 +60,17 @@ inline double gamma_n(double n, double u) { return n * u / (1.0 - n * u) * (1.0 
 
 // Template width that holds every padded layer width of a model.
 inline int template_width(int wmax) {
+  if (wmax <= 32) return 32;
   if (wmax <= 64) return 64;
   if (wmax <= 128) return 128;
   if (wmax <= 256) return 256;
   if (wmax <= 512) return 512;
   return -1;
 }
+
+// Width class by which serving requests merge into shared launches: the two
+// narrowest templates are one class (a mixed merge runs the wider of them).
+inline int merge_width(int wt) { return std::max(wt, 64); }
 
 // closest_point: rounds between host checks of the stack (up to 32 while the
 // room they need, 2 K B rows, stays small) and the stack's initial rows.
@@ -128,6 +133,7 @@ struct niq_model {
   bool bf16_ok = true;         // no FP32 subnormal weights (precision mode)
   bool relu_only = false;      // every hidden activation is ReLU
   bool tanh_only = false;      // every hidden activation is TanH
+  bool elu_only = false;       // every hidden activation is ELU
   DevModelBf16 host16;         // precision-mode copy (bf16 hi/lo/|W| weights)
   DevModelBf16* dev16 = nullptr;
   void* weights16 = nullptr;

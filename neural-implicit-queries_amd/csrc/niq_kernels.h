@@ -7,34 +7,53 @@
 
 // Workgroup shapes per padded max width: boxes per tile (NB) and waves (NW).
 // OCC: waves per SIMD the register budget is set for (0: what LDS admits).
+// Width 32 (the 32-wide nets) is a tile of one wave: its two feature tiles
+// would leave half the waves of the 64-wide tile idle at every layer, and one
+// wave needs no barrier.  100,003 boxes of an 8-layer 32-wide ReLU net: 102
+// against 157 us on the 64-wide tile; 160,000 of its rays: 17.1 against 23.5
+// ms; 400,001 of its points: 79 against 98 us.
 template <int WMAX> struct TileCfg;
+template <> struct TileCfg<32>  { static constexpr int NB = 16, NW = 1, NBP = 32, OCC = 0; };
 template <> struct TileCfg<64>  { static constexpr int NB = 32, NW = 4, NBP = 64, OCC = 0; };
 template <> struct TileCfg<128> { static constexpr int NB = 32, NW = 4, NBP = 64, OCC = 0; };
 template <> struct TileCfg<256> { static constexpr int NB = 16, NW = 8, NBP = 64, OCC = 0; };
 template <> struct TileCfg<512> { static constexpr int NB = 16, NW = 8, NBP = 64, OCC = 0; };
 
+// Tile of a classify launch.  16 boxes at widths 64 and 128, where the other
+// kernels take 32: twice the workgroups per CU, so that one's activation rules
+// (vector ALU) overlap another's contraction, and half the work in the last,
+// partly filled round.  20,011 boxes of a 128x8 TanH net: 298 against 416 us;
+// 100,003 of a 64x8 ELU net: 400 against 425 us.
+// Width 32 puts four tiles of one wave each into a workgroup (TPW).
+template <int WMAX> struct BoxTile { static constexpr int NB = 16, NW = 8, OCC = 0, TPW = 1; };
+template <> struct BoxTile<32> { static constexpr int NB = 16, NW = 1, OCC = 0, TPW = 4; };
+template <> struct BoxTile<64> { static constexpr int NB = 16, NW = 4, OCC = 0, TPW = 1; };
+
 // Alternative tiles offered to the autotuner (eval cfg variant 2): twice the
 // boxes per workgroup where LDS allows it (weights read half as often per box),
 // fewer waves per workgroup at width 512.
 template <int WMAX> struct TileCfgAlt;
-template <> struct TileCfgAlt<64>  { static constexpr int NB = 64, NW = 4, OCC = 0; };
-template <> struct TileCfgAlt<128> { static constexpr int NB = 64, NW = 8, OCC = 0; };
-template <> struct TileCfgAlt<256> { static constexpr int NB = 32, NW = 8, OCC = 0; };
-template <> struct TileCfgAlt<512> { static constexpr int NB = 16, NW = 4, OCC = 0; };
+template <> struct TileCfgAlt<32>  { static constexpr int NB = 64, NW = 4, OCC = 0, TPW = 1; };
+template <> struct TileCfgAlt<64>  { static constexpr int NB = 64, NW = 4, OCC = 0, TPW = 1; };
+template <> struct TileCfgAlt<128> { static constexpr int NB = 64, NW = 8, OCC = 0, TPW = 1; };
+template <> struct TileCfgAlt<256> { static constexpr int NB = 32, NW = 8, OCC = 0, TPW = 1; };
+template <> struct TileCfgAlt<512> { static constexpr int NB = 16, NW = 4, OCC = 0, TPW = 1; };
 
 // The default tile with a 256-register budget (eval cfg variant 3): no
 // spills, fewer resident workgroups where LDS would admit more.
 template <int WMAX> struct TileCfgRegs {
-  static constexpr int NB = TileCfg<WMAX>::NB, NW = TileCfg<WMAX>::NW, OCC = 2;
+  static constexpr int NB = BoxTile<WMAX>::NB, NW = BoxTile<WMAX>::NW, OCC = 2;
+  static constexpr int TPW = BoxTile<WMAX>::TPW;
 };
 
 // Tiles for levels too small to fill the chip: a workgroup's latency bounds
 // them, so its feature tiles are spread over more waves (one or two each).
 template <int WMAX> struct TileCfgWide;
-template <> struct TileCfgWide<64>  { static constexpr int NB = 16, NW = 4, OCC = 0; };
-template <> struct TileCfgWide<128> { static constexpr int NB = 16, NW = 8, OCC = 0; };
-template <> struct TileCfgWide<256> { static constexpr int NB = 16, NW = 16, OCC = 0; };
-template <> struct TileCfgWide<512> { static constexpr int NB = 16, NW = 16, OCC = 0; };
+template <> struct TileCfgWide<32>  { static constexpr int NB = 16, NW = 4, OCC = 0, TPW = 1; };
+template <> struct TileCfgWide<64>  { static constexpr int NB = 16, NW = 4, OCC = 0, TPW = 1; };
+template <> struct TileCfgWide<128> { static constexpr int NB = 16, NW = 8, OCC = 0, TPW = 1; };
+template <> struct TileCfgWide<256> { static constexpr int NB = 16, NW = 16, OCC = 0, TPW = 1; };
+template <> struct TileCfgWide<512> { static constexpr int NB = 16, NW = 16, OCC = 0, TPW = 1; };
 
 constexpr int kLdsLimit = 160 * 1024;
 
@@ -46,11 +65,12 @@ constexpr int kLdsLimit = 160 * 1024;
 // at width 256, also with 256 registers.  Every variant sums each (ray,
 // feature) in the same order, so the results are bit-identical.
 template <int WMAX, int VAR> struct RayTile {
-  static constexpr int NB = TileCfg<WMAX>::NB, NW = TileCfg<WMAX>::NW, OCC = VAR == 0 ? 0 : 2;
+  static constexpr int NB = TileCfg<WMAX>::NB, NW = TileCfg<WMAX>::NW, OCC = VAR == 0 ? 0 : 2, TPW = 1;
 };
-template <> struct RayTile<64, 2> { static constexpr int NB = 16, NW = 4, OCC = 2; };
-template <> struct RayTile<128, 2> { static constexpr int NB = 16, NW = 4, OCC = 2; };
-template <> struct RayTile<256, 2> { static constexpr int NB = 32, NW = 8, OCC = 2; };
+template <> struct RayTile<32, 2> { static constexpr int NB = 32, NW = 2, OCC = 2, TPW = 1; };
+template <> struct RayTile<64, 2> { static constexpr int NB = 16, NW = 4, OCC = 2, TPW = 1; };
+template <> struct RayTile<128, 2> { static constexpr int NB = 16, NW = 4, OCC = 2, TPW = 1; };
+template <> struct RayTile<256, 2> { static constexpr int NB = 32, NW = 8, OCC = 2, TPW = 1; };
 
 template <int R, int NB, int WMAX>
 struct Fits { static constexpr bool value = (size_t)R * NB * WMAX * 4 <= (size_t)kLdsLimit; };
@@ -101,56 +121,69 @@ __device__ __forceinline__ int sdf_code(float val, float rad, float lipschitz, f
 }
 
 // Fill the layer-0 input planes of one tile (features 0..15, zero padded).
+// One thread per (box, input): its box is read once and every plane's value
+// written from it.
 template <int KIND, int V, int NB, int NT, int WMAX>
 __device__ __forceinline__ void fill_box_inputs(float* X, const ClassifyArgs& a, long long i0, long long n) {
   using PL = Planes<KIND, V, 0>;
   constexpr int RB = PL::RB;
-  for (int e = threadIdx.x; e < RB * NB * 16; e += NT) {
-    const int p = e / (NB * 16);
-    const int b = (e / 16) % NB;
-    const int k = e & 15;
+#pragma unroll
+  for (int e0 = 0; e0 < NB * 16; e0 += NT) {
+    const int e = e0 + (int)threadIdx.x % NT;
+    if (NB * 16 % NT != 0 && e >= NB * 16) break;
+    const int b = e >> 4, k = e & 15;
     const long long i = i0 + b;
-    float val = 0.f;
+    float val[RB];
+#pragma unroll
+    for (int p = 0; p < RB; ++p) val[p] = 0.f;
     if (i < n && k < a.d) {
-      float c, h = 0.f;
       if (a.lower) {
         const float lo = a.lower[i * a.d + k], up = a.upper[i * a.d + k];
-        c = 0.5f * (lo + up);
-        h = up - c;
-        if (p == 0) val = c;
-        else if (KIND == 0 && V == 0) val = fabsf(h);              // interval err
-        else if (p >= 1 && p <= V) val = (p - 1 == k) ? h : 0.f;   // diag(half)
-        else val = 0.f;
+        const float c = 0.5f * (lo + up);
+        const float h = up - c;
+        val[0] = c;
+        if constexpr (KIND == 0 && V == 0) val[1] = fabsf(h);      // interval err
+        else {
+#pragma unroll
+          for (int p = 1; p <= V; ++p) val[p] = (p - 1 == k) ? h : 0.f;   // diag(half)
+        }
       } else {
-        if (p == 0) val = a.center[i * a.d + k];
-        else if (KIND == 0 && V == 0) {
+        val[0] = a.center[i * a.d + k];
+        if constexpr (KIND == 0 && V == 0) {
           float s = 0.f;
           for (int r = 0; r < a.vin; ++r) s = s + fabsf(a.vecs[(i * a.vin + r) * a.d + k]);
-          val = s;
-        } else if (p >= 1 && p <= V) val = a.vecs[(i * a.vin + (p - 1)) * a.d + k];
-        else val = 0.f;
+          val[1] = s;
+        } else {
+#pragma unroll
+          for (int p = 1; p <= V; ++p) val[p] = a.vecs[(i * a.vin + (p - 1)) * a.d + k];
+        }
       }
     }
-    X[xoff<NB, WMAX>(p, b, k)] = val;
+#pragma unroll
+    for (int p = 0; p < RB; ++p) X[xoff<NB, WMAX>(p, b, k)] = val[p];
   }
 }
 
-template <int KIND, int V, int NB, int NW, int WMAX, bool GX = false, int OCC = 0, int AS = ACTS_ALL>
-__global__ void __launch_bounds__(NW * 64, (OCC ? OCC : (GX ? 2 : LdsOcc<Planes<KIND, V, 0>::R, NB, NW, WMAX>::value)))
+// TPW: tiles per workgroup (tiles of one wave only; they share nothing).
+template <int KIND, int V, int NB, int NW, int WMAX, bool GX = false, int OCC = 0, int AS = ACTS_ALL, int TPW = 1>
+__global__ void __launch_bounds__(TPW * NW * 64,
+                                  (OCC ? OCC : (GX ? 2 : LdsOcc<Planes<KIND, V, 0>::R, NB, NW, WMAX>::value)))
 k_classify(const DevModel* __restrict__ Mp, ClassifyArgs a) {
   using PL = Planes<KIND, V, 0>;
   constexpr int NT = NW * 64;
+  static_assert(TPW == 1 || NW == 1, "several tiles per workgroup only for tiles of one wave");
+  const int sub = TPW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   float* X;
   if constexpr (GX) {
     // this workgroup's slice of the global activation planes (L2-resident)
     X = a.gx + (size_t)blockIdx.x * (PL::R * NB * WMAX);
   } else {
-    __shared__ float Xs[PL::R * NB * WMAX];
-    X = Xs;
+    __shared__ float Xs[TPW * PL::R * NB * WMAX];
+    X = Xs + sub * (PL::R * NB * WMAX);
   }
   const long long n = a.n_dev ? (long long)(*a.n_dev) : a.n;
   const long long ntiles = (n + NB - 1) / NB;
-  for (long long tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+  for (long long tile = (long long)blockIdx.x * TPW + sub; tile < ntiles; tile += (long long)gridDim.x * TPW) {
     const long long i0 = tile * NB;
     fill_box_inputs<KIND, V, NB, NT, WMAX>(X, a, i0, n);
     mlp_forward<PL, KIND, V, NB, NW, WMAX, AS>(*Mp, X, [&](const float* v, int b) {
