@@ -10,16 +10,15 @@ struct TreeLayout {
   long long cap;      // max nodes in any level list
   long long nbmax;    // max batches per level
   int top_levels;     // levels 0 .. top_levels - 1 are classified in one launch (0: none)
-  long long heap_cap; // heap-index entries per level list
   size_t off_counters, off_codes, off_bcnt, off_boff, off_lvl[2], off_recheck, off_lw, lw_bytes;
-  size_t off_top_box, off_top_codes, off_heap[2], total;
+  size_t off_top_box, off_top_codes, total;
 };
 
 // The top levels of a tree hold at most 2^k nodes each and would each cost a
 // whole launch of one-tile latency; instead every node of levels
 // 0 .. kTopLevels - 1 (8191 boxes, two tiles per CU) is classified in one
-// launch, and those levels take their codes from it by heap index.
-constexpr int kTopLevels = 13;
+// launch, and one workgroup builds those levels' lists from the codes
+// (k_tree_top).
 
 int top_levels_for(const niq_eval_cfg* cfg, const niq_tree_params* p) {
   if (cfg && cfg->recheck_tol > 0.f) return 0;   // the FP64 re-test indexes the level list
@@ -67,11 +66,8 @@ niq_status tree_layout(const niq_model* m, const niq_eval_cfg* cfg, const niq_tr
   L->off_lw = take(L->lw_bytes);
   L->top_levels = top_levels_for(cfg, p);
   const long long n_top = L->top_levels ? (1LL << L->top_levels) - 1 : 0;
-  L->heap_cap = L->top_levels ? std::min(cap, 1LL << (L->top_levels - 1)) : 0;
   L->off_top_box = take(sizeof(float) * 6 * n_top);
   L->off_top_codes = take(sizeof(int) * n_top);
-  L->off_heap[0] = take(sizeof(int) * L->heap_cap);
-  L->off_heap[1] = take(sizeof(int) * L->heap_cap);
   L->total = o;
   return NIQ_OK;
 }
@@ -103,23 +99,13 @@ __global__ void k_top_boxes(float l0, float l1, float l2, float u0, float u1, fl
   top_box_body(r, n_top, lo, up, blockIdx.x * blockDim.x + threadIdx.x + 1);
 }
 
-// Codes of a top level's list from the one launch over the top of the tree.
-__global__ void k_top_gather(const int* __restrict__ heap, const TreeCounters* __restrict__ C, int level,
-                             const int* __restrict__ top_codes, int* __restrict__ codes) {
-  const int n = C->n[level & 1];
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-    codes[i] = top_codes[heap[i] - 1];
-}
-
 // Root box from the arguments, or from `root` (6 floats on the device:
 // lower then upper) when it is given, so a captured build can be replayed for
 // any root box.
-__device__ __forceinline__ void k_tree_init_body(TreeCounters* C, float* lo, float* up, const float* root6,
-                                                 int* heap0) {
+__device__ __forceinline__ void k_tree_init_body(TreeCounters* C, float* lo, float* up, const float* root6) {
   if (threadIdx.x == 0) {
     C->n[0] = 1; C->n[1] = 0; C->n_int = 0; C->n_ext = 0; C->n_classified = 0; C->overflow = 0;
-    C->recheck_cnt = 0; C->n_recheck = 0;
-    if (heap0) heap0[0] = 1;
+    C->recheck_cnt = 0; C->n_recheck = 0; C->top_end = 0; C->top_done = 0;
     lo[0] = root6[0]; lo[1] = root6[1]; lo[2] = root6[2];
     up[0] = root6[3]; up[1] = root6[4]; up[2] = root6[5];
   }
@@ -127,11 +113,11 @@ __device__ __forceinline__ void k_tree_init_body(TreeCounters* C, float* lo, flo
 }
 
 __global__ void k_tree_init(TreeCounters* C, float* lo, float* up, float l0, float l1, float l2, float u0,
-                            float u1, float u2, const float* root, int* heap0) {
+                            float u1, float u2, const float* root) {
   float r[6] = {l0, l1, l2, u0, u1, u2};
   if (root)
     for (int k = 0; k < 6; ++k) r[k] = root[k];
-  k_tree_init_body(C, lo, up, r, heap0);
+  k_tree_init_body(C, lo, up, r);
 }
 
 // ------------------------------------------------- batched builds
@@ -149,8 +135,8 @@ struct TreeItem {
 
 // Offsets of the shared layout, for the device.
 struct TreeOffs {
-  size_t counters, codes, bcnt, boff, lvl[2], top_box, top_codes, heap[2];
-  long long cap, heap_cap;
+  size_t counters, codes, bcnt, boff, lvl[2], top_box, top_codes;
+  long long cap;
   int n_top, top_levels, with_int, with_ext;
 };
 
@@ -165,7 +151,7 @@ __global__ void k_tree_init_b(const TreeItem* __restrict__ items, TreeOffs o) {
   const TreeItem& it = items[blockIdx.x];
   TreeCounters* C = item_counters(it, o);
   float* lo = item_lvl(it, o, 0);
-  k_tree_init_body(C, lo, lo + 3 * o.cap, it.root, o.top_levels ? reinterpret_cast<int*>(it.ws + o.heap[0]) : nullptr);
+  k_tree_init_body(C, lo, lo + 3 * o.cap, it.root);
 }
 
 __global__ void k_top_boxes_b(const TreeItem* __restrict__ items, TreeOffs o) {
@@ -174,15 +160,22 @@ __global__ void k_top_boxes_b(const TreeItem* __restrict__ items, TreeOffs o) {
   top_box_body(it.root, o.n_top, lo, lo + 3 * (size_t)o.n_top, blockIdx.x * blockDim.x + threadIdx.x + 1);
 }
 
-__global__ void k_top_gather_b(const TreeItem* __restrict__ items, TreeOffs o, int level) {
-  const TreeItem& it = items[blockIdx.y];
-  const TreeCounters* C = item_counters(it, o);
-  const int* heap = reinterpret_cast<const int*>(it.ws + o.heap[level & 1]);
-  const int* top_codes = reinterpret_cast<const int*>(it.ws + o.top_codes);
-  int* codes = reinterpret_cast<int*>(it.ws + o.codes);
-  const int n = C->n[level & 1];
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-    codes[i] = top_codes[heap[i] - 1];
+__global__ void __launch_bounds__(1024) k_tree_top_b(const TreeItem* __restrict__ items, TreeOffs o, int n_levels,
+                                                     int B) {
+  const TreeItem& it = items[blockIdx.x];
+  TreeTopArgs a{};
+  a.box_lo = reinterpret_cast<const float*>(it.ws + o.top_box);
+  a.box_up = a.box_lo + 3 * (size_t)o.n_top;
+  a.codes = reinterpret_cast<const int*>(it.ws + o.top_codes);
+  a.top_levels = o.top_levels; a.n_levels = n_levels; a.B = B;
+  a.next_lower = item_lvl(it, o, o.top_levels);
+  a.next_upper = a.next_lower + 3 * o.cap;
+  a.cap = o.cap;
+  a.unk_lower = it.unk_lo; a.unk_upper = it.unk_up; a.cap_unk = it.cap_unk;
+  a.cap_int = a.cap_ext = LLONG_MAX;
+  if (o.with_int) { a.int_lower = it.int_lo; a.int_upper = it.int_up; a.cap_int = it.cap_int; }
+  if (o.with_ext) { a.ext_lower = it.ext_lo; a.ext_upper = it.ext_up; a.cap_ext = it.cap_ext; }
+  tree_top_body(a, item_counters(it, o));
 }
 
 __global__ void __launch_bounds__(256) k_tree_count_b(const TreeItem* __restrict__ items, TreeOffs o, int level,
@@ -213,11 +206,6 @@ __global__ void __launch_bounds__(256) k_tree_scatter_b(const TreeItem* __restri
     sa.cap_next = o.cap;
   } else {
     sa.next_lower = it.unk_lo; sa.next_upper = it.unk_up; sa.cap_next = it.cap_unk;
-  }
-  if (split && level + 1 < o.top_levels) {
-    sa.heap = reinterpret_cast<const int*>(it.ws + o.heap[level & 1]);
-    sa.next_heap = reinterpret_cast<int*>(it.ws + o.heap[(level + 1) & 1]);
-    sa.cap_heap = o.heap_cap;
   }
   if (o.with_int) { sa.int_lower = it.int_lo; sa.int_upper = it.int_up; sa.cap_int = it.cap_int; }
   if (o.with_ext) { sa.ext_lower = it.ext_lo; sa.ext_upper = it.ext_up; sa.cap_ext = it.cap_ext; }
@@ -384,11 +372,9 @@ niq_status tree_enqueue(const niq_model* m, const niq_eval_cfg* cfg, const niq_t
   const int B = p->batch_process_size;
 
   const int T = L.top_levels;
-  int* heap[2] = {reinterpret_cast<int*>(base + L.off_heap[0]), reinterpret_cast<int*>(base + L.off_heap[1])};
   int* top_codes = reinterpret_cast<int*>(base + L.off_top_codes);
-  hipLaunchKernelGGL(k_tree_init, dim3(1), dim3(64), 0, s, C, lvl[0], lvl[0] + 3 * cap, p->lower[0], p->lower[1],
-                     p->lower[2], p->upper[0], p->upper[1], p->upper[2], root_dev, T ? heap[0] : nullptr);
-  HIPCHK(hipGetLastError());
+  const int n_levels = p->split_depth >= 0 ? p->split_depth + 1 : 64;
+  int level = 0;
   if (T) {
     const int n_top = (1 << T) - 1;
     float* top_lo = reinterpret_cast<float*>(base + L.off_top_box);
@@ -401,10 +387,37 @@ niq_status tree_enqueue(const niq_model* m, const niq_eval_cfg* cfg, const niq_t
     a.codes = top_codes;
     if (L.lw_bytes) { a.lw_buf = base + L.off_lw; a.lw_bytes = L.lw_bytes; }
     if (niq_status st = classify_dispatch(m, cfg, 3, a, n_top, s)) return st;
+    TreeTopArgs ta{};
+    ta.box_lo = top_lo; ta.box_up = top_up; ta.codes = top_codes;
+    ta.top_levels = T; ta.n_levels = n_levels; ta.B = B;
+    ta.thresh = sync_allowed ? std::max<long long>(p->node_terminate_thresh, 0) : 0;
+    ta.next_lower = lvl[T & 1]; ta.next_upper = ta.next_lower + 3 * cap; ta.cap = cap;
+    ta.unk_lower = res->unknown_lower; ta.unk_upper = res->unknown_upper; ta.cap_unk = res->unknown_capacity;
+    ta.cap_int = ta.cap_ext = LLONG_MAX;
+    if (p->with_interior_nodes) { ta.int_lower = res->interior_lower; ta.int_upper = res->interior_upper; ta.cap_int = res->interior_capacity; }
+    if (p->with_exterior_nodes) { ta.ext_lower = res->exterior_lower; ta.ext_upper = res->exterior_upper; ta.cap_ext = res->exterior_capacity; }
+    hipLaunchKernelGGL(k_tree_top, dim3(1), dim3(1024), 0, s, ta, C);
+    HIPCHK(hipGetLastError());
+    level = T;
+    bool ended = n_levels <= T;
+    if (ta.thresh > 0) {   // where the node count ended the tree, only the device knows
+      int end[2] = {0, 0};
+      HIPCHK(hipMemcpyAsync(end, &C->top_end, sizeof(end), hipMemcpyDeviceToHost, s));
+      HIPCHK(hipStreamSynchronize(s));
+      level = end[0];
+      ended = end[1] != 0;
+    }
+    if (ended) {
+      if (levels_out) *levels_out = level;
+      if (counters_offset) *counters_offset = L.off_counters;
+      return NIQ_OK;
+    }
+  } else {
+    hipLaunchKernelGGL(k_tree_init, dim3(1), dim3(64), 0, s, C, lvl[0], lvl[0] + 3 * cap, p->lower[0], p->lower[1],
+                       p->lower[2], p->upper[0], p->upper[1], p->upper[2], root_dev);
+    HIPCHK(hipGetLastError());
   }
 
-  const int n_levels = p->split_depth >= 0 ? p->split_depth + 1 : 64;
-  int level = 0;
   for (; level < std::min(n_levels, 62); ++level) {
     bool quit_next = (level + 1 == n_levels);
     if (p->node_terminate_thresh > 0 && sync_allowed) {
@@ -428,13 +441,7 @@ niq_status tree_enqueue(const niq_model* m, const niq_eval_cfg* cfg, const niq_t
       a.recheck_idx = reinterpret_cast<int*>(base + L.off_recheck);
       a.recheck_cap = (int)std::min<long long>(cap, INT_MAX);
     }
-    if (level < T) {
-      hipLaunchKernelGGL(k_top_gather, dim3((unsigned)((max_n + 255) / 256)), dim3(256), 0, s, heap[level & 1], C,
-                         level, top_codes, codes);
-      HIPCHK(hipGetLastError());
-    } else if (niq_status st = classify_dispatch(m, cfg, 3, a, max_n, s)) {
-      return st;
-    }
+    if (niq_status st = classify_dispatch(m, cfg, 3, a, max_n, s)) return st;
 
     const unsigned nb = (unsigned)((max_n + B - 1) / B);
     hipLaunchKernelGGL(k_tree_count, dim3(nb), dim3(256), 0, s, codes, C, level, B, bcnt);
@@ -450,11 +457,6 @@ niq_status tree_enqueue(const niq_model* m, const niq_eval_cfg* cfg, const niq_t
       sa.next_lower = res->unknown_lower;
       sa.next_upper = res->unknown_upper;
       sa.cap_next = res->unknown_capacity;
-    }
-    if (split && level + 1 < T) {
-      sa.heap = heap[level & 1];
-      sa.next_heap = heap[(level + 1) & 1];
-      sa.cap_heap = L.heap_cap;
     }
     if (p->with_interior_nodes) { sa.int_lower = res->interior_lower; sa.int_upper = res->interior_upper; sa.cap_int = res->interior_capacity; }
     if (p->with_exterior_nodes) { sa.ext_lower = res->exterior_lower; sa.ext_upper = res->exterior_upper; sa.cap_ext = res->exterior_capacity; }
@@ -589,8 +591,7 @@ niq_status tree_batch_build(const niq_model* const* models, int ng, const niq_ev
   TreeOffs o{};
   o.counters = L.off_counters; o.codes = L.off_codes; o.bcnt = L.off_bcnt; o.boff = L.off_boff;
   o.lvl[0] = L.off_lvl[0]; o.lvl[1] = L.off_lvl[1]; o.top_box = L.off_top_box; o.top_codes = L.off_top_codes;
-  o.heap[0] = L.off_heap[0]; o.heap[1] = L.off_heap[1];
-  o.cap = L.cap; o.heap_cap = L.heap_cap;
+  o.cap = L.cap;
   o.top_levels = L.top_levels;
   o.n_top = L.top_levels ? (1 << L.top_levels) - 1 : 0;
   o.with_int = p->with_interior_nodes ? 1 : 0; o.with_ext = p->with_exterior_nodes ? 1 : 0;
@@ -613,25 +614,22 @@ niq_status tree_batch_build(const niq_model* const* models, int ng, const niq_ev
     }
   };
   hipfail(hipMemcpyAsync(d_items, items.data(), sizeof(TreeItem) * ng, hipMemcpyHostToDevice, s), "tree batch table");
-  if (st == NIQ_OK) {
-    hipLaunchKernelGGL(k_tree_init_b, dim3(ng), dim3(64), 0, s, d_items, o);
-    hipfail(hipGetLastError(), "k_tree_init_b");
-  }
   if (st == NIQ_OK && o.top_levels) {
     hipLaunchKernelGGL(k_top_boxes_b, dim3((o.n_top + 255) / 256, ng), dim3(256), 0, s, d_items, o);
     hipfail(hipGetLastError(), "k_top_boxes_b");
     classify(-1, o.n_top);
+    if (st == NIQ_OK) {
+      hipLaunchKernelGGL(k_tree_top_b, dim3(ng), dim3(1024), 0, s, d_items, o, n_levels, B);
+      hipfail(hipGetLastError(), "k_tree_top_b");
+    }
+  } else if (st == NIQ_OK) {
+    hipLaunchKernelGGL(k_tree_init_b, dim3(ng), dim3(64), 0, s, d_items, o);
+    hipfail(hipGetLastError(), "k_tree_init_b");
   }
-  for (int level = 0; level < n_levels && st == NIQ_OK; ++level) {
+  for (int level = o.top_levels; level < n_levels && st == NIQ_OK; ++level) {
     const int split = level + 1 < n_levels ? 1 : 0;
     const long long max_n = level < 40 ? std::min(L.cap, 1LL << level) : L.cap;
-    if (level < o.top_levels) {
-      hipLaunchKernelGGL(k_top_gather_b, dim3((unsigned)((max_n + 255) / 256), ng), dim3(256), 0, s, d_items, o,
-                         level);
-      hipfail(hipGetLastError(), "k_top_gather_b");
-    } else {
-      classify(level, max_n);
-    }
+    classify(level, max_n);
     if (st != NIQ_OK) break;
     const unsigned nb = (unsigned)((max_n + B - 1) / B);
     hipLaunchKernelGGL(k_tree_count_b, dim3(nb, ng), dim3(256), 0, s, d_items, o, level, B);

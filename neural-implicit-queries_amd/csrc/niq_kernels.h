@@ -393,6 +393,8 @@ struct TreeCounters {
   int overflow;
   int recheck_cnt;       // cells listed for the FP64 re-test in this level
   long long n_recheck;   // over all levels
+  int top_end;           // levels run by k_tree_top (0: it did not run)
+  int top_done;          // 1: the tree ended in them
   int level_n[64];
   int level_int[64];
   int level_ext[64];
@@ -502,13 +504,29 @@ struct TreeScatterArgs {
   long long cap_next;
   float* int_lower; float* int_upper; long long cap_int;   // nullable
   float* ext_lower; float* ext_upper; long long cap_ext;   // nullable
-  // heap indices of the nodes (root 1, children 2h and 2h + 1) while the
-  // level lies in the precomputed top of the tree; null below it
-  const int* heap; int* next_heap; long long cap_heap;
 };
 
 __device__ __forceinline__ void store3(float* p, long long i, float x, float y, float z) {
   p[3 * i] = x; p[3 * i + 1] = y; p[3 * i + 2] = z;
+}
+
+// The two children of a node at rows pa and pb: its halves along the widest
+// axis (the first on ties).
+__device__ __forceinline__ void store_children(float* lo, float* up, long long cap, long long pa, long long pb,
+                                               float l0, float l1, float l2, float u0, float u1, float u2) {
+  const float e0 = u0 - l0, e1 = u1 - l1, e2 = u2 - l2;
+  int dim = 0; float em = e0;
+  if (e1 > em) { dim = 1; em = e1; }
+  if (e2 > em) { dim = 2; }
+  const float m0 = 0.5f * (l0 + u0), m1 = 0.5f * (l1 + u1), m2 = 0.5f * (l2 + u2);
+  if (pa < cap) {
+    store3(lo, pa, l0, l1, l2);
+    store3(up, pa, dim == 0 ? m0 : u0, dim == 1 ? m1 : u1, dim == 2 ? m2 : u2);
+  }
+  if (pb < cap) {
+    store3(lo, pb, dim == 0 ? m0 : l0, dim == 1 ? m1 : l1, dim == 2 ? m2 : l2);
+    store3(up, pb, u0, u1, u2);
+  }
 }
 
 // Stable per-batch placement of children and finished leaves, in the
@@ -553,25 +571,8 @@ __device__ __forceinline__ void tree_scatter_body(const TreeScatterArgs& a, cons
       if (c == CODE_UNKNOWN) {
         const long long ru = ru0 + pu + __popcll(mu & below);
         if (split) {
-          const float e0 = u0 - l0, e1 = u1 - l1, e2 = u2 - l2;
-          int dim = 0; float em = e0;
-          if (e1 > em) { dim = 1; em = e1; }
-          if (e2 > em) { dim = 2; }
-          const float m0 = 0.5f * (l0 + u0), m1 = 0.5f * (l1 + u1), m2 = 0.5f * (l2 + u2);
           const long long pa = 2 * Ub + ru, pb = 2 * Ub + nUb + ru;
-          if (pa < a.cap_next) {
-            store3(a.next_lower, pa, l0, l1, l2);
-            store3(a.next_upper, pa, dim == 0 ? m0 : u0, dim == 1 ? m1 : u1, dim == 2 ? m2 : u2);
-          }
-          if (pb < a.cap_next) {
-            store3(a.next_lower, pb, dim == 0 ? m0 : l0, dim == 1 ? m1 : l1, dim == 2 ? m2 : l2);
-            store3(a.next_upper, pb, u0, u1, u2);
-          }
-          if (a.next_heap) {
-            const int h = a.heap[i];
-            if (pa < a.cap_heap) a.next_heap[pa] = 2 * h;
-            if (pb < a.cap_heap) a.next_heap[pb] = 2 * h + 1;
-          }
+          store_children(a.next_lower, a.next_upper, a.cap_next, pa, pb, l0, l1, l2, u0, u1, u2);
         } else {
           const long long p = Ub + ru;
           if (p < a.cap_next) { store3(a.next_lower, p, l0, l1, l2); store3(a.next_upper, p, u0, u1, u2); }
@@ -587,6 +588,145 @@ __device__ __forceinline__ void tree_scatter_body(const TreeScatterArgs& a, cons
     ru0 += tu; rp0 += tp; rn0 += tn;
   }
 }
+
+// The compaction of the top levels in one workgroup of 1024.  Levels
+// 0 .. top_levels - 1 hold at most kTopMaxN nodes, all classified beforehand
+// (codes and boxes by heap index: root 1, children 2h and 2h + 1), so the lists
+// are heap indices in LDS and a level is one block scan: the order and counts
+// are those of the per-level kernels.  Bound by the barriers of that scan,
+// about 1.5 us a level; as a gather, count, scan and scatter launch a level cost
+// about 12 us, whatever its size.
+constexpr int kTopLevels = 13;
+constexpr int kTopMaxN = 1 << (kTopLevels - 1);
+
+struct TreeTopArgs {
+  const float* box_lo; const float* box_up;   // boxes by heap index - 1
+  const int* codes;
+  int top_levels;                             // levels to run
+  int n_levels;                               // of the whole tree (the last one is not split)
+  long long thresh;                           // > 0: a level of at least this many nodes is not split
+  int B;
+  float* next_lower; float* next_upper; long long cap;      // list of level top_levels
+  float* unk_lower; float* unk_upper; long long cap_unk;
+  float* int_lower; float* int_upper; long long cap_int;    // nullable (capacity LLONG_MAX)
+  float* ext_lower; float* ext_upper; long long cap_ext;
+};
+
+__device__ __forceinline__ void tree_top_body(const TreeTopArgs& a, TreeCounters* C) {
+  constexpr int NT = 1024, PER = kTopMaxN / NT, NWV = NT / 64;
+  __shared__ unsigned char s_code[2 * kTopMaxN];
+  __shared__ unsigned short s_heap[2][kTopMaxN];
+  __shared__ int s_pre[kTopMaxN + 1];               // unknown nodes before each node
+  __shared__ unsigned long long s_wave[NWV];        // per wave: unknown, positive, negative (21 bits each)
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int n_top = (1 << a.top_levels) - 1;
+  for (int h = tid; h < n_top; h += NT) s_code[h + 1] = (unsigned char)a.codes[h];
+  for (int i = tid; i < 64; i += NT) { C->level_n[i] = 0; C->level_int[i] = 0; C->level_ext[i] = 0; }
+  if (tid == 0) s_heap[0][0] = 1;
+  __syncthreads();
+  int n = 1, n_int = 0, n_ext = 0, overflow = 0, level = 0, done = 0;
+  long long classified = 0;
+  for (; level < a.top_levels && !done; ++level) {
+    const bool split = !(level + 1 == a.n_levels || (a.thresh > 0 && n >= a.thresh));
+    const unsigned short* heap = s_heap[level & 1];
+    unsigned short* next = s_heap[(level + 1) & 1];
+    // exclusive scan of the code counts, PER consecutive nodes a thread
+    int h[PER], code[PER];
+    unsigned long long mine = 0;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int i = tid * PER + k;
+      h[k] = i < n ? heap[i] : 0;
+      code[k] = i < n ? s_code[h[k]] : -1;
+      if (i < n) mine += 1ull << (21 * (code[k] == CODE_UNKNOWN ? 0 : (code[k] == CODE_POSITIVE ? 1 : 2)));
+    }
+    unsigned long long incl = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const unsigned long long v = __shfl_up(incl, d);
+      if (lane >= d) incl += v;
+    }
+    if (lane == 63) s_wave[wave] = incl;
+    __syncthreads();
+    unsigned long long before = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < NWV; ++w) {
+      const unsigned long long v = s_wave[w];
+      if (w < wave) before += v;
+      total += v;
+    }
+    const unsigned long long ex = before + incl - mine;
+    constexpr unsigned long long M21 = (1ull << 21) - 1;
+    const int U = (int)(total & M21), P = (int)((total >> 21) & M21), N = (int)(total >> 42);
+    int ru = (int)(ex & M21), rp = (int)((ex >> 21) & M21), rn = (int)(ex >> 42);
+    const int ru0 = ru;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int i = tid * PER + k;
+      if (i < n) s_pre[i] = ru;
+      if (code[k] == CODE_UNKNOWN) ++ru;
+    }
+    if (tid == 0) s_pre[n] = U;
+    __syncthreads();
+    ru = ru0;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int i = tid * PER + k;
+      if (i >= n) continue;
+      const int c = code[k], hb = 3 * (h[k] - 1);
+      if (c == CODE_UNKNOWN) {
+        const int b0 = i & ~(a.B - 1);   // the batch's first node (B is a power of 2)
+        const int Ub = s_pre[b0], nUb = s_pre[min((long long)b0 + a.B, (long long)n)] - Ub;
+        const long long pa = ru + Ub, pb = pa + nUb;
+        if (!split) {
+          if (ru < a.cap_unk) {
+            store3(a.unk_lower, ru, a.box_lo[hb], a.box_lo[hb + 1], a.box_lo[hb + 2]);
+            store3(a.unk_upper, ru, a.box_up[hb], a.box_up[hb + 1], a.box_up[hb + 2]);
+          }
+        } else if (level + 1 < a.top_levels) {
+          if (pa < min(a.cap, (long long)kTopMaxN)) next[pa] = (unsigned short)(2 * h[k]);
+          if (pb < min(a.cap, (long long)kTopMaxN)) next[pb] = (unsigned short)(2 * h[k] + 1);
+        } else {
+          store_children(a.next_lower, a.next_upper, a.cap, pa, pb, a.box_lo[hb], a.box_lo[hb + 1],
+                         a.box_lo[hb + 2], a.box_up[hb], a.box_up[hb + 1], a.box_up[hb + 2]);
+        }
+        ++ru;
+      } else if (c == CODE_POSITIVE) {
+        const long long p = n_ext + rp++;
+        if (a.ext_lower && p < a.cap_ext) {
+          store3(a.ext_lower, p, a.box_lo[hb], a.box_lo[hb + 1], a.box_lo[hb + 2]);
+          store3(a.ext_upper, p, a.box_up[hb], a.box_up[hb + 1], a.box_up[hb + 2]);
+        }
+      } else {
+        const long long p = n_int + rn++;
+        if (a.int_lower && p < a.cap_int) {
+          store3(a.int_lower, p, a.box_lo[hb], a.box_lo[hb + 1], a.box_lo[hb + 2]);
+          store3(a.int_upper, p, a.box_up[hb], a.box_up[hb + 1], a.box_up[hb + 2]);
+        }
+      }
+    }
+    if (tid == 0) { C->level_n[level] = n; C->level_int[level] = n_int; C->level_ext[level] = n_ext; }
+    classified += n;
+    n_ext += P;
+    n_int += N;
+    const long long nn = split ? 2LL * U : (long long)U, cap_next = split ? a.cap : a.cap_unk;
+    if (nn > cap_next || n_ext > a.cap_ext || n_int > a.cap_int) overflow = 1;
+    n = (int)min(nn, cap_next);
+    done = !split;
+    __syncthreads();   // next list complete; s_wave and s_pre free
+  }
+  if (tid == 0) {
+    C->n[level & 1] = n;
+    C->n[(level + 1) & 1] = 0;
+    C->n_int = n_int; C->n_ext = n_ext;
+    C->n_classified = classified;
+    C->overflow = overflow;
+    C->recheck_cnt = 0; C->n_recheck = 0;
+    C->top_end = level; C->top_done = done;
+  }
+}
+
+static __global__ void __launch_bounds__(1024) k_tree_top(TreeTopArgs a, TreeCounters* C) { tree_top_body(a, C); }
 
 static __global__ void __launch_bounds__(256)
 k_tree_scatter(TreeScatterArgs a, const int* __restrict__ bcnt, const int* __restrict__ boff,
