@@ -68,19 +68,22 @@ extern "C" niq_status niq_cast_rays_frustum(const niq_model* const* models, int 
   FrustList Ls[2], F;
   mk_list(Ls[0]); mk_list(Ls[1]); mk_list(F);
   int* fin_hit = static_cast<int*>(al(sizeof(int) * cap));
-  FrustWork W{};
-  W.geo = static_cast<float*>(al(sizeof(float) * 14 * cap));
-  W.center = static_cast<float*>(al(sizeof(float) * 3 * cap));
-  W.vecs = static_cast<float*>(al(sizeof(float) * 9 * cap));
-  W.pts = static_cast<float*>(al(sizeof(float) * 6 * cap));
-  W.codes = static_cast<int*>(al(sizeof(int) * cap * n_models));
-  W.vals = static_cast<float*>(al(sizeof(float) * 2 * cap * n_models));
-  W.is_hit = static_cast<int*>(al(sizeof(int) * cap));
-  W.hit_id = static_cast<int*>(al(sizeof(int) * cap));
-  W.demands = static_cast<int*>(al(sizeof(int) * cap));
-  W.nsteps = static_cast<int*>(al(sizeof(int) * cap));
-  W.can_step = static_cast<int*>(al(sizeof(int) * cap));
-  FrustCounters* C = static_cast<FrustCounters*>(al(sizeof(FrustCounters)));
+  FrustWork Ws[2];   // each iteration writes the next one's (in another order)
+  int* codes = static_cast<int*>(al(sizeof(int) * cap * n_models));
+  float* vals = static_cast<float*>(al(sizeof(float) * 2 * cap * n_models));
+  int4* state = o.n_substeps > 1 ? static_cast<int4*>(al(sizeof(int4) * cap)) : nullptr;
+  for (FrustWork& W : Ws) {
+    W = FrustWork{};
+    W.geo = static_cast<float*>(al(sizeof(float) * 14 * cap));
+    W.center = static_cast<float*>(al(sizeof(float) * 3 * cap));
+    W.vecs = static_cast<float*>(al(sizeof(float) * 9 * cap));
+    W.pts = static_cast<float*>(al(sizeof(float) * 6 * cap));
+    W.codes = codes; W.vals = vals; W.state = state;
+  }
+  // counts[j]: the live frusta of iteration j of a group, then the finished
+  constexpr int kGroup = 8;
+  FrustCount* counts = static_cast<FrustCount*>(al(sizeof(FrustCount) * (kGroup + 2)));
+  int* n_fin = reinterpret_cast<int*>(counts + kGroup + 1);
   int* ticks = static_cast<int*>(al(sizeof(int) * 2 * (ns + 1)));
 
   // initial tiles: linspace(0, res, n_side + 1) truncated (src/queries.py:497-505)
@@ -93,56 +96,82 @@ extern "C" niq_status niq_cast_rays_frustum(const niq_model* const* models, int 
   long long n = n0, bucket = n0, empty = n0, evals = 0;
   int it = 0, cur = 0;
   if (st == NIQ_OK && (hipMemcpyAsync(ticks, ht.data(), sizeof(int) * ht.size(), hipMemcpyHostToDevice, s) != hipSuccess ||
-                       hipMemsetAsync(C, 0, sizeof(FrustCounters), s) != hipSuccess))
+                       hipMemsetAsync(n_fin, 0, sizeof(int), s) != hipSuccess))
     st = fail(NIQ_ERR_HIP, "frustum set-up failed");
-  if (st == NIQ_OK) {
-    hipLaunchKernelGGL(k_frust_init, dim3((n0 + 255) / 256), dim3(256), 0, s, Ls[0], ns, ticks, ticks + ns + 1,
-                       o.init_step);
-  }
-  FrustCounters h{};
-  while (st == NIQ_OK) {
-    evals += bucket;
-    const FrustList& L = Ls[cur];
-    const unsigned g = (unsigned)std::min<long long>((n + 255) / 256, 8192);
-    hipLaunchKernelGGL(k_frust_geom, dim3(g), dim3(256), 0, s, c, L, W, (int)n);
-    for (int sub = 0; sub < o.n_substeps && st == NIQ_OK; ++sub) {
-      hipLaunchKernelGGL(k_frust_prep, dim3(g), dim3(256), 0, s, c, P, L, W, (int)n);
-      for (int f = 0; f < n_models && st == NIQ_OK; ++f) {
-        ClassifyArgs a{};
-        a.center = W.center; a.vecs = W.vecs; a.vin = 3; a.d = 3; a.n = n; a.offset = 0.f;
-        a.codes = W.codes + (size_t)f * cap;
-        if ((st = classify_dispatch(models[f], cfg, mode == NIQ_MODE_INTERVAL ? 0 : 3, a, n, s))) break;
-        st = points_dev(models[f], W.pts, nullptr, 2, 2 * n, W.vals + (size_t)f * 2 * cap, s);
+  if (st == NIQ_OK)
+    hipLaunchKernelGGL(k_frust_init, dim3((n0 + 255) / 256), dim3(256), 0, s, c, P, Ls[0], Ws[0], ns, ticks,
+                       ticks + ns + 1, o.init_step);
+  // Iterations run in groups without a host read between them: the live count
+  // stays on the device, and the host reads a group's counts at its end (an
+  // iteration past the last finds none live).  A group is short while the
+  // count grows, so that launches are not sized for a count long outgrown
+  // (sizes only choose tiles and grids: every kernel strides over the device
+  // count).  The layer-by-layer precision mode sizes its scratch by max_n and
+  // gets a true bound.
+  const bool strict = cfg && cfg->precision == NIQ_PREC_BF16 && cfg->variant == 3;
+  FrustCount h[kGroup + 2];
+  int hfin = 0;
+  bool done = st != NIQ_OK, growing = true;
+  long long start = n;
+  int from = 0;
+  while (!done) {
+    const int K = growing ? 2 : kGroup;
+    hipLaunchKernelGGL(k_frust_counts, dim3(1), dim3(64), 0, s, counts, from, start, K + 1);
+    start = -1;
+    from = K;
+    for (int j = 0; j < K && st == NIQ_OK; ++j) {
+      const FrustList& L = Ls[cur];
+      const FrustWork& W = Ws[cur];
+      const long long bound = std::min(cap, n << j);
+      const long long est = growing || strict ? bound : std::min(cap, n + n / 4);
+      const int* n_live = reinterpret_cast<const int*>(counts + j);   // the low word
+      const unsigned g = (unsigned)std::min<long long>((est + 255) / 256, 8192);
+      for (int sub = 0; sub < o.n_substeps && st == NIQ_OK; ++sub) {
+        for (int f = 0; f < n_models && st == NIQ_OK; ++f) {
+          ClassifyArgs a{};
+          a.center = W.center; a.vecs = W.vecs; a.vin = 3; a.d = 3; a.n_dev = n_live; a.offset = 0.f;
+          a.codes = W.codes + (size_t)f * cap;
+          if ((st = classify_dispatch(models[f], cfg, mode == NIQ_MODE_INTERVAL ? 0 : 3, a, est, s))) break;
+          st = points_dev(models[f], W.pts, n_live, 2, 2 * est, W.vals + (size_t)f * 2 * cap, s);
+        }
+        if (st) break;
+        const int first = sub == 0 ? 1 : 0;
+        if (sub + 1 < o.n_substeps) {
+          hipLaunchKernelGGL(k_frust_sub, dim3(g), dim3(256), 0, s, c, P, L, W, counts + j, (int)cap, first);
+        } else {
+          hipLaunchKernelGGL(k_frust_step, dim3(g), dim3(kFrustBlock), 0, s, c, P, L, W, counts + j, (int)cap,
+                             first, it + j * o.n_substeps >= o.n_max_step ? 1 : 0, Ls[cur ^ 1], Ws[cur ^ 1], F, fin_hit,
+                             n_fin);
+        }
       }
-      if (st) break;
-      hipLaunchKernelGGL(k_frust_sub, dim3(g), dim3(256), 0, s, P, L, W, (int)n, (int)cap);
+      cur ^= 1;
     }
     if (st) break;
-    hipLaunchKernelGGL(k_frust_finish, dim3(g), dim3(256), 0, s, c, P, L, W, (int)n, it >= o.n_max_step ? 1 : 0,
-                       Ls[cur ^ 1], F, fin_hit, C);
-    if (hipGetLastError() != hipSuccess || hipMemcpyAsync(&h, C, sizeof(h), hipMemcpyDeviceToHost, s) != hipSuccess ||
+    if (hipGetLastError() != hipSuccess ||
+        hipMemcpyAsync(h, counts, sizeof(h), hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess) {
       st = fail(NIQ_ERR_HIP, "frustum iteration failed");
       break;
     }
-    it += o.n_substeps;
-    if (h.n_valid == 0) break;
-    // the reference's padded-array bookkeeping, for N_evals (src/queries.py:557-569)
-    const long long nb = next_bucket_size((long long)h.n_valid + h.n_refine);
-    if (empty + h.n_refine > bucket || nb < bucket) { bucket = nb; empty = h.n_valid; }
-    empty += h.n_refine;
-    n = h.n_next;
-    cur ^= 1;
-    FrustCounters z{0, h.n_fin, 0, 0};
-    if (hipMemcpyAsync(C, &z, sizeof(z), hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess) {
-      st = fail(NIQ_ERR_HIP, "frustum counter reset failed");
-      break;
+    std::memcpy(&hfin, &h[kGroup + 1], sizeof(int));
+    const long long n_before = n;
+    for (int j = 1; j <= K && !done; ++j) {
+      const long long n_next = (long long)(h[j].next & 0xffffffffull), n_refine = (long long)(h[j].next >> 32);
+      const long long n_valid = n_next - n_refine;   // a split adds one entry
+      evals += bucket;
+      it += o.n_substeps;
+      if (n_valid == 0) { done = true; break; }
+      // the reference's padded-array bookkeeping, for N_evals (src/queries.py:557-569)
+      const long long nb = next_bucket_size(n_valid + n_refine);
+      if (empty + n_refine > bucket || nb < bucket) { bucket = nb; empty = n_valid; }
+      empty += n_refine;
+      n = n_next;
     }
+    growing = n > n_before + n_before / 16;
   }
-  if (st == NIQ_OK && h.n_fin > 0) {
-    hipLaunchKernelGGL(k_frust_write, dim3((unsigned)std::min<long long>(h.n_fin, 65536)), dim3(256), 0, s, F,
-                       fin_hit, h.n_fin, ry, out_t, out_hit_id, out_count);
+  if (st == NIQ_OK && hfin > 0) {
+    hipLaunchKernelGGL(k_frust_write, dim3((unsigned)std::min<long long>(hfin, 65536)), dim3(256), 0, s, F,
+                       fin_hit, hfin, ry, out_t, out_hit_id, out_count);
     if (hipGetLastError() != hipSuccess) st = fail(NIQ_ERR_HIP, "frustum output write failed");
   }
   for (void* p : allocs) (void)hipFreeAsync(p, s);
