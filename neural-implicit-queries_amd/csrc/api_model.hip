@@ -83,6 +83,17 @@ niq_status niq_model_create(int n_layers, const int* dims, const int* acts, cons
     if (acts[i] != NIQ_ACT_TANH && acts[i] != NIQ_ACT_NONE) m->tanh_only = false;
     if (acts[i] != NIQ_ACT_ELU && acts[i] != NIQ_ACT_NONE) m->elu_only = false;
   }
+  // first-layer biases at most 8 times the features' sums |W| (both in the
+  // mean square): pre-activations over a box of the unit cube then round by
+  // little beside its size
+  double b2 = 0.0, w2 = 0.0;
+  for (int f = 0; f < dims[1]; ++f) {
+    double sum = 0.0;
+    for (int k = 0; k < dims[0]; ++k) sum += std::fabs((double)W[0][(size_t)k * dims[1] + f]);
+    w2 += sum * sum;
+    if (b && b[0]) b2 += (double)b[0][f] * (double)b[0][f];
+  }
+  m->bias_small = b2 <= 64.0 * w2;
   hipError_t e = hipMalloc(&m->weights, total);
   if (e == hipSuccess) e = hipMemcpy(m->weights, host.data(), total, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&m->dev), sizeof(DevModel));

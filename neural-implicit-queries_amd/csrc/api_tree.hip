@@ -27,6 +27,10 @@ int top_levels_for(const niq_eval_cfg* cfg, const niq_tree_params* p) {
   return t >= 3 ? t : 0;
 }
 
+// The deepest level whose boxes (1/128 of the root's sides) the split
+// contraction takes.
+constexpr int kSplitMaxLevel = 21;
+
 // Boxes per chunk of the layer-by-layer precision mode inside a tree build.
 constexpr long long kTreeLwChunk = 32768;
 
@@ -55,7 +59,10 @@ niq_status tree_layout(const niq_model* m, const niq_eval_cfg* cfg, const niq_tr
   L->off_boff = take(sizeof(int) * 4 * L->nbmax);
   L->off_lvl[0] = take(sizeof(float) * 6 * cap);
   L->off_lvl[1] = take(sizeof(float) * 6 * cap);
-  L->off_recheck = take(sizeof(int) * cap);
+  L->top_levels = top_levels_for(cfg, p);
+  const long long n_top = L->top_levels ? (1LL << L->top_levels) - 1 : 0;
+  // boxes listed for the FP64 re-test, or left over by the split contraction
+  L->off_recheck = take(sizeof(int) * std::max(cap, n_top));
   // activation scratch of the layer-by-layer precision mode (variant 3):
   // two ping-pong buffers of 10 bf16 planes at the widest layer
   L->lw_bytes = 0;
@@ -64,8 +71,6 @@ niq_status tree_layout(const niq_model* m, const niq_eval_cfg* cfg, const niq_tr
     L->lw_bytes = 2 * (size_t)nch * 10 * (size_t)std::max(m->host16.wmax, 32) * 2;
   }
   L->off_lw = take(L->lw_bytes);
-  L->top_levels = top_levels_for(cfg, p);
-  const long long n_top = L->top_levels ? (1LL << L->top_levels) - 1 : 0;
   L->off_top_box = take(sizeof(float) * 6 * n_top);
   L->off_top_codes = take(sizeof(int) * n_top);
   L->total = o;
@@ -92,7 +97,8 @@ __device__ __forceinline__ void top_box_body(const float* root6, int n_top, floa
 }
 
 __global__ void k_top_boxes(float l0, float l1, float l2, float u0, float u1, float u2, const float* root,
-                            int n_top, float* __restrict__ lo, float* __restrict__ up) {
+                            int n_top, float* __restrict__ lo, float* __restrict__ up, TreeCounters* C) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) C->near_cnt = 0;
   float r[6] = {l0, l1, l2, u0, u1, u2};
   if (root)
     for (int k = 0; k < 6; ++k) r[k] = root[k];
@@ -105,7 +111,8 @@ __global__ void k_top_boxes(float l0, float l1, float l2, float u0, float u1, fl
 __device__ __forceinline__ void k_tree_init_body(TreeCounters* C, float* lo, float* up, const float* root6) {
   if (threadIdx.x == 0) {
     C->n[0] = 1; C->n[1] = 0; C->n_int = 0; C->n_ext = 0; C->n_classified = 0; C->overflow = 0;
-    C->recheck_cnt = 0; C->n_recheck = 0; C->top_end = 0; C->top_done = 0;
+    C->recheck_cnt = 0; C->n_recheck = 0; C->near_cnt = 0; C->top_end = 0;
+    C->top_done = 0;
     lo[0] = root6[0]; lo[1] = root6[1]; lo[2] = root6[2];
     up[0] = root6[3]; up[1] = root6[4]; up[2] = root6[5];
   }
@@ -375,18 +382,39 @@ niq_status tree_enqueue(const niq_model* m, const niq_eval_cfg* cfg, const niq_t
   int* top_codes = reinterpret_cast<int*>(base + L.off_top_codes);
   const int n_levels = p->split_depth >= 0 ? p->split_depth + 1 : 64;
   int level = 0;
+  // Levels whose boxes are large enough, beside the root's distance from the
+  // origin, take the split contraction where the net is eligible (smaller boxes
+  // would all be listed for the plain one).
+  int split_levels = 0;
+  if (split_eligible(m, cfg)) {
+    float ext = INFINITY, far = 0.f;
+    for (int k = 0; k < 3; ++k) {
+      ext = std::min(ext, p->upper[k] - p->lower[k]);
+      far = std::max(far, std::max(std::fabs(p->lower[k]), std::fabs(p->upper[k])));
+    }
+    while (split_levels <= kSplitMaxLevel &&
+           0.5f * std::ldexp(ext, -(split_levels + 2) / 3) >= far * kSplitMinSize)
+      ++split_levels;
+  }
+  auto classify = [&](ClassifyArgs a, long long max_n, int lv) -> niq_status {
+    if (lv >= split_levels) return classify_dispatch(m, cfg, 3, a, max_n, s);
+    a.list = reinterpret_cast<int*>(base + L.off_recheck);
+    a.list_n = &C->near_cnt;
+    a.list_cap = (int)std::min<long long>(max_n, INT_MAX);
+    return classify_split(m, a, max_n, s);
+  };
   if (T) {
     const int n_top = (1 << T) - 1;
     float* top_lo = reinterpret_cast<float*>(base + L.off_top_box);
     float* top_up = top_lo + 3 * (size_t)n_top;
     hipLaunchKernelGGL(k_top_boxes, dim3((n_top + 255) / 256), dim3(256), 0, s, p->lower[0], p->lower[1],
-                       p->lower[2], p->upper[0], p->upper[1], p->upper[2], root_dev, n_top, top_lo, top_up);
+                       p->lower[2], p->upper[0], p->upper[1], p->upper[2], root_dev, n_top, top_lo, top_up, C);
     HIPCHK(hipGetLastError());
     ClassifyArgs a{};
     a.lower = top_lo; a.upper = top_up; a.d = 3; a.n = n_top; a.offset = p->offset;
     a.codes = top_codes;
     if (L.lw_bytes) { a.lw_buf = base + L.off_lw; a.lw_bytes = L.lw_bytes; }
-    if (niq_status st = classify_dispatch(m, cfg, 3, a, n_top, s)) return st;
+    if (niq_status st = classify(a, n_top, T - 1)) return st;
     TreeTopArgs ta{};
     ta.box_lo = top_lo; ta.box_up = top_up; ta.codes = top_codes;
     ta.top_levels = T; ta.n_levels = n_levels; ta.B = B;
@@ -441,7 +469,7 @@ niq_status tree_enqueue(const niq_model* m, const niq_eval_cfg* cfg, const niq_t
       a.recheck_idx = reinterpret_cast<int*>(base + L.off_recheck);
       a.recheck_cap = (int)std::min<long long>(cap, INT_MAX);
     }
-    if (niq_status st = classify_dispatch(m, cfg, 3, a, max_n, s)) return st;
+    if (niq_status st = classify(a, max_n, level)) return st;
 
     const unsigned nb = (unsigned)((max_n + B - 1) / B);
     hipLaunchKernelGGL(k_tree_count, dim3(nb), dim3(256), 0, s, codes, C, level, B, bcnt);

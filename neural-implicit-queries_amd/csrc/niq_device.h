@@ -422,6 +422,99 @@ __device__ __forceinline__ void tile_sync() {
   }
 }
 
+// The end of a hidden layer: biases, the activation's rule and the write back to
+// X, for the feature tiles wave + f NW of this wave.
+template <class PL, int KIND, int V, int NB, int NW, int WMAX, int AS, int FTMAX, int R, int BT>
+__device__ __forceinline__ void layer_epilogue(int act, int nft, int wave, int lane,
+                                               const floatx4 (&acc)[FTMAX][R][BT], const floatx4 (&bias4)[FTMAX],
+                                               float* __restrict__ X) {
+  const int ln = lane & 15, lg = lane >> 4;
+  // The layer's activation is chosen once per layer (uniform).  ReLU and the
+  // identity run on the accumulators, the 4 features of a lane together:
+  // their chains (a division each) have no branch between them and
+  // interleave.  (Unrolled by hand: past a size the compiler keeps
+  // `#pragma unroll` loops rolled, and the accumulators then live in
+  // scratch.)
+  auto epilogue = [&](auto act_tag) __attribute__((always_inline)) {
+    constexpr int ACT = decltype(act_tag)::value;
+    constexpr bool LIGHT = ACT == ACT_RELU || ACT == ACT_NONE;
+    static_for<FTMAX>([&](auto fc) __attribute__((always_inline)) {
+      constexpr int f = decltype(fc)::value;
+      const int ft = wave + f * NW;
+      if (ft >= nft) return;
+      static_for<BT>([&](auto tc) __attribute__((always_inline)) {
+        constexpr int t = decltype(tc)::value;
+        const int b = t * 16 + ln;
+        floatx4 outv[R];
+        static_for<4>([&](auto jc) __attribute__((always_inline)) {
+          constexpr int j = decltype(jc)::value;
+          float v[R];
+#pragma unroll
+          for (int p = 0; p < R; ++p) v[p] = acc[f][p][t][j] + (PL::bias(p) ? bias4[f][j] : 0.f);
+          if constexpr (LIGHT) apply_hidden<PL, KIND, V>(ACT, v);
+#pragma unroll
+          for (int p = 0; p < R; ++p) outv[p][j] = v[p];
+        });
+#pragma unroll
+        for (int p = 0; p < R; ++p)
+          *reinterpret_cast<floatx4*>(&X[xoff<NB, WMAX>(p, b, ft * 16 + lg * 4)]) = outv[p];
+      });
+    });
+    // The transcendental rules are hundreds of instructions per feature:
+    // unrolled over a wave's features they overflow the instruction cache
+    // and spill.  They run in a loop over the values just written (each
+    // lane reads its own back), one copy of the rule in all.
+    if constexpr (!LIGHT) {
+#pragma unroll 1
+      for (int i = 0; i < FTMAX * BT; ++i) {
+        const int ft = wave + (i / BT) * NW;
+        if (ft >= nft) break;
+        const int o = xoff<NB, WMAX>(0, (i % BT) * 16 + ln, ft * 16 + lg * 4);
+        floatx4 q[R];
+#pragma unroll
+        for (int p = 0; p < R; ++p) q[p] = *reinterpret_cast<const floatx4*>(&X[o + p * NB * WMAX]);
+        if constexpr (KIND == 2 && R == 1) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) q[0][j] = act_point(ACT, q[0][j]);
+        } else {
+          // two features at a time where the kernel has one rule only:
+          // their chains interleave (with every rule in it, they spill)
+          constexpr int JU = AS == ACTS_ALL ? 1 : 2;
+#pragma unroll 1
+          for (int j = 0; j < 4; j += JU) {
+            float v[JU][R];
+#pragma unroll
+            for (int u = 0; u < JU; ++u) {
+#pragma unroll
+              for (int p = 0; p < R; ++p) v[u][p] = q[p][u];
+              apply_hidden<PL, KIND, V>(ACT, v[u]);
+            }
+#pragma unroll
+            for (int p = 0; p < R; ++p)
+              if constexpr (JU == 2) q[p] = floatx4{q[p][2], q[p][3], v[0][p], v[1][p]};
+              else q[p] = floatx4{q[p][1], q[p][2], q[p][3], v[0][p]};
+          }
+        }
+#pragma unroll
+        for (int p = 0; p < R; ++p) *reinterpret_cast<floatx4*>(&X[o + p * NB * WMAX]) = q[p];
+      }
+    }
+  };
+  if constexpr (AS != ACTS_ALL) {
+    constexpr int A = AS == ACTS_RELU ? ACT_RELU : (AS == ACTS_TANH ? ACT_TANH : ACT_ELU);
+    if (act == A) epilogue(std::integral_constant<int, A>{});
+    else epilogue(std::integral_constant<int, ACT_NONE>{});
+  } else {
+    switch (act) {
+      case ACT_RELU: epilogue(std::integral_constant<int, ACT_RELU>{}); break;
+      case ACT_ELU: epilogue(std::integral_constant<int, ACT_ELU>{}); break;
+      case ACT_SIN: epilogue(std::integral_constant<int, ACT_SIN>{}); break;
+      case ACT_TANH: epilogue(std::integral_constant<int, ACT_TANH>{}); break;
+      default: epilogue(std::integral_constant<int, ACT_NONE>{}); break;
+    }
+  }
+}
+
 template <class PL, int KIND, int V, int NB, int NW, int WMAX, int AS = ACTS_ALL, class Fin>
 __device__ __forceinline__ void mlp_forward(const DevModel& M, float* __restrict__ X, Fin&& fin) {
   constexpr int R = PL::R;
@@ -596,90 +689,7 @@ __device__ __forceinline__ void mlp_forward(const DevModel& M, float* __restrict
         }
       }
     } else {
-      // The layer's activation is chosen once per layer (uniform).  ReLU and the
-      // identity run on the accumulators, the 4 features of a lane together:
-      // their chains (a division each) have no branch between them and
-      // interleave.  (Unrolled by hand: past a size the compiler keeps
-      // `#pragma unroll` loops rolled, and the accumulators then live in
-      // scratch.)
-      auto epilogue = [&](auto act_tag) __attribute__((always_inline)) {
-        constexpr int ACT = decltype(act_tag)::value;
-        constexpr bool LIGHT = ACT == ACT_RELU || ACT == ACT_NONE;
-        static_for<FTMAX>([&](auto fc) __attribute__((always_inline)) {
-          constexpr int f = decltype(fc)::value;
-          const int ft = wave + f * NW;
-          if (ft >= nft) return;
-          static_for<BT>([&](auto tc) __attribute__((always_inline)) {
-            constexpr int t = decltype(tc)::value;
-            const int b = t * 16 + ln;
-            floatx4 outv[R];
-            static_for<4>([&](auto jc) __attribute__((always_inline)) {
-              constexpr int j = decltype(jc)::value;
-              float v[R];
-#pragma unroll
-              for (int p = 0; p < R; ++p) v[p] = acc[f][p][t][j] + (PL::bias(p) ? bias4[f][j] : 0.f);
-              if constexpr (LIGHT) apply_hidden<PL, KIND, V>(ACT, v);
-#pragma unroll
-              for (int p = 0; p < R; ++p) outv[p][j] = v[p];
-            });
-#pragma unroll
-            for (int p = 0; p < R; ++p)
-              *reinterpret_cast<floatx4*>(&X[xoff<NB, WMAX>(p, b, ft * 16 + lg * 4)]) = outv[p];
-          });
-        });
-        // The transcendental rules are hundreds of instructions per feature:
-        // unrolled over a wave's features they overflow the instruction cache
-        // and spill.  They run in a loop over the values just written (each
-        // lane reads its own back), one copy of the rule in all.
-        if constexpr (!LIGHT) {
-#pragma unroll 1
-          for (int i = 0; i < FTMAX * BT; ++i) {
-            const int ft = wave + (i / BT) * NW;
-            if (ft >= nft) break;
-            const int o = xoff<NB, WMAX>(0, (i % BT) * 16 + ln, ft * 16 + lg * 4);
-            floatx4 q[R];
-#pragma unroll
-            for (int p = 0; p < R; ++p) q[p] = *reinterpret_cast<const floatx4*>(&X[o + p * NB * WMAX]);
-            if constexpr (KIND == 2 && R == 1) {
-#pragma unroll
-              for (int j = 0; j < 4; ++j) q[0][j] = act_point(ACT, q[0][j]);
-            } else {
-              // two features at a time where the kernel has one rule only:
-              // their chains interleave (with every rule in it, they spill)
-              constexpr int JU = AS == ACTS_ALL ? 1 : 2;
-#pragma unroll 1
-              for (int j = 0; j < 4; j += JU) {
-                float v[JU][R];
-#pragma unroll
-                for (int u = 0; u < JU; ++u) {
-#pragma unroll
-                  for (int p = 0; p < R; ++p) v[u][p] = q[p][u];
-                  apply_hidden<PL, KIND, V>(ACT, v[u]);
-                }
-#pragma unroll
-                for (int p = 0; p < R; ++p)
-                  if constexpr (JU == 2) q[p] = floatx4{q[p][2], q[p][3], v[0][p], v[1][p]};
-                  else q[p] = floatx4{q[p][1], q[p][2], q[p][3], v[0][p]};
-              }
-            }
-#pragma unroll
-            for (int p = 0; p < R; ++p) *reinterpret_cast<floatx4*>(&X[o + p * NB * WMAX]) = q[p];
-          }
-        }
-      };
-      if constexpr (AS != ACTS_ALL) {
-        constexpr int A = AS == ACTS_RELU ? ACT_RELU : (AS == ACTS_TANH ? ACT_TANH : ACT_ELU);
-        if (Ly.act == A) epilogue(std::integral_constant<int, A>{});
-        else epilogue(std::integral_constant<int, ACT_NONE>{});
-      } else {
-        switch (Ly.act) {
-          case ACT_RELU: epilogue(std::integral_constant<int, ACT_RELU>{}); break;
-          case ACT_ELU: epilogue(std::integral_constant<int, ACT_ELU>{}); break;
-          case ACT_SIN: epilogue(std::integral_constant<int, ACT_SIN>{}); break;
-          case ACT_TANH: epilogue(std::integral_constant<int, ACT_TANH>{}); break;
-          default: epilogue(std::integral_constant<int, ACT_NONE>{}); break;
-        }
-      }
+      layer_epilogue<PL, KIND, V, NB, NW, WMAX, AS>(Ly.act, nft, wave, lane, acc, bias4, X);
     }
     Ly = Ln;
   }

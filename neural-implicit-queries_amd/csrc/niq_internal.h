@@ -134,6 +134,7 @@ struct niq_model {
   bool relu_only = false;      // every hidden activation is ReLU
   bool tanh_only = false;      // every hidden activation is TanH
   bool elu_only = false;       // every hidden activation is ELU
+  bool bias_small = false;     // first-layer biases are small beside the weights (split contraction)
   DevModelBf16 host16;         // precision-mode copy (bf16 hi/lo/|W| weights)
   DevModelBf16* dev16 = nullptr;
   void* weights16 = nullptr;
@@ -182,6 +183,12 @@ niq_status classify_bf16(const niq_model* m, const niq_eval_cfg* cfg, int nvec, 
                          long long max_n, hipStream_t s);
 niq_status classify_rows(const niq_model* m, const niq_eval_cfg* cfg, const ClassifyArgs& a, long long max_n,
                          hipStream_t s);
+// Sign codes of axis-aligned boxes (a.list, a.list_n set; no bounds, no FP64
+// re-test) by the split contraction, the boxes near the threshold by k_classify:
+// the codes of classify_dispatch, faster on wide ReLU nets.  Needs
+// split_eligible(m, cfg).  Defined in api_classify_split.hip.
+bool split_eligible(const niq_model* m, const niq_eval_cfg* cfg);
+niq_status classify_split(const niq_model* m, const ClassifyArgs& a, long long max_n, hipStream_t s);
 // ... with the optional FP64 re-test list in stream-ordered scratch.
 niq_status classify_with_recheck(const niq_model* m, const niq_eval_cfg* cfg, int nvec, ClassifyArgs a,
                                  long long n, hipStream_t s);

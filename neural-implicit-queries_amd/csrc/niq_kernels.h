@@ -3,6 +3,8 @@
 // ray caster.  Everything here is gfx950-only HIP; host dispatch lives in
 // niq_api.hip.
 #pragma once
+#include <climits>
+
 #include "niq_device.h"
 
 // Workgroup shapes per padded max width: boxes per tile (NB) and waves (NW).
@@ -105,10 +107,17 @@ struct ClassifyArgs {
   int recheck_cap;
   void* lw_buf;            // precision mode, layer by layer: activation scratch
   size_t lw_bytes;         //   (null: allocated per call, stream ordered)
+  int* list;               // split contraction: the boxes left to k_classify,
+  int* list_n;             //   their count (zero on entry) and capacity
+  int list_cap;
   float lipschitz;         // weak-SDF test: Lipschitz bound of f
   float* gx;               // forms too large for LDS: activation planes in global
                            //   memory, R * NB * WMAX floats per workgroup
 };
+
+// The smallest box half-width the split contraction judges by, relative to the
+// box's distance from the origin.
+constexpr float kSplitMinSize = 1.f / 200.f;
 
 // Weak-SDF sign code (src/sdf.py:42-48): UNKNOWN where the value at the centre
 // could change sign within the box, else its sign against the offset.
@@ -123,7 +132,7 @@ __device__ __forceinline__ int sdf_code(float val, float rad, float lipschitz, f
 // Fill the layer-0 input planes of one tile (features 0..15, zero padded).
 // One thread per (box, input): its box is read once and every plane's value
 // written from it.
-template <int KIND, int V, int NB, int NT, int WMAX>
+template <int KIND, int V, int NB, int NT, int WMAX, bool LIST = false>
 __device__ __forceinline__ void fill_box_inputs(float* X, const ClassifyArgs& a, long long i0, long long n) {
   using PL = Planes<KIND, V, 0>;
   constexpr int RB = PL::RB;
@@ -132,11 +141,12 @@ __device__ __forceinline__ void fill_box_inputs(float* X, const ClassifyArgs& a,
     const int e = e0 + (int)threadIdx.x % NT;
     if (NB * 16 % NT != 0 && e >= NB * 16) break;
     const int b = e >> 4, k = e & 15;
-    const long long i = i0 + b;
+    long long i = i0 + b;
+    if constexpr (LIST) i = i < n ? a.list[i] : LLONG_MAX;
     float val[RB];
 #pragma unroll
     for (int p = 0; p < RB; ++p) val[p] = 0.f;
-    if (i < n && k < a.d) {
+    if ((LIST ? i != LLONG_MAX : i < n) && k < a.d) {
       if (a.lower) {
         const float lo = a.lower[i * a.d + k], up = a.upper[i * a.d + k];
         const float c = 0.5f * (lo + up);
@@ -165,7 +175,9 @@ __device__ __forceinline__ void fill_box_inputs(float* X, const ClassifyArgs& a,
 }
 
 // TPW: tiles per workgroup (tiles of one wave only; they share nothing).
-template <int KIND, int V, int NB, int NW, int WMAX, bool GX = false, int OCC = 0, int AS = ACTS_ALL, int TPW = 1>
+// LIST: classify the boxes of a.list (their indices) instead of all.
+template <int KIND, int V, int NB, int NW, int WMAX, bool GX = false, int OCC = 0, int AS = ACTS_ALL, int TPW = 1,
+          bool LIST = false>
 __global__ void __launch_bounds__(TPW * NW * 64,
                                   (OCC ? OCC : (GX ? 2 : LdsOcc<Planes<KIND, V, 0>::R, NB, NW, WMAX>::value)))
 k_classify(const DevModel* __restrict__ Mp, ClassifyArgs a) {
@@ -181,14 +193,15 @@ k_classify(const DevModel* __restrict__ Mp, ClassifyArgs a) {
     __shared__ float Xs[TPW * PL::R * NB * WMAX];
     X = Xs + sub * (PL::R * NB * WMAX);
   }
-  const long long n = a.n_dev ? (long long)(*a.n_dev) : a.n;
+  const long long n = LIST ? (long long)min(*a.list_n, a.list_cap) : (a.n_dev ? (long long)(*a.n_dev) : a.n);
   const long long ntiles = (n + NB - 1) / NB;
   for (long long tile = (long long)blockIdx.x * TPW + sub; tile < ntiles; tile += (long long)gridDim.x * TPW) {
     const long long i0 = tile * NB;
-    fill_box_inputs<KIND, V, NB, NT, WMAX>(X, a, i0, n);
+    fill_box_inputs<KIND, V, NB, NT, WMAX, LIST>(X, a, i0, n);
     mlp_forward<PL, KIND, V, NB, NW, WMAX, AS>(*Mp, X, [&](const float* v, int b) {
-      const long long i = i0 + b;
+      long long i = i0 + b;
       if (i >= n) return;
+      if constexpr (LIST) i = a.list[i];
       float lo, hi, scale;
       final_bounds<KIND, V>(v, lo, hi, scale);
       a.codes[i] = sign_code(lo, hi, a.offset);
@@ -393,6 +406,7 @@ struct TreeCounters {
   int overflow;
   int recheck_cnt;       // cells listed for the FP64 re-test in this level
   long long n_recheck;   // over all levels
+  int near_cnt;          // boxes the split contraction leaves to k_classify
   int top_end;           // levels run by k_tree_top (0: it did not run)
   int top_done;          // 1: the tree ended in them
   int level_n[64];
@@ -480,6 +494,7 @@ __device__ __forceinline__ void tree_scan_body(const int* __restrict__ bcnt, int
     C->level_n[level] = n;
     C->n_recheck += C->recheck_cnt;
     C->recheck_cnt = 0;
+    C->near_cnt = 0;
     C->level_int[level] = C->n_int;
     C->level_ext[level] = C->n_ext;
     C->n_classified += n;
@@ -721,7 +736,7 @@ __device__ __forceinline__ void tree_top_body(const TreeTopArgs& a, TreeCounters
     C->n_int = n_int; C->n_ext = n_ext;
     C->n_classified = classified;
     C->overflow = overflow;
-    C->recheck_cnt = 0; C->n_recheck = 0;
+    C->recheck_cnt = 0; C->n_recheck = 0; C->near_cnt = 0;
     C->top_end = level; C->top_done = done;
   }
 }

@@ -1,0 +1,235 @@
+// Classification with the FP32 contraction carried by bf16 matrix
+// instructions, for launches that ask for sign codes only.
+//
+// Every activation and weight is split into three bf16 terms that add up to it
+// exactly (x = x1 + x2 + x3: 8 bits of significand each, 24 in all), and a
+// dense layer sums the six products down to 2^-18 of the largest,
+//     x3 w1 + x2 w2 + x1 w3 + x2 w1 + x1 w2 + x1 w1
+// (the three dropped ones are below 2^-26 |x w|, a quarter of half an ulp),
+// each exact, with v_mfma_f32_16x16x32_bf16 into one FP32 accumulator.  30 such
+// instructions of 16 cycles do the work of 40 FP32 ones of 32 over 5 planes and
+// 32 inputs: 480 against 1,280 matrix cycles.  Inputs, accumulator and the
+// layer rules stay FP32; there are fewer roundings than in the FP32 chain (6
+// accumulations per 32 inputs instead of 32).
+//
+// The sums round differently from k_classify's, so a box whose bound lies near
+// the threshold is listed and classified again by k_classify's own forward:
+// the codes are the plain kernel's.
+#pragma once
+#include "niq_bf16.h"
+
+// Tiles: 16 boxes, each wave 4 feature tiles (a fragment of X split once in a
+// wave's registers serves them all).
+template <int WMAX> struct SplitTile;
+template <> struct SplitTile<256> { static constexpr int NB = 16, NW = 4; };
+template <> struct SplitTile<512> { static constexpr int NB = 16, NW = 8; };
+
+// 8 FP32 values to their three bf16 terms.
+__device__ __forceinline__ void split_x8(const floatx4 lo, const floatx4 hi, bf16x8& b1, bf16x8& b2, bf16x8& b3) {
+  uintx4_t u1, u2, u3;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float a = q < 2 ? lo[2 * q] : hi[2 * q - 4];
+    const float b = q < 2 ? lo[2 * q + 1] : hi[2 * q - 3];
+    unsigned h1, h2, h3;
+    split3_pair(a, b, h1, h2, h3);
+    u1[q] = h1; u2[q] = h2; u3[q] = h3;
+  }
+  b1 = __builtin_bit_cast(bf16x8, u1);
+  b2 = __builtin_bit_cast(bf16x8, u2);
+  b3 = __builtin_bit_cast(bf16x8, u3);
+}
+
+// The terms of |W| from those of W: w2 and w3 change sign with w1.
+__device__ __forceinline__ void abs_terms(bf16x8& w1, bf16x8& w2, bf16x8& w3) {
+  const uintx4_t u1 = __builtin_bit_cast(uintx4_t, w1);
+  const uintx4_t s = u1 & 0x80008000u;
+  w1 = __builtin_bit_cast(bf16x8, u1 ^ s);
+  w2 = __builtin_bit_cast(bf16x8, __builtin_bit_cast(uintx4_t, w2) ^ s);
+  w3 = __builtin_bit_cast(bf16x8, __builtin_bit_cast(uintx4_t, w3) ^ s);
+}
+
+__device__ __forceinline__ floatx4 mfma_bf16(bf16x8 a, bf16x8 b, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// mlp_forward (affine planes) with the split contraction, for nets whose hidden
+// layers are all WMAX wide (padded).  On entry the input planes hold features
+// 0..31, zero padded.
+template <int V, int NB, int NW, int WMAX, int AS, class Fin>
+__device__ __forceinline__ void mlp_forward_split(const DevModelBf16& M, float* __restrict__ X, Fin&& fin) {
+  using PL = Planes<0, V, 0>;
+  constexpr int R = PL::R;
+  constexpr int FTMAX = (WMAX / 16 + NW - 1) / NW;
+  static_assert(NB == 16, "one box tile");
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ln = lane & 15, lg = lane >> 4;
+
+  for (int l = 0; l < M.n_layers; ++l) {
+    const DevLayerBf16& Ly = M.L[l];
+    const int nkb = Ly.in_pad >> 5;
+    const int nft = Ly.out_pad >> 4;
+    const bool last = (l == M.n_layers - 1);
+    const auto* W1 = as_global(Ly.W1);
+    const auto* W2 = as_global(Ly.W2);
+    const auto* W3 = as_global(Ly.W3);
+    floatx4 acc[FTMAX][R][1];
+#pragma unroll
+    for (int f = 0; f < FTMAX; ++f)
+#pragma unroll
+      for (int p = 0; p < R; ++p) acc[f][p][0] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+    __syncthreads();   // layer input complete in X
+
+    auto step = [&](auto nf_tag, int kb, const bf16x8* w1, const bf16x8* w2, const bf16x8* w3)
+        __attribute__((always_inline)) {
+      constexpr int NF = decltype(nf_tag)::value;
+#pragma unroll
+      for (int p = 0; p < R; ++p) {
+        const floatx4 lo = *reinterpret_cast<const floatx4*>(&X[xoff<NB, WMAX>(p, ln, kb * 32 + lg * 8)]);
+        const floatx4 hi = *reinterpret_cast<const floatx4*>(&X[xoff<NB, WMAX>(p, ln, kb * 32 + lg * 8 + 4)]);
+        bf16x8 b1, b2, b3;
+        split_x8(lo, hi, b1, b2, b3);
+        bf16x8 a1[NF], a2[NF], a3[NF];
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+          a1[f] = w1[f]; a2[f] = w2[f]; a3[f] = w3[f];
+          if (PL::absw(p)) abs_terms(a1[f], a2[f], a3[f]);
+        }
+        // Smallest products first, the feature tiles' independent chains
+        // interleaved.  The matrix unit does not round a sum to nearest, which
+        // shows where all terms have one sign (the error plane) and in the
+        // base: there a chunk sums from zero and is added by the vector ALU.
+        const bool fresh = PL::absw(p) || p == 0;
+        floatx4 c[NF];
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+          c[f] = mfma_bf16(a1[f], b3, fresh ? floatx4{0.f, 0.f, 0.f, 0.f} : acc[f][p][0]);
+#pragma unroll
+        for (int f = 0; f < NF; ++f) c[f] = mfma_bf16(a2[f], b2, c[f]);
+#pragma unroll
+        for (int f = 0; f < NF; ++f) c[f] = mfma_bf16(a3[f], b1, c[f]);
+#pragma unroll
+        for (int f = 0; f < NF; ++f) c[f] = mfma_bf16(a1[f], b2, c[f]);
+#pragma unroll
+        for (int f = 0; f < NF; ++f) c[f] = mfma_bf16(a2[f], b1, c[f]);
+#pragma unroll
+        for (int f = 0; f < NF; ++f) c[f] = mfma_bf16(a1[f], b1, c[f]);
+#pragma unroll
+        for (int f = 0; f < NF; ++f) acc[f][p][0] = fresh ? acc[f][p][0] + c[f] : c[f];
+      }
+    };
+    // one chunk of 32 inputs ahead
+    bf16x8 n1[FTMAX], n2[FTMAX], n3[FTMAX];
+    auto fetch = [&](int kb) __attribute__((always_inline)) {
+#pragma unroll
+      for (int f = 0; f < FTMAX; ++f) {
+        const size_t o = (size_t)((wave + f * NW) * nkb + kb) * 64 + lane;
+        n1[f] = W1[o]; n2[f] = W2[o]; n3[f] = W3[o];
+      }
+    };
+    if (!last) {   // a hidden layer: every feature tile of the wave exists
+      fetch(0);
+      for (int kb = 0; kb < nkb; ++kb) {
+        bf16x8 w1[FTMAX], w2[FTMAX], w3[FTMAX];
+#pragma unroll
+        for (int f = 0; f < FTMAX; ++f) { w1[f] = n1[f]; w2[f] = n2[f]; w3[f] = n3[f]; }
+        fetch(kb + 1 < nkb ? kb + 1 : kb);
+        step(std::integral_constant<int, FTMAX>{}, kb, w1, w2, w3);
+      }
+    } else {
+      // the last layer's one tile: its chunks shared out over the waves, the
+      // partial sums added below
+      for (int kb = wave; kb < nkb; kb += NW) {
+        const size_t o = (size_t)kb * 64 + lane;
+        const bf16x8 w1[1] = {W1[o]}, w2[1] = {W2[o]}, w3[1] = {W3[o]};
+        step(std::integral_constant<int, 1>{}, kb, w1, w2, w3);
+      }
+    }
+
+    floatx4 bias4[FTMAX];
+#pragma unroll
+    for (int f = 0; f < FTMAX; ++f) {
+      const int ft = wave + f * NW;
+      if (ft < nft) bias4[f] = *reinterpret_cast<const __attribute__((address_space(1))) floatx4*>(
+                        as_global(Ly.bias) + ft * 16 + lg * 4);
+    }
+    __syncthreads();   // every wave has consumed X
+
+    if (last) {
+      floatx4* Pp = reinterpret_cast<floatx4*>(X);
+      if (wave > 0) {
+#pragma unroll
+        for (int p = 0; p < R; ++p) Pp[((wave - 1) * R + p) * 64 + lane] = acc[0][p][0];
+      }
+      __syncthreads();
+      if (wave == 0) {
+#pragma unroll
+        for (int w = 1; w < NW; ++w)
+#pragma unroll
+          for (int p = 0; p < R; ++p) acc[0][p][0] += Pp[((w - 1) * R + p) * 64 + lane];
+      }
+      __syncthreads();   // partials read before the caller reuses X
+      if (wave == 0 && lg == 0) {
+        float v[R];
+#pragma unroll
+        for (int p = 0; p < R; ++p) v[p] = acc[0][p][0][0] + (PL::bias(p) ? bias4[0][0] : 0.f);
+        fin(v, ln);
+      }
+    } else {
+      layer_epilogue<PL, 0, V, NB, NW, WMAX, AS>(Ly.act, nft, wave, lane, acc, bias4, X);
+    }
+  }
+}
+
+// Classify axis-aligned boxes by the split contraction.  A box goes to the list
+// that k_classify then classifies when its bound lies within kSplitNear * (|base|
+// + radius) of the threshold, is not a number or is too small to judge by, or
+// when the box is smaller than 1/200 of its distance from the origin.
+//
+// The band: the two forms' bounds differ by their rounding alone, which the
+// ReLU crossings amplify by (rounding of a pre-activation) / (its radius), the
+// more the smaller the box.  Largest difference over 131,072 random boxes each
+// of ReLU nets 256x3, 256x6 (He and Xavier) and 512x8, relative to |base| +
+// radius: 1e-6 at half-width 1/16, 1.3e-4 at 1/64, 5e-4 at 1/128; at 1/1000 it
+// reaches 0.2, so boxes that small take the plain kernel.  At 1/128 the band
+// holds 40 times that difference, and 1 % of the boxes of a shallow net (none of
+// a deep one's, whose bounds all span the threshold widely).
+constexpr float kSplitNear = 2e-2f;
+
+template <int V, int NB, int NW, int WMAX, int AS>
+__global__ void __launch_bounds__(NW * 64, 2)
+k_classify_split(const DevModelBf16* __restrict__ Mp, ClassifyArgs a) {
+  using PL = Planes<0, V, 0>;
+  constexpr int NT = NW * 64, R = PL::R;
+  __shared__ float X[R * NB * WMAX];
+  const long long n = a.n_dev ? (long long)(*a.n_dev) : a.n;
+  const long long ntiles = (n + NB - 1) / NB;
+  for (long long tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    const long long i0 = tile * NB;
+    fill_box_inputs<0, V, NB, NT, WMAX>(X, a, i0, n);
+    for (int e = threadIdx.x; e < R * NB * 16; e += NT)   // the chunk's upper half
+      X[xoff<NB, WMAX>(e / (NB * 16), (e / 16) % NB, 16 + (e & 15))] = 0.f;
+    mlp_forward_split<V, NB, NW, WMAX, AS>(*Mp, X, [&](const float* v, int b) {
+      const long long i = i0 + b;
+      if (i >= n) return;
+      float hmin = INFINITY, cmax = 0.f;
+      for (int k = 0; k < a.d; ++k) {
+        const float l = a.lower[i * a.d + k], u = a.upper[i * a.d + k];
+        hmin = fminf(hmin, 0.5f * (u - l));
+        cmax = fmaxf(cmax, fmaxf(fabsf(l), fabsf(u)));
+      }
+      float lo, hi, scale;
+      final_bounds<0, V>(v, lo, hi, scale);
+      a.codes[i] = sign_code(lo, hi, a.offset);
+      const float tol = kSplitNear * scale;
+      const bool clear = fabsf(lo - a.offset) > tol && fabsf(hi + a.offset) > tol && scale > 1e-20f &&
+                         scale < 1e30f && hmin >= kSplitMinSize * cmax;
+      if (!clear) {
+        const int slot = atomicAdd(a.list_n, 1);
+        if (slot < a.list_cap) a.list[slot] = (int)i;
+      }
+    });
+  }
+}
