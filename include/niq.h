@@ -178,6 +178,19 @@ size_t niq_tree_counters_bytes(void);
 niq_status niq_tree_decode(const void* host_counters, const niq_tree_params* p,
                            niq_tree_result* res);
 
+/* The node lists of a finished build in the arrays the reference returns
+ * (src/kd_tree.py:202-218): the first min(n, size) rows of lower and upper, zero
+ * rows up to `size`, and the valid mask (bytes 0 and 1).  Up to 3 lists in one
+ * launch; sizes at least 0, null outputs only at size 0.  Asynchronous on
+ * `stream`. */
+typedef struct niq_tree_list {
+  const float* lower; const float* upper;       /* (n, 3) device */
+  int64_t n, size;
+  float* out_lower; float* out_upper;           /* (size, 3) device */
+  uint8_t* out_valid;                           /* (size,) device */
+} niq_tree_list;
+niq_status niq_tree_export(const niq_tree_list* lists, int n_lists, void* stream);
+
 /* ---- ray casting ------------------------------------------------------------
  * Replaces cast_rays / cast_rays_iter (src/queries.py:134-175, 39-132) with the
  * options of get_default_cast_opts (src/queries.py:23-36). */

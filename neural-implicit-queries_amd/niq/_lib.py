@@ -26,7 +26,7 @@ PREC = {"fp32": 0, "bf16": 1}
 EXPORTS = ("niq_model_create", "niq_model_destroy", "niq_model_device_bytes",
            "niq_classify_boxes", "niq_classify_general_boxes", "niq_tile_shape", "niq_eval_points",
            "niq_tree_workspace_bytes", "niq_tree_build", "niq_tree_enqueue",
-           "niq_tree_counters_bytes", "niq_tree_decode", "niq_cast_workspace_bytes",
+           "niq_tree_counters_bytes", "niq_tree_decode", "niq_tree_export", "niq_cast_workspace_bytes",
            "niq_cast_rays", "niq_cast_rays_frustum", "niq_find_any_intersection", "niq_closest_point",
            "niq_sample_workspace_bytes", "niq_sample_surface_nodes", "niq_bulk_sums_nodes",
            "niq_camera_rays", "niq_hit_positions", "niq_outward_normals", "niq_shade_image", "niq_mc_extract", "niq_mc_table",
@@ -71,6 +71,12 @@ class TreeResult(ctypes.Structure):
                 ("n_recheck", ctypes.c_int64), ("n_levels", ctypes.c_int),
                 ("level_n", ctypes.c_int32 * 64), ("level_interior", ctypes.c_int32 * 64),
                 ("level_exterior", ctypes.c_int32 * 64)]
+
+
+class TreeList(ctypes.Structure):
+    _fields_ = [("lower", ctypes.c_void_p), ("upper", ctypes.c_void_p),
+                ("n", ctypes.c_int64), ("size", ctypes.c_int64),
+                ("out_lower", ctypes.c_void_p), ("out_upper", ctypes.c_void_p), ("out_valid", ctypes.c_void_p)]
 
 
 class CastOpts(ctypes.Structure):
@@ -136,6 +142,7 @@ def load_library():
         "niq_tree_enqueue": (I, [P, P, P, P, S, P, ctypes.POINTER(S), P]),
         "niq_tree_counters_bytes": (S, []),
         "niq_tree_decode": (I, [P, P, P]),
+        "niq_tree_export": (I, [P, I, P]),
         "niq_cast_workspace_bytes": (S, [P]),
         "niq_cast_rays": (I, [P, I, P, P, P, I64, P, P, P, P, P, S, ctypes.POINTER(I64), P]),
         "niq_closest_point": (I, [P, P, P, P, P, I64, F, I, P, P, ctypes.POINTER(I64), P]),
@@ -179,18 +186,27 @@ def check(status):
         raise NiqError(status, msg)
 
 
+_gpu_seen = False   # once visible, the GPU stays so for the process
+
+
 def require_gpu():
+    global _gpu_seen
+    if _gpu_seen:
+        return
     if not torch.cuda.is_available():
         raise RuntimeError("niq needs a ROCm GPU (gfx950); none is visible")
+    _gpu_seen = True
 
 
+# Pointers and streams go to the library as plain integers (the argument types
+# above convert them).
 def stream_handle(stream=None):
     s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    return s.cuda_stream
 
 
 def ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
+    return t.data_ptr() if t is not None else None
 
 
 def eval_cfg(mode="affine_fixed", precision="fp32", truncate_count=0, n_append=0, recheck_tol=0.0, variant=0,

@@ -23,6 +23,9 @@ def as_device_f32(x):
     """float32, contiguous, on the current GPU."""
     if isinstance(x, torch.Tensor):
         t = x.detach()
+        if t.dtype is torch.float32 and t.is_cuda and t.is_contiguous() and \
+                t.device.index == torch.cuda.current_device():
+            return t
     else:
         t = torch.as_tensor(np.asarray(x, dtype=np.float32))
     return t.to(device="cuda", dtype=torch.float32).contiguous()
@@ -43,10 +46,11 @@ class ImplicitFunction:
         x = as_device_f32(x)
         single = x.dim() == 1
         xb = x.reshape(1, -1) if single else x
-        out = torch.empty(xb.shape[0], dtype=torch.float32, device=xb.device)
+        n, d = xb.shape
+        out = torch.empty(n, dtype=torch.float32, device=xb.device)
         m = _mlp.device_model(params)
         _lib.check(_lib.load_library().niq_eval_points(
-            m.handle, _lib.ptr(xb), xb.shape[0], xb.shape[1], _lib.ptr(out), _lib.stream_handle()))
+            m.handle, _lib.ptr(xb), n, d, _lib.ptr(out), _lib.stream_handle()))
         return out[0] if single else out
 
     # -- classification -----------------------------------------------------

@@ -10,6 +10,7 @@ ordering rules).
 """
 import ctypes
 
+import numpy as np
 import torch
 
 from . import _lib
@@ -29,12 +30,11 @@ def _finished_size(level_counts, level_finished, B):
     return size
 
 
-def _pad_rows(src, n, size):
-    out = torch.zeros((size, 3), dtype=torch.float32, device=src.device)
-    m = min(n, size)
-    if m > 0:
-        out[:m] = src[:m]
-    return out
+def _corner(v):
+    """A box corner as a list of floats."""
+    if isinstance(v, np.ndarray):
+        return [float(x) for x in v.reshape(-1).tolist()]
+    return [float(x) for x in torch.as_tensor(v).reshape(-1).tolist()]
 
 
 def tree_request(func, params, lower, upper, node_terminate_thresh=None, split_depth=None,
@@ -48,8 +48,7 @@ def tree_request(func, params, lower, upper, node_terminate_thresh=None, split_d
         raise ValueError("must specify at least one of node_terminate_thresh or split_depth as a terminating condition")
     _lib.require_gpu()
     m = _mlp.device_model(params)
-    lower = [float(v) for v in torch.as_tensor(lower).reshape(-1).tolist()]
-    upper = [float(v) for v in torch.as_tensor(upper).reshape(-1).tolist()]
+    lower, upper = _corner(lower), _corner(upper)
     if len(lower) != 3 or len(upper) != 3:
         raise ValueError("the level-set tree is built over 3D boxes")
     p = _lib.TreeParams()
@@ -96,24 +95,24 @@ class TreeBuffers:
         level_n = list(r.level_n[:n_lv])
         B = int(p.batch_process_size)
         n_unk = int(r.n_unknown)
-        bucket = get_next_bucket_size(n_unk)
-        out = {
-            'unknown_node_valid': torch.arange(bucket, device=dev) < n_unk,
-            'unknown_node_lower': _pad_rows(self.unk[0], n_unk, bucket),
-            'unknown_node_upper': _pad_rows(self.unk[1], n_unk, bucket),
-        }
+        lists = [('unknown', self.unk, n_unk, get_next_bucket_size(n_unk))]
         if self.fin_i is not None:
-            n = int(r.n_interior)
-            size = _finished_size(level_n, list(r.level_interior[:n_lv]), B)
-            out['interior_node_valid'] = torch.arange(size, device=dev) < n
-            out['interior_node_lower'] = _pad_rows(self.fin_i[0], n, size)
-            out['interior_node_upper'] = _pad_rows(self.fin_i[1], n, size)
+            lists.append(('interior', self.fin_i, int(r.n_interior),
+                          _finished_size(level_n, list(r.level_interior[:n_lv]), B)))
         if self.fin_e is not None:
-            n = int(r.n_exterior)
-            size = _finished_size(level_n, list(r.level_exterior[:n_lv]), B)
-            out['exterior_node_valid'] = torch.arange(size, device=dev) < n
-            out['exterior_node_lower'] = _pad_rows(self.fin_e[0], n, size)
-            out['exterior_node_upper'] = _pad_rows(self.fin_e[1], n, size)
+            lists.append(('exterior', self.fin_e, int(r.n_exterior),
+                          _finished_size(level_n, list(r.level_exterior[:n_lv]), B)))
+        out = {}
+        arr = (_lib.TreeList * len(lists))()
+        for a, (name, src, n, size) in zip(arr, lists):
+            valid = torch.empty(size, dtype=torch.bool, device=dev)
+            lo = torch.empty((size, 3), dtype=torch.float32, device=dev)
+            up = torch.empty((size, 3), dtype=torch.float32, device=dev)
+            out[name + '_node_valid'], out[name + '_node_lower'], out[name + '_node_upper'] = valid, lo, up
+            p0 = src.data_ptr()
+            a.lower, a.upper, a.n, a.size = p0, p0 + 12 * src.shape[1], n, size
+            a.out_lower, a.out_upper, a.out_valid = lo.data_ptr(), up.data_ptr(), valid.data_ptr()
+        _lib.check(_lib.load_library().niq_tree_export(arr, len(lists), _lib.stream_handle()))
         stats = {"n_classified": int(r.n_classified), "n_unknown": n_unk,
                  "n_interior": int(r.n_interior), "n_exterior": int(r.n_exterior),
                  "n_recheck": int(r.n_recheck), "level_counts": level_n}

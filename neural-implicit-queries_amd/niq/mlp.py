@@ -243,7 +243,7 @@ def _fingerprint(params):
     identity, shape and dtype of each array.  Replacing an entry changes it;
     writing into an array in place does not (params are treated as immutable,
     as JAX arrays are in the reference)."""
-    return tuple((k, id(v), getattr(v, "shape", None), str(getattr(v, "dtype", ""))) for k, v in params.items())
+    return [(k, id(v), getattr(v, "shape", None), getattr(v, "dtype", None)) for k, v in params.items()]
 
 
 def device_model(params):
