@@ -314,7 +314,13 @@ niq_status niq_classify_general_boxes(const niq_model* m, const niq_eval_cfg* cf
 niq_status niq_eval_points(const niq_model* m, const float* x, int64_t n, int d, float* out, void* stream) {
   if (niq_status st = check_model(m, d)) return st;
   if (n < 0 || (n > 0 && (!x || !out))) return fail(NIQ_ERR_INVALID, "bad buffers");
-  hipStream_t s = (hipStream_t)stream;
+  if (points_split_eligible(m)) return points_split(m, x, d, n, out, (hipStream_t)stream);
+  return points_plain(m, x, d, n, out, (hipStream_t)stream);
+}
+
+}  // extern "C"
+
+niq_status niqi::points_plain(const niq_model* m, const float* x, int d, long long n, float* out, hipStream_t s) {
   switch (m->wt) {
     case 32: return launch_points_w<32>(m, x, d, n, out, s);
     case 64: return launch_points_w<64>(m, x, d, n, out, s);
@@ -325,5 +331,3 @@ niq_status niq_eval_points(const niq_model* m, const float* x, int64_t n, int d,
   return fail(NIQ_ERR_UNSUPPORTED, "width");
 }
 
-
-}  // extern "C"

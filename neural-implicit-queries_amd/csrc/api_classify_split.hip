@@ -21,7 +21,44 @@ niq_status launch_split_w(const niq_model* m, const ClassifyArgs& a, long long m
   return NIQ_OK;
 }
 
+// 64 points a workgroup: 4 point tiles share a wave's weight fragments.
+template <int W, int AS>
+niq_status launch_points_split_w(const niq_model* m, const float* x, int d, long long n, float* out, hipStream_t s) {
+  constexpr int NB = 64, NW = SplitTile<W>::NW;
+  auto k = k_points_split<NB, NW, W, AS>;
+  const long long tiles = (n + NB - 1) / NB;
+  if (tiles == 0) return NIQ_OK;
+  hipLaunchKernelGGL(k, dim3(grid_for(tiles, persistent_blocks(k, NW * 64))), dim3(NW * 64), 0, s, m->dev16, m->dev,
+                     x, d, n, out);
+  HIPCHK(hipGetLastError());
+  return NIQ_OK;
+}
+
+template <int W>
+niq_status launch_points_split(const niq_model* m, const float* x, int d, long long n, float* out, hipStream_t s) {
+  if (m->relu_only) return launch_points_split_w<W, ACTS_RELU>(m, x, d, n, out, s);
+  return launch_points_split_w<W, ACTS_ALL>(m, x, d, n, out, s);
+}
+
+// Every hidden layer fills the template width, the widths where the contraction
+// is the cost.
+bool split_shape(const niq_model* m) {
+  for (int i = 1; i < m->n_layers; ++i)
+    if (round32(m->dims[i]) != m->wt) return false;
+  return m->n_layers > 1 && m->bf16_ok && m->bounded && m->wt >= 256 && m->wt16 == m->wt;
+}
+
 }  // namespace
+
+bool niqi::points_split_eligible(const niq_model* m) { return split_shape(m); }
+
+niq_status niqi::points_split(const niq_model* m, const float* x, int d, long long n, float* out, hipStream_t s) {
+  switch (m->wt) {
+    case 256: return launch_points_split<256>(m, x, d, n, out, s);
+    case 512: return launch_points_split<512>(m, x, d, n, out, s);
+  }
+  return fail(NIQ_ERR_UNSUPPORTED, "width");
+}
 
 // Widths 256 and 512, where the contraction is the cost (131,072 boxes of the
 // 256x6 net 3.46 ms by FP32 matrix instructions, 2.07 split; of the 512x8 net
@@ -32,9 +69,7 @@ bool niqi::split_eligible(const niq_model* m, const niq_eval_cfg* cfg) {
   if (cfg && (cfg->mode != NIQ_MODE_AFFINE_FIXED || cfg->precision != NIQ_PREC_FP32 || cfg->recheck_tol > 0.f ||
               cfg->variant > 1))
     return false;
-  for (int i = 1; i < m->n_layers; ++i)
-    if (round32(m->dims[i]) != m->wt) return false;   // every feature tile in use
-  return m->n_layers > 1 && m->relu_only && m->bias_small && m->bf16_ok && m->in_dim == 3 && m->wt >= 256 && m->wt16 == m->wt;
+  return split_shape(m) && m->relu_only && m->bias_small && m->in_dim == 3;
 }
 
 niq_status niqi::classify_split(const niq_model* m, const ClassifyArgs& a, long long max_n, hipStream_t s) {

@@ -339,7 +339,7 @@ extern "C" niq_status niq_mc_extract(const niq_model* m, const float* leaf_lower
     const long long npts = nl * np3;
     hipLaunchKernelGGL(k_mc_grid, dim3((unsigned)std::min<long long>((npts + 255) / 256, 65535)), dim3(256), 0, s,
                        leaf_lower, leaf_upper, l0, nl, sd, (float*)ppts);
-    if ((st = niq_eval_points(m, (const float*)ppts, npts, 3, (float*)pvals, s))) break;
+    if ((st = points_plain(m, (const float*)ppts, 3, npts, (float*)pvals, s))) break;
     const unsigned gl = (unsigned)std::min<long long>(nl, 65535);
     hipLaunchKernelGGL(k_mc_count, dim3(gl), dim3(256), 0, s, T, (const float*)pvals, nl, sd, (long long*)pcnt);
     hipLaunchKernelGGL(k_scan_i64, dim3(1), dim3(1024), 0, s, (const long long*)pcnt, nl, written,

@@ -94,6 +94,18 @@ niq_status niq_model_create(int n_layers, const int* dims, const int* acts, cons
     if (b && b[0]) b2 += (double)b[0][f] * (double)b[0][f];
   }
   m->bias_small = b2 <= 64.0 * w2;
+  // largest magnitude a layer's sum can take on inputs up to 1e6
+  double mag = 1e6;
+  for (int i = 0; i < n_layers; ++i) {
+    double next = 0.0;
+    for (int f = 0; f < dims[i + 1]; ++f) {
+      double sum = (b && b[i]) ? std::fabs((double)b[i][f]) : 0.0;
+      for (int k = 0; k < dims[i]; ++k) sum += mag * std::fabs((double)W[i][(size_t)k * dims[i + 1] + f]);
+      next = std::isnan(sum) ? INFINITY : std::max(next, sum);
+    }
+    mag = std::max(next, 1.0);   // (and activations of magnitude 1)
+  }
+  m->bounded = mag < 1e30;
   hipError_t e = hipMalloc(&m->weights, total);
   if (e == hipSuccess) e = hipMemcpy(m->weights, host.data(), total, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&m->dev), sizeof(DevModel));

@@ -134,6 +134,7 @@ struct niq_model {
   bool relu_only = false;      // every hidden activation is ReLU
   bool tanh_only = false;      // every hidden activation is TanH
   bool elu_only = false;       // every hidden activation is ELU
+  bool bounded = false;        // activations below 1e30 on inputs up to 1e6 (split contraction)
   bool bias_small = false;     // first-layer biases are small beside the weights (split contraction)
   DevModelBf16 host16;         // precision-mode copy (bf16 hi/lo/|W| weights)
   DevModelBf16* dev16 = nullptr;
@@ -189,6 +190,12 @@ niq_status classify_rows(const niq_model* m, const niq_eval_cfg* cfg, const Clas
 // split_eligible(m, cfg).  Defined in api_classify_split.hip.
 bool split_eligible(const niq_model* m, const niq_eval_cfg* cfg);
 niq_status classify_split(const niq_model* m, const ClassifyArgs& a, long long max_n, hipStream_t s);
+// Point values by the FP32 matrix instructions (api_classify.hip).  Marching
+// cubes samples with these: its cells' signs, and so its triangles, are theirs.
+niq_status points_plain(const niq_model* m, const float* x, int d, long long n, float* out, hipStream_t s);
+// Point values by the split contraction (points_split_eligible(m)).
+bool points_split_eligible(const niq_model* m);
+niq_status points_split(const niq_model* m, const float* x, int d, long long n, float* out, hipStream_t s);
 // ... with the optional FP64 re-test list in stream-ordered scratch.
 niq_status classify_with_recheck(const niq_model* m, const niq_eval_cfg* cfg, int nvec, ClassifyArgs a,
                                  long long n, hipStream_t s);
