@@ -47,14 +47,20 @@ niq_status launch_rays_v(int wt, const DevModel* models, const RayArgs& a, long 
   return fail(NIQ_ERR_UNSUPPORTED, "width");
 }
 
-// relu_only: every model of the cast has only ReLU hidden layers; the default
-// affine_fixed tile then runs the kernel compiled for ReLU alone
-// (bit-identical, fewer registers).
+// acts: the one activation of every model of the cast, or ACTS_ALL; the default
+// affine_fixed tile then runs the kernel compiled for it alone (bit-identical,
+// fewer registers).
 template <int KIND, int V>
-niq_status launch_rays(int wt, int variant, bool relu_only, const DevModel* models, const RayArgs& a,
+niq_status launch_rays(int wt, int variant, int acts, const DevModel* models, const RayArgs& a,
                        long long n_rays, hipStream_t s) {
   if constexpr (KIND == 0 && V == 1) {
-    if (variant == 0 && relu_only) return launch_rays_v<KIND, V, 0, ACTS_RELU>(wt, models, a, n_rays, s);
+    if (variant == 0) {
+      switch (acts) {
+        case ACTS_RELU: return launch_rays_v<KIND, V, 0, ACTS_RELU>(wt, models, a, n_rays, s);
+        case ACTS_TANH: return launch_rays_v<KIND, V, 0, ACTS_TANH>(wt, models, a, n_rays, s);
+        case ACTS_ELU: return launch_rays_v<KIND, V, 0, ACTS_ELU>(wt, models, a, n_rays, s);
+      }
+    }
   }
   switch (variant) {
     case 0: return launch_rays_v<KIND, V, 0>(wt, models, a, n_rays, s);
@@ -235,11 +241,13 @@ niq_status cast_run_groups(CastGroupReq* reqs, int ng, const niq_eval_cfg* cfg, 
   }
   long long n_rays = 0;
   int m0 = 0;
-  bool relu = true;
+  bool relu = true, tanh = true, elu = true;
   for (int g = 0; g < ng; ++g) {
     const CastGroupReq& r = reqs[g];
     for (int f = 0; f < r.n_models; ++f) {
       relu = relu && r.models[f]->relu_only;
+      tanh = tanh && r.models[f]->tanh_only;
+      elu = elu && r.models[f]->elu_only;
       ht[m0 + f] = r.models[f]->host;
       if (bf16) ht16[m0 + f] = r.models[f]->host16;
     }
@@ -272,15 +280,16 @@ niq_status cast_run_groups(CastGroupReq* reqs, int ng, const niq_eval_cfg* cfg, 
   if (st == NIQ_OK)
     hipfail(hipMemcpyAsync(gtab, hg, sizeof(RayGroup) * ng, hipMemcpyHostToDevice, s), "group table");
   if (st == NIQ_OK && n_rays > 0) {
+    const int acts = relu ? ACTS_RELU : (tanh ? ACTS_TANH : (elu ? ACTS_ELU : ACTS_ALL));
     RayArgs a{};
     a.groups = gtab;
     a.n_groups = ng;
     if (bf16) st = mode == NIQ_MODE_AFFINE_FIXED ? launch_rays_bf16<1>(wt16, relu, table16, a, n_rays, s)
                                                  : launch_rays_bf16<0>(wt16, relu, table16, a, n_rays, s);
-    else if (mode == NIQ_MODE_AFFINE_FIXED) st = launch_rays<0, 1>(wt, rv, relu, table, a, n_rays, s);
-    else if (mode == NIQ_MODE_INTERVAL) st = launch_rays<0, 0>(wt, rv, relu, table, a, n_rays, s);
-    else if (mode == NIQ_MODE_SLOPE_INTERVAL) st = launch_rays<1, 1>(wt, rv, relu, table, a, n_rays, s);
-    else st = launch_rays<2, 0>(wt, rv, relu, table, a, n_rays, s);
+    else if (mode == NIQ_MODE_AFFINE_FIXED) st = launch_rays<0, 1>(wt, rv, acts, table, a, n_rays, s);
+    else if (mode == NIQ_MODE_INTERVAL) st = launch_rays<0, 0>(wt, rv, acts, table, a, n_rays, s);
+    else if (mode == NIQ_MODE_SLOPE_INTERVAL) st = launch_rays<1, 1>(wt, rv, acts, table, a, n_rays, s);
+    else st = launch_rays<2, 0>(wt, rv, acts, table, a, n_rays, s);
   }
   long long hb_fix[2 * 1];
   std::vector<long long> hb_vec;
