@@ -16,9 +16,11 @@ niq_status launch_cp_round_w(const niq_model* m, CpState* S, const CpArgs& a, hi
   if constexpr (!Fits<Planes<KIND, V, 0>::R, 16, W>::value) {
     return fail(NIQ_ERR_UNSUPPORTED, "closest_point round: box planes above LDS");
   } else {
-    constexpr int NW = TileCfgWide<W>::NW;
-    const long long g_box = (a.B + 15) / 16, g_pts = (7LL * a.B + 15) / 16;
-    hipLaunchKernelGGL((k_cp_forward<KIND, V, NW, W, AS>), dim3((unsigned)(g_box + g_pts)), dim3(NW * 64), 0, s,
+    // width 32: box tiles of two waves (one a feature tile) and point tiles of
+    // one, so that every wave has work and each about a SIMD to itself
+    constexpr int NW = W == 32 ? 2 : TileCfgWide<W>::NW, PW = W == 32 ? 1 : NW;
+    const long long g_box = (a.B + 15) / 16, g_pts = (7LL * a.B + 16 * (NW / PW) - 1) / (16 * (NW / PW));
+    hipLaunchKernelGGL((k_cp_forward<KIND, V, NW, PW, W, AS>), dim3((unsigned)(g_box + g_pts)), dim3(NW * 64), 0, s,
                        m->dev, S, a, (int)g_box);
     hipLaunchKernelGGL(k_cp_update, dim3(1), dim3(1024), 0, s, S, a);
     HIPCHK(hipGetLastError());
@@ -120,7 +122,7 @@ extern "C" niq_status niq_closest_point(const niq_model* m, const niq_eval_cfg* 
   auto hipfail = [&](hipError_t e, const char* what) {
     if (e != hipSuccess && st == NIQ_OK) st = fail(NIQ_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e));
   };
-  void *pS, *pbq, *pblo, *pbup, *ppts, *pcodes, *pvals, *pwin, *pidist, *pineeds;
+  void *pS, *pbq, *pblo, *pbup, *ppts, *pcodes, *pvals, *pwin, *pidist, *pineeds, *pbdc;
   own(sizeof(CpState), &pS);
   own(sizeof(int) * B, &pbq);
   own(sizeof(float) * 3 * B, &pblo);
@@ -131,6 +133,7 @@ extern "C" niq_status niq_closest_point(const niq_model* m, const niq_eval_cfg* 
   own(sizeof(int) * Q, &pwin);
   own(sizeof(float) * B, &pidist);
   own(sizeof(int) * B, &pineeds);
+  own(sizeof(float) * B, &pbdc);
   CpArgs a{};
   void *pwq = nullptr, *pwlo = nullptr, *pwup = nullptr;
   if (st == NIQ_OK) hipfail(al(sizeof(int) * cap, &pwq), "closest_point: hipMallocAsync");
@@ -150,7 +153,7 @@ extern "C" niq_status niq_closest_point(const niq_model* m, const niq_eval_cfg* 
   a.bq = (int*)pbq; a.blo = (float*)pblo; a.bup = (float*)pbup; a.pts = (float*)ppts;
   a.codes = (int*)pcodes; a.vals = (float*)pvals; a.q = query_points; a.Q = Q;
   a.qmin = out_dist; a.qloc = out_loc; a.win = (int*)pwin;
-  a.idist = (float*)pidist; a.ineeds = (int*)pineeds;
+  a.idist = (float*)pidist; a.ineeds = (int*)pineeds; a.bdc = (float*)pbdc;
   // eps / sqrt(d) in float32 (src/kd_tree.py:688)
   a.eps_cube_width = eps / sqrtf(3.0f);
   CpState* S = (CpState*)pS;

@@ -41,8 +41,36 @@ struct CpArgs {
   float* qloc;                  // (Q, 3)
   int* win;                     // (Q,) scratch, -1 between rounds
   float* idist; int* ineeds;    // per-item scratch (B,)
+  float* bdc;                   // (B,) distance of the query to the node's centre
   float eps_cube_width;
 };
+
+__device__ __forceinline__ float norm3(float x, float y, float z) { return sqrtf((x * x + y * y) + z * z); }
+
+// Three packed floats, moved as one access.
+struct F3 { float v[3]; };
+__device__ __forceinline__ F3 load3(const float* p) {
+  F3 r;
+  __builtin_memcpy(&r, p, sizeof(r));
+  return r;
+}
+
+// Item j of the batch: its stack row s copied to the batch buffers, with the
+// distance of its query to the node's centre (formed here, where the update
+// would wait for the query's index first).
+__device__ __forceinline__ void cp_copy_item(const CpArgs& a, long long s, long long j, float* lo, float* up) {
+  const int qid = a.wq[s];
+  const F3 l = load3(a.wlo + 3 * s), u = load3(a.wup + 3 * s), q = load3(a.q + 3LL * qid);
+  float c[3];
+  for (int k = 0; k < 3; ++k) {
+    lo[k] = l.v[k]; up[k] = u.v[k];
+    c[k] = 0.5f * (lo[k] + up[k]);
+  }
+  a.bq[j] = qid;
+  __builtin_memcpy(a.blo + 3 * j, &l, sizeof(l));
+  __builtin_memcpy(a.bup + 3 * j, &u, sizeof(u));
+  a.bdc[j] = norm3(q.v[0] - c[0], q.v[1] - c[1], q.v[2] - c[2]);
+}
 
 // Pop the top B items into the batch buffers and form their sample points
 // (src/kd_tree.py:679-686, 703-704).
@@ -52,11 +80,9 @@ static __global__ void __launch_bounds__(256) k_cp_gather(CpState* S, CpArgs a) 
   const int n = top - pop;
   for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
     const long long s = pop + j;
-    a.bq[j] = a.wq[s];
     float lo[3], up[3], c[3], e[3];
+    cp_copy_item(a, s, j, lo, up);
     for (int k = 0; k < 3; ++k) {
-      lo[k] = a.wlo[3 * s + k]; up[k] = a.wup[3 * s + k];
-      a.blo[3 * j + k] = lo[k]; a.bup[3 * j + k] = up[k];
       c[k] = 0.5f * (lo[k] + up[k]);
       e[k] = up[k] - lo[k];
     }
@@ -75,8 +101,6 @@ static __global__ void __launch_bounds__(256) k_cp_gather(CpState* S, CpArgs a) 
     if (n > 0) S->rounds += 1;
   }
 }
-
-__device__ __forceinline__ float norm3(float x, float y, float z) { return sqrtf((x * x + y * y) + z * z); }
 
 // A value another thread of this round changed with an atomic, read past the
 // caches (device scope).
@@ -97,35 +121,37 @@ __device__ __forceinline__ void cp_push_children(const CpArgs& a, int pop, int r
   const float mid = 0.5f * (lo[dim] + up[dim]);
   const long long pa = (long long)pop + 2LL * r, pb = pa + 1;
   if (pb < a.cap) {
+    float l2[6], u2[6];   // rows pa and pb are adjacent
     for (int k = 0; k < 3; ++k) {
-      a.wlo[3 * pa + k] = lo[k];
-      a.wup[3 * pa + k] = (k == dim) ? mid : up[k];
-      a.wlo[3 * pb + k] = (k == dim) ? mid : lo[k];
-      a.wup[3 * pb + k] = up[k];
+      l2[k] = lo[k];
+      u2[k] = (k == dim) ? mid : up[k];
+      l2[3 + k] = (k == dim) ? mid : lo[k];
+      u2[3 + k] = up[k];
     }
-    a.wq[pa] = qid;
-    a.wq[pb] = qid;
+    __builtin_memcpy(a.wlo + 3 * pa, l2, sizeof(l2));
+    __builtin_memcpy(a.wup + 3 * pa, u2, sizeof(u2));
+    const int q2[2] = {qid, qid};
+    __builtin_memcpy(a.wq + pa, q2, sizeof(q2));
   }
 }
 
 // The per-item part of the update: the distance the item offers its query
 // (its centre distance plus the node diagonal when the samples change sign)
 // and whether it is subdivided (src/kd_tree.py:692-716).
-__device__ __forceinline__ void cp_item(const CpArgs& a, int j, int qid, const float* lo, const float* up,
-                                        float qmin_pre, float& idist, int& needs) {
-  float c[3], e[3];
-  for (int k = 0; k < 3; ++k) { c[k] = 0.5f * (lo[k] + up[k]); e[k] = up[k] - lo[k]; }
+struct CpVals { float v[7]; };
+__device__ __forceinline__ void cp_item(const CpArgs& a, int code, const CpVals& vals, float dc, const float* lo,
+                                        const float* up, float qmin_pre, float& idist, int& needs) {
+  float e[3];
+  for (int k = 0; k < 3; ++k) e[k] = up[k] - lo[k];
   const float width = fmaxf(fmaxf(e[0], e[1]), e[2]);
   const float diag = norm3(e[0], e[1], e[2]);
-  const float dc = norm3(a.q[3 * qid] - c[0], a.q[3 * qid + 1] - c[1], a.q[3 * qid + 2] - c[2]);
   const bool is_small = width < a.eps_cube_width;
-  const int code = a.codes[j];
   const bool outside = code == CODE_NEGATIVE || code == CODE_POSITIVE;
   bool all_neg = true, all_pos = true;
+#pragma unroll
   for (int t = 0; t < 7; ++t) {
-    const float v = a.vals[7 * j + t];
-    all_neg = all_neg && (v < 0.f);
-    all_pos = all_pos && (v > 0.f);
+    all_neg = all_neg && (vals.v[t] < 0.f);
+    all_pos = all_pos && (vals.v[t] > 0.f);
   }
   idist = !(all_neg || all_pos) ? dc + diag : INFINITY;
   needs = (!outside && !is_small && dc < qmin_pre) ? 1 : 0;
@@ -136,7 +162,7 @@ __device__ __forceinline__ void cp_item(const CpArgs& a, int j, int qid, const f
 // instead of scattered L2 atomics and reads per item).
 constexpr int kCpLdsQ = 4096;
 
-// The update for n <= 2 NT items (the default batch of 2048 on 1024
+// The update for batches of up to 2 NT items (the default batch of 2048 on 1024
 // threads): item j = threadIdx + k NT stays in thread registers through all
 // phases, and the stable compaction scans slice k = 0, 1 in turn, so ranks
 // follow the item order as in cp_update_body.  With at most kCpLdsQ queries
@@ -144,29 +170,42 @@ constexpr int kCpLdsQ = 4096;
 // min over non-negative float bits, max item index) in the same phases, so
 // the results are those of the global form.
 template <int NT>
-__device__ __forceinline__ void cp_update_regs(CpState* S, const CpArgs& a, int n, int pop) {
+__device__ __forceinline__ void cp_update_regs(CpState* S, const CpArgs& a) {
   using Scan = rocprim::block_scan<int, NT>;
   __shared__ typename Scan::storage_type scan_storage;
   __shared__ float s_qmin[kCpLdsQ];
   __shared__ int s_win[kCpLdsQ];
   const bool lds = a.Q <= kCpLdsQ;   // uniform
   const int nq = (int)a.Q;
+  // Every item's inputs and the round's counts in one round trip: rows up to
+  // B exist whatever the count, so the loads need not wait for it.
+  constexpr int KI = 2;
+  const int n = S->n, pop = S->pop;
+  int qid[KI], needs[KI], code[KI];
+  float lo[KI][3], up[KI][3], idist[KI], dc[KI];
+  CpVals vals[KI];
+#pragma unroll
+  for (int k = 0; k < KI; ++k) {
+    const int j = min((int)threadIdx.x + k * NT, a.B - 1);
+    qid[k] = a.bq[j];
+    const F3 l = load3(a.blo + 3 * j), u = load3(a.bup + 3 * j);
+    for (int d = 0; d < 3; ++d) { lo[k][d] = l.v[d]; up[k][d] = u.v[d]; }
+    dc[k] = a.bdc[j];
+    code[k] = a.codes[j];
+    __builtin_memcpy(&vals[k], a.vals + 7 * j, sizeof(CpVals));
+  }
   if (lds) {
     for (int i = threadIdx.x; i < nq; i += NT) { s_qmin[i] = a.qmin[i]; s_win[i] = -1; }
     __syncthreads();
   }
-  constexpr int KI = 2;
-  int qid[KI], needs[KI];
-  float lo[KI][3], up[KI][3], idist[KI];
+  if (n == 0) return;   // uniform
 #pragma unroll
   for (int k = 0; k < KI; ++k) {
     const int j = threadIdx.x + k * NT;
-    needs[k] = 0; idist[k] = INFINITY; qid[k] = 0;
+    needs[k] = 0; idist[k] = INFINITY;
     if (j < n) {
-      qid[k] = a.bq[j];
-      for (int d = 0; d < 3; ++d) { lo[k][d] = a.blo[3 * j + d]; up[k][d] = a.bup[3 * j + d]; }
       const float pre = lds ? s_qmin[qid[k]] : load_fresh(&a.qmin[qid[k]]);
-      cp_item(a, j, qid[k], lo[k], up[k], pre, idist[k], needs[k]);
+      cp_item(a, code[k], vals[k], dc[k], lo[k], up[k], pre, idist[k], needs[k]);
     }
   }
   __syncthreads();   // every pre-round minimum is read before the scatter
@@ -219,10 +258,6 @@ __device__ __forceinline__ void cp_update_regs(CpState* S, const CpArgs& a, int 
 // the stable compaction with the interleaved push at the pop position.
 template <int NT>
 __device__ __forceinline__ void cp_update_body(CpState* S, const CpArgs& a, int n, int pop) {
-  if (n <= 2 * NT) {
-    cp_update_regs<NT>(S, a, n, pop);
-    return;
-  }
   using Scan = rocprim::block_scan<int, NT>;
   __shared__ typename Scan::storage_type scan_storage;
   // phase 1: per-item distance and subdivision flag (pruning uses the minimum
@@ -232,7 +267,9 @@ __device__ __forceinline__ void cp_update_body(CpState* S, const CpArgs& a, int 
     for (int k = 0; k < 3; ++k) { lo[k] = a.blo[3 * j + k]; up[k] = a.bup[3 * j + k]; }
     float idist;
     int needs;
-    cp_item(a, j, a.bq[j], lo, up, load_fresh(&a.qmin[a.bq[j]]), idist, needs);
+    CpVals vals;
+    __builtin_memcpy(&vals, a.vals + 7LL * j, sizeof(vals));
+    cp_item(a, a.codes[j], vals, a.bdc[j], lo, up, load_fresh(&a.qmin[a.bq[j]]), idist, needs);
     a.idist[j] = idist;
     a.ineeds[j] = needs;
   }
@@ -282,8 +319,11 @@ __device__ __forceinline__ void cp_update_body(CpState* S, const CpArgs& a, int 
 
 // One workgroup applies the update of the round k_cp_gather popped.
 static __global__ void __launch_bounds__(1024) k_cp_update(CpState* S, CpArgs a) {
+  if (a.B <= 2 * 1024 || S->n <= 2 * 1024) {
+    cp_update_regs<1024>(S, a);
+    return;
+  }
   const int n = S->n;
-  if (n == 0) return;
   cp_update_body<1024>(S, a, n, S->pop);
 }
 
@@ -304,12 +344,16 @@ __device__ __forceinline__ float cp_sample(const float* lo, const float* up, int
 // k_points_dev), so box and point tiles fill the chip together.  Every
 // (node, feature) and (point, feature) sums in the order of those kernels:
 // codes and values are theirs bit for bit.
-template <int KIND, int V, int NW, int WMAX, int AS = ACTS_ALL>
+// PW: waves of a point tile (1: several tiles of one wave each share a
+// workgroup, without barriers; a tile of all NW waves otherwise).
+template <int KIND, int V, int NW, int PW, int WMAX, int AS = ACTS_ALL>
 __global__ void __launch_bounds__(NW * 64, (LdsOcc<Planes<KIND, V, 0>::R, 16, NW, WMAX>::value))
 k_cp_forward(const DevModel* __restrict__ Mp, CpState* S, CpArgs a, int g_box) {
   using PB = Planes<KIND, V, 0>;
   using PP = Planes<2, 0, 1>;
   constexpr int NB = 16, NT = NW * 64;
+  static_assert(PW == NW || PW == 1, "point tiles of one wave or of the workgroup");
+  static_assert(NW / PW <= PB::R, "point tiles fit beside each other in X");
   __shared__ float X[PB::R * NB * WMAX];
   const int top = S->top;
   const int pop = max(top - a.B, 0);
@@ -326,9 +370,8 @@ k_cp_forward(const DevModel* __restrict__ Mp, CpState* S, CpArgs a, int g_box) {
     for (int b = threadIdx.x; b < NB; b += NT) {
       const long long i = i0 + b;
       if (i < n) {
-        const long long s = pop + i;
-        a.bq[i] = a.wq[s];
-        for (int k = 0; k < 3; ++k) { a.blo[3 * i + k] = a.wlo[3 * s + k]; a.bup[3 * i + k] = a.wup[3 * s + k]; }
+        float lo[3], up[3];
+        cp_copy_item(a, pop + i, i, lo, up);
       }
     }
     ClassifyArgs ca{};
@@ -344,10 +387,17 @@ k_cp_forward(const DevModel* __restrict__ Mp, CpState* S, CpArgs a, int g_box) {
       a.codes[i] = sign_code(lo, hi, 0.f);
     });
   } else {
-    const long long p0 = (long long)(blockIdx.x - g_box) * NB;
+    // point tiles of PW waves, NW / PW of them to the workgroup
+    const int sub = PW == NW ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (PW * 64));
+    constexpr int PT = PW * 64;
+    float* Xp = X + sub * (NB * WMAX);
+    const long long p0 = ((long long)(blockIdx.x - g_box) * (NW / PW) + sub) * NB;
     const long long np = 7LL * n;
     if (p0 >= np) return;
-    for (int e = threadIdx.x; e < NB * 16; e += NT) {
+#pragma unroll
+    for (int e0 = 0; e0 < NB * 16; e0 += PT) {
+      const int e = e0 + (int)threadIdx.x % PT;
+      if (NB * 16 % PT != 0 && e >= NB * 16) break;
       const int b = e >> 4, k = e & 15;
       const long long q = p0 + b;
       float val = 0.f;
@@ -355,9 +405,9 @@ k_cp_forward(const DevModel* __restrict__ Mp, CpState* S, CpArgs a, int g_box) {
         const long long s = pop + q / 7;
         val = cp_sample(a.wlo + 3 * s, a.wup + 3 * s, (int)(q % 7), k);
       }
-      X[xoff<NB, WMAX>(0, b, k)] = val;
+      Xp[xoff<NB, WMAX>(0, b, k)] = val;
     }
-    mlp_forward<PP, 2, 0, NB, NW, WMAX, AS>(*Mp, X, [&](const float* v, int b) {
+    mlp_forward<PP, 2, 0, NB, PW, WMAX, AS>(*Mp, Xp, [&](const float* v, int b) {
       const long long q = p0 + b;
       if (q < np) a.vals[q] = v[0];
     });

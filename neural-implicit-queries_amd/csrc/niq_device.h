@@ -564,6 +564,10 @@ __device__ __forceinline__ void mlp_forward(const DevModel& M, float* __restrict
     // input fragments (LDS, unchanged until the barrier below) are loaded
     // while the current one's MFMAs run.  `FULL`: every feature tile of this
     // wave exists, so the loop carries no per-tile test.
+    // The weights come through a global-address-space pointer: as flat loads
+    // they would also count against the LDS wait, which then waits for the next
+    // k-block's weights (an L2 latency a layer in the narrow templates).
+    const auto Wp = as_global(Ly.Wp);
     auto contract = [&](auto full_tag) __attribute__((always_inline)) {
       constexpr bool FULL = decltype(full_tag)::value;
       floatx4 a_nx[FTMAX];
@@ -583,7 +587,7 @@ __device__ __forceinline__ void mlp_forward(const DevModel& M, float* __restrict
 #pragma unroll
           for (int f = 0; f < FTMAX; ++f) {
             const int ft = wave + f * NW;
-            if (FULL || ft < nft) a_nx[f] = Ly.Wp[(size_t)(ft * nkb + kb + 1) * 64 + lane];
+            if (FULL || ft < nft) a_nx[f] = Wp[(size_t)(ft * nkb + kb + 1) * 64 + lane];
           }
         }
 #pragma unroll
@@ -617,7 +621,7 @@ __device__ __forceinline__ void mlp_forward(const DevModel& M, float* __restrict
       if (wave < kKSplit) {
         const int kb0 = wave * nkb / kKSplit, kb1 = (wave + 1) * nkb / kKSplit;
         floatx4 a_nx = {0.f, 0.f, 0.f, 0.f};
-        if (kb0 < kb1) a_nx = Ly.Wp[(size_t)kb0 * 64 + lane];
+        if (kb0 < kb1) a_nx = Wp[(size_t)kb0 * 64 + lane];
         for (int kb = kb0; kb < kb1; ++kb) {
           const floatx4 a = a_nx;
           floatx4 bx[R][BT];
@@ -626,7 +630,7 @@ __device__ __forceinline__ void mlp_forward(const DevModel& M, float* __restrict
 #pragma unroll
             for (int t = 0; t < BT; ++t)
               bx[p][t] = *reinterpret_cast<const floatx4*>(&X[xoff<NB, WMAX>(p, t * 16 + ln, kb * 16 + lg * 4)]);
-          if (kb + 1 < kb1) a_nx = Ly.Wp[(size_t)(kb + 1) * 64 + lane];
+          if (kb + 1 < kb1) a_nx = Wp[(size_t)(kb + 1) * 64 + lane];
 #pragma unroll
           for (int p = 0; p < R; ++p)
 #pragma unroll
