@@ -631,15 +631,26 @@ __device__ __forceinline__ void tree_top_body(const TreeTopArgs& a, TreeCounters
   constexpr int NT = 1024, PER = kTopMaxN / NT, NWV = NT / 64;
   __shared__ unsigned char s_code[2 * kTopMaxN];
   __shared__ unsigned short s_heap[2][kTopMaxN];
-  __shared__ int s_pre[kTopMaxN + 1];               // unknown nodes before each node
-  __shared__ unsigned long long s_wave[NWV];        // per wave: unknown, positive, negative (21 bits each)
+  __shared__ int s_pre[kTopMaxN + 1];       // unknown nodes before each node
+  __shared__ unsigned s_wave[NWV];          // per wave: unknown (low half), positive (high half)
+  // finished nodes in list order: interior from the front, exterior from the
+  // back (at most one per leaf of the top, kTopMaxN in all)
+  __shared__ unsigned short s_fin[kTopMaxN];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int n_top = (1 << a.top_levels) - 1;
-  for (int h = tid; h < n_top; h += NT) s_code[h + 1] = (unsigned char)a.codes[h];
+  {
+    constexpr int NL = 2 * kTopMaxN / NT;   // every load issued before any is used
+    int c[NL];
+#pragma unroll
+    for (int j = 0; j < NL; ++j) c[j] = a.codes[min(tid + j * NT, n_top - 1)];
+#pragma unroll
+    for (int j = 0; j < NL; ++j)
+      if (tid + j * NT < n_top) s_code[tid + j * NT + 1] = (unsigned char)c[j];
+  }
   for (int i = tid; i < 64; i += NT) { C->level_n[i] = 0; C->level_int[i] = 0; C->level_ext[i] = 0; }
   if (tid == 0) s_heap[0][0] = 1;
   __syncthreads();
-  int n = 1, n_int = 0, n_ext = 0, overflow = 0, level = 0, done = 0;
+  int n = 1, n_int = 0, n_ext = 0, overflow = 0, level = 0, done = 0, U = 0, n_list = 0;
   long long classified = 0;
   for (; level < a.top_levels && !done; ++level) {
     const bool split = !(level + 1 == a.n_levels || (a.thresh > 0 && n >= a.thresh));
@@ -647,33 +658,33 @@ __device__ __forceinline__ void tree_top_body(const TreeTopArgs& a, TreeCounters
     unsigned short* next = s_heap[(level + 1) & 1];
     // exclusive scan of the code counts, PER consecutive nodes a thread
     int h[PER], code[PER];
-    unsigned long long mine = 0;
+    unsigned mine = 0;
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
       const int i = tid * PER + k;
       h[k] = i < n ? heap[i] : 0;
       code[k] = i < n ? s_code[h[k]] : -1;
-      if (i < n) mine += 1ull << (21 * (code[k] == CODE_UNKNOWN ? 0 : (code[k] == CODE_POSITIVE ? 1 : 2)));
+      mine += code[k] == CODE_UNKNOWN ? 1u : (code[k] == CODE_POSITIVE ? 0x10000u : 0u);
     }
-    unsigned long long incl = mine;
+    unsigned incl = mine;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
-      const unsigned long long v = __shfl_up(incl, d);
+      const unsigned v = __shfl_up(incl, d);
       if (lane >= d) incl += v;
     }
     if (lane == 63) s_wave[wave] = incl;
     __syncthreads();
-    unsigned long long before = 0, total = 0;
+    unsigned before = 0, total = 0;
 #pragma unroll
     for (int w = 0; w < NWV; ++w) {
-      const unsigned long long v = s_wave[w];
+      const unsigned v = s_wave[w];
       if (w < wave) before += v;
       total += v;
     }
-    const unsigned long long ex = before + incl - mine;
-    constexpr unsigned long long M21 = (1ull << 21) - 1;
-    const int U = (int)(total & M21), P = (int)((total >> 21) & M21), N = (int)(total >> 42);
-    int ru = (int)(ex & M21), rp = (int)((ex >> 21) & M21), rn = (int)(ex >> 42);
+    const unsigned ex = before + incl - mine;
+    U = (int)(total & 0xffffu);
+    const int P = (int)(total >> 16), N = n - U - P;
+    int ru = (int)(ex & 0xffffu), rp = (int)(ex >> 16);
     const int ru0 = ru;
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
@@ -683,44 +694,30 @@ __device__ __forceinline__ void tree_top_body(const TreeTopArgs& a, TreeCounters
     }
     if (tid == 0) s_pre[n] = U;
     __syncthreads();
+    const bool keep = !split || level + 1 == a.top_levels;   // the unknown nodes are written out below
     ru = ru0;
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
       const int i = tid * PER + k;
       if (i >= n) continue;
-      const int c = code[k], hb = 3 * (h[k] - 1);
+      const int c = code[k];
       if (c == CODE_UNKNOWN) {
-        const int b0 = i & ~(a.B - 1);   // the batch's first node (B is a power of 2)
-        const int Ub = s_pre[b0], nUb = s_pre[min((long long)b0 + a.B, (long long)n)] - Ub;
-        const long long pa = ru + Ub, pb = pa + nUb;
-        if (!split) {
-          if (ru < a.cap_unk) {
-            store3(a.unk_lower, ru, a.box_lo[hb], a.box_lo[hb + 1], a.box_lo[hb + 2]);
-            store3(a.unk_upper, ru, a.box_up[hb], a.box_up[hb + 1], a.box_up[hb + 2]);
-          }
-        } else if (level + 1 < a.top_levels) {
-          if (pa < min(a.cap, (long long)kTopMaxN)) next[pa] = (unsigned short)(2 * h[k]);
-          if (pb < min(a.cap, (long long)kTopMaxN)) next[pb] = (unsigned short)(2 * h[k] + 1);
-        } else {
-          store_children(a.next_lower, a.next_upper, a.cap, pa, pb, a.box_lo[hb], a.box_lo[hb + 1],
-                         a.box_lo[hb + 2], a.box_up[hb], a.box_up[hb + 1], a.box_up[hb + 2]);
+        if (!keep) {
+          const int b0 = i & ~(a.B - 1);   // the batch's first node (B is a power of 2)
+          const int Ub = s_pre[b0], nUb = s_pre[min((long long)b0 + a.B, (long long)n)] - Ub;
+          const long long pa = ru + Ub, pb = pa + nUb, room = min(a.cap, (long long)kTopMaxN);
+          if (pa < room) next[pa] = (unsigned short)(2 * h[k]);
+          if (pb < room) next[pb] = (unsigned short)(2 * h[k] + 1);
         }
         ++ru;
       } else if (c == CODE_POSITIVE) {
-        const long long p = n_ext + rp++;
-        if (a.ext_lower && p < a.cap_ext) {
-          store3(a.ext_lower, p, a.box_lo[hb], a.box_lo[hb + 1], a.box_lo[hb + 2]);
-          store3(a.ext_upper, p, a.box_up[hb], a.box_up[hb + 1], a.box_up[hb + 2]);
-        }
+        s_fin[kTopMaxN - 1 - (n_ext + rp++)] = (unsigned short)h[k];
       } else {
-        const long long p = n_int + rn++;
-        if (a.int_lower && p < a.cap_int) {
-          store3(a.int_lower, p, a.box_lo[hb], a.box_lo[hb + 1], a.box_lo[hb + 2]);
-          store3(a.int_upper, p, a.box_up[hb], a.box_up[hb + 1], a.box_up[hb + 2]);
-        }
+        s_fin[n_int + (i - ru - rp)] = (unsigned short)h[k];
       }
     }
     if (tid == 0) { C->level_n[level] = n; C->level_int[level] = n_int; C->level_ext[level] = n_ext; }
+    n_list = n;
     classified += n;
     n_ext += P;
     n_int += N;
@@ -729,6 +726,37 @@ __device__ __forceinline__ void tree_top_body(const TreeTopArgs& a, TreeCounters
     n = (int)min(nn, cap_next);
     done = !split;
     __syncthreads();   // next list complete; s_wave and s_pre free
+  }
+  // The lists, from the boxes in global memory: the last level's unknown nodes
+  // (s_pre and its heap list still hold it), then the finished nodes.
+  {
+    const unsigned short* heap = s_heap[(level - 1) & 1];
+    for (int i = tid; i < n_list; i += NT) {
+      const int hb = 3 * (heap[i] - 1);
+      if (s_code[heap[i]] != CODE_UNKNOWN) continue;
+      const int ru = s_pre[i];
+      if (done) {
+        if (ru < a.cap_unk) {
+          store3(a.unk_lower, ru, a.box_lo[hb], a.box_lo[hb + 1], a.box_lo[hb + 2]);
+          store3(a.unk_upper, ru, a.box_up[hb], a.box_up[hb + 1], a.box_up[hb + 2]);
+        }
+      } else {
+        const int b0 = i & ~(a.B - 1);
+        const int Ub = s_pre[b0], nUb = s_pre[min((long long)b0 + a.B, (long long)n_list)] - Ub;
+        store_children(a.next_lower, a.next_upper, a.cap, ru + Ub, ru + Ub + nUb, a.box_lo[hb], a.box_lo[hb + 1],
+                       a.box_lo[hb + 2], a.box_up[hb], a.box_up[hb + 1], a.box_up[hb + 2]);
+      }
+    }
+    for (int i = tid; i < n_int && a.int_lower && i < a.cap_int; i += NT) {
+      const int hb = 3 * (s_fin[i] - 1);
+      store3(a.int_lower, i, a.box_lo[hb], a.box_lo[hb + 1], a.box_lo[hb + 2]);
+      store3(a.int_upper, i, a.box_up[hb], a.box_up[hb + 1], a.box_up[hb + 2]);
+    }
+    for (int i = tid; i < n_ext && a.ext_lower && i < a.cap_ext; i += NT) {
+      const int hb = 3 * (s_fin[kTopMaxN - 1 - i] - 1);
+      store3(a.ext_lower, i, a.box_lo[hb], a.box_lo[hb + 1], a.box_lo[hb + 2]);
+      store3(a.ext_upper, i, a.box_up[hb], a.box_up[hb + 1], a.box_up[hb + 2]);
+    }
   }
   if (tid == 0) {
     C->n[level & 1] = n;
