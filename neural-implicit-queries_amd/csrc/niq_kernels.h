@@ -793,6 +793,7 @@ struct RayGroup {
   unsigned long long* next_ray;  // work counter, zero on entry
   int* iter_hist;          // (n_max_step + 2,) rays by iterations lived, nullable
   float lipschitz;         // weak-SDF form (KIND 2): Lipschitz bound of f
+  long long stride;        // claim k is ray k * stride mod n (coprime with n; pooled caster)
 };
 
 struct RayArgs {
