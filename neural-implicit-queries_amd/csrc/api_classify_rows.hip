@@ -26,10 +26,23 @@ niq_status launch_rows_w(const niq_model* m, const niq_eval_cfg* cfg, const Clas
   if (max_n == 0) return NIQ_OK;
   long long g = std::min<long long>(max_n, persistent_blocks(k, NW * 64));
   g = std::max<long long>(1, std::min<long long>(g, (long long)((16ull << 30) / per_wg)));
+  // Boxes that their corners decide (k_rows_signs): in a tree's levels, which give
+  // room for a list of the others.  Not with Sin layers, whose affine rule (the
+  // reference's) may carry a negative error term into err and then is no bound.
+  const bool signs = a.list && a.lower && a.d == 3 && !a.bounds && m->bounded &&
+                     (m->relu_only || m->tanh_only || m->elu_only) && max_n >= kRowsSignsMin;
   void* scratch = nullptr;
   HIPCHK(hipMallocAsync(&scratch, per_wg * g, s));
   RowsArgs ra{};
   ra.c = a;
+  if (signs) {
+    constexpr int NW_S = W <= 64 ? 4 : 8;
+    auto ks = k_rows_signs<16, NW_S, W>;
+    hipLaunchKernelGGL(ks, dim3(tile_grid((max_n + 15) / 16, persistent_blocks(ks, NW_S * 64))), dim3(NW_S * 64), 0, s,
+                       m->dev, a);
+  } else {
+    ra.c.list = nullptr;
+  }
   ra.scratch = static_cast<float*>(scratch);
   ra.max_rows = max_rows;
   ra.n_keep = n_keep;

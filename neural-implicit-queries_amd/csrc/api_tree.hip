@@ -413,10 +413,12 @@ niq_status tree_enqueue(const niq_model* m, const niq_eval_cfg* cfg, const niq_t
       ++split_levels;
   }
   auto classify = [&](ClassifyArgs a, long long max_n, int lv) -> niq_status {
-    if (lv >= split_levels) return classify_dispatch(m, cfg, 3, a, max_n, s);
+    // room for the boxes that a first look leaves (the split contraction, or the
+    // growing-row modes' corners); the FP64 re-test's, which neither path has
     a.list = reinterpret_cast<int*>(base + L.off_recheck);
     a.list_n = &C->near_cnt;
     a.list_cap = (int)std::min<long long>(max_n, INT_MAX);
+    if (lv >= split_levels) return classify_dispatch(m, cfg, 3, a, max_n, s);
     return classify_split(m, a, max_n, s);
   };
   if (T) {

@@ -37,6 +37,70 @@ struct RowsArgs {
   int n_append;            // affine_append
 };
 
+// Fewest boxes of a launch whose corners are looked at first: below a box per
+// compute unit the boxes run side by side, and leaving some out saves no time.
+constexpr int kRowsSignsMin = 256;
+
+// The boxes whose code the signs of f at their corners decide.  A bound contains
+// f's values in the box, so with one value below the offset and one above its
+// negative the code is UNKNOWN, whatever the mode; only the other boxes, listed for
+// k_classify_rows, need the bound.  The values must clear the thresholds by 2 % of
+// the largest and the box be no smaller than 2^-11 of its distance from the
+// origin, where float32 rounding of values and bound is far below that.  A box
+// costs 8 points here (4, every other corner, at width 512, for LDS), about 1/50 of
+// its growing error terms, and in the trees of random nets two thirds of all boxes
+// are decided: the depth-18 affine_all tree of a 128x8 TanH net 54 -> 24 ms,
+// the depth-15 one of a 32x4 TanH net 1.25 -> 0.95 ms.
+template <int NB, int NW, int WMAX>
+__global__ void __launch_bounds__(NW * 64)
+k_rows_signs(const DevModel* __restrict__ Mp, ClassifyArgs a) {
+  constexpr int P = WMAX <= 256 ? 8 : 4;
+  constexpr int NT = NW * 64;
+  using PL = Planes<2, 0, P>;
+  __shared__ float X[P * NB * WMAX];
+  const long long n = a.n_dev ? (long long)(*a.n_dev) : a.n;
+  const long long ntiles = (n + NB - 1) / NB;
+  for (long long tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    const long long i0 = tile * NB;
+    for (int e = threadIdx.x; e < NB * 16; e += NT) {
+      const int b = e >> 4, k = e & 15;
+      const long long i = i0 + b;
+      const bool in = i < n && k < 3;
+      const float lo = in ? a.lower[i * 3 + k] : 0.f, up = in ? a.upper[i * 3 + k] : 0.f;
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        const int corner = P == 8 ? p : (p == 0 ? 0 : 7 ^ (1 << (p - 1)));
+        X[xoff<NB, WMAX>(p, b, k)] = (corner >> k) & 1 ? up : lo;
+      }
+    }
+    mlp_forward<PL, 2, 0, NB, NW, WMAX>(*Mp, X, [&](const float* v, int b) {
+      const long long i = i0 + b;
+      if (i >= n) return;
+      float mn = v[0], mx = v[0], big = 0.f, half = 0.f, far = 0.f;
+      bool finite = true;
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        mn = fminf(mn, v[p]); mx = fmaxf(mx, v[p]);
+        big = fmaxf(big, fabsf(v[p]));
+        finite = finite && fabsf(v[p]) <= 3.4028234663852886e38f;
+      }
+      for (int k = 0; k < 3; ++k) {
+        const float lo = a.lower[i * 3 + k], up = a.upper[i * 3 + k];
+        finite = finite && lo <= up;
+        half = fmaxf(half, 0.5f * (up - lo));
+        far = fmaxf(far, fmaxf(fabsf(lo), fabsf(up)));
+      }
+      const float m = 0.02f * big;
+      const bool unknown = finite && far <= 1e6f && half >= far * 0x1p-11f && mn < a.offset - m && mx > m - a.offset;
+      if (unknown) a.codes[i] = CODE_UNKNOWN;
+      else {
+        const int at = atomicAdd(a.list_n, 1);
+        if (at < a.list_cap) a.list[at] = (int)i;
+      }
+    });
+  }
+}
+
 // Block-wide argmax over n values (largest first, lowest index on ties);
 // every thread gets the result.  `sv`/`si` are 2 * NT scratch entries.
 template <int NT>
@@ -102,11 +166,13 @@ k_classify_rows(const DevModel* __restrict__ Mp, RowsArgs ra) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // scalar tile tests
   const int ln = lane & 15, lg = lane >> 4;
-  const long long n = a.n_dev ? (long long)(*a.n_dev) : a.n;
+  // the boxes of a.list (k_rows_signs), or all
+  const long long n = a.list ? (long long)min(*a.list_n, a.list_cap) : (a.n_dev ? (long long)(*a.n_dev) : a.n);
   float* buf[2] = {ra.scratch + (size_t)blockIdx.x * 2 * ra.max_rows * WMAX,
                    ra.scratch + (size_t)blockIdx.x * 2 * ra.max_rows * WMAX + (size_t)ra.max_rows * WMAX};
 
-  for (long long i = blockIdx.x; i < n; i += gridDim.x) {
+  for (long long j = blockIdx.x; j < n; j += gridDim.x) {
+    const long long i = a.list ? a.list[j] : j;
     // Layer-0 input (src/affine.py:109-117).  Axis boxes: the d rows
     // diag(half) enter as added rows (image half_k * A[k, :]); general boxes:
     // the v box vectors enter as stored rows.
