@@ -65,14 +65,15 @@ typedef struct niq_eval_cfg {
   int truncate_count;  /* affine_truncate: rows kept */
   int n_append;        /* affine_append: rows appended per activation */
   float recheck_tol;   /* > 0: FP64 re-test of cells within tol*scale of the threshold */
-  int variant;         /* kernel variant, 0 = default; plain FP32: 1 TileCfg,
-                          2 TileCfgAlt, 3 TileCfg with 256 registers, 4
+  int variant;         /* kernel variant, 0 = default; plain FP32: 1 BoxTile,
+                          2 TileCfgAlt, 3 BoxTile with 256 registers, 4
                           TileCfgWide (the most waves, the narrowest width
                           tile per wave) (niq_tile_shape); growing-row modes: 2 half the
                           error-term rows per chunk, 3 a 2-waves-per-SIMD
                           register budget; precision mode: 1 streams the
                           packed bf16 weight copies, 2 splits FP32 weights in
-                          registers (the default), 3 layer by layer; closest
+                          registers where a layer does not fill the
+                          template (the default), 3 layer by layer; closest
                           point runs its round as one forward launch only at
                           variant 0.  Every variant gives the same results. */
   float sdf_lipschitz; /* NIQ_MODE_SDF: Lipschitz bound of f (sdf_lipschitz kwarg) */

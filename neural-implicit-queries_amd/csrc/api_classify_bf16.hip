@@ -100,7 +100,8 @@ niq_status launch_lw(const niq_model* m, const ClassifyArgs& a, long long max_n,
 }
 
 // Weight source: cfg->variant = 1 streams the four packed bf16 copies, 2 (and
-// the default) the FP32 weights split in registers; 3 runs layer by layer
+// the default) the FP32 weights split in registers, but in layers that fill the
+// template the packed terms side by side (contract_wide, same splits); 3 runs layer by layer
 // (hidden widths multiples of 128, interval or three box vectors; otherwise
 // the fused kernel of variant 2).
 template <int V>

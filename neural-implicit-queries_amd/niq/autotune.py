@@ -3,14 +3,15 @@
 The search space is the kernels' tile shapes, each a compiled variant:
 
 * plain FP32 classify (interval and affine_fixed over 3 box vectors),
-  ``EvalCfg.variant``: 1 the default tile (``TileCfg``: 16-32 boxes per
-  workgroup, 4-8 waves, the register budget LDS occupancy allows), 2 twice
+  ``EvalCfg.variant``: 1 the default tile (``BoxTile``: 16 boxes, 64 at
+  width 32, 4-8 waves, the register budget LDS occupancy allows), 2 twice
   the boxes per workgroup where LDS allows (fewer waves at width 512), 3 the
   default tile with a 256-register budget (no spills, fewer resident
   workgroups), 4 16 boxes with the most waves (the narrowest width tile: the
   waves of a tile split the layer's 16-feature tiles among them);
 * precision mode (BF16) classify: 1 streams the packed bf16 weight copies,
-  2 loads the FP32 weights once and splits them in registers, 3 runs layer
+  2 loads the FP32 weights once and splits them in registers (layers that
+  fill the template read the packed terms side by side), 3 runs layer
   by layer (one batched launch per hidden layer, activations through HBM);
 * the growing-row classify (affine_all, affine_truncate, affine_append; one
   box per workgroup, its error terms streamed in chunks): 1 the default, 2
