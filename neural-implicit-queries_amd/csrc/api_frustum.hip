@@ -10,6 +10,19 @@ long long next_bucket_size(long long s) {
   return -1;
 }
 
+// est: the frusta to size the launch for (it strides over the live count).
+template <int V, int AS>
+niq_status launch_frust_forward(const niq_model* m, const ClassifyArgs& a, const float* pts, float* vals, long long est,
+                                hipStream_t s) {
+  auto k = k_frust_forward<V, AS>;
+  const long long cap = persistent_blocks(k, 128) * kTileGridMult;
+  const int g_box = (int)std::max<long long>(1, std::min((est + 15) / 16, cap));
+  const int g_pts = (int)std::max<long long>(1, std::min((2 * est + 31) / 32, cap));
+  hipLaunchKernelGGL(k, dim3(g_box + g_pts), dim3(128), 0, s, m->dev, a, pts, vals, g_box);
+  HIPCHK(hipGetLastError());
+  return NIQ_OK;
+}
+
 }  // namespace
 
 extern "C" niq_status niq_cast_rays_frustum(const niq_model* const* models, int n_models, const niq_eval_cfg* cfg,
@@ -109,6 +122,10 @@ extern "C" niq_status niq_cast_rays_frustum(const niq_model* const* models, int 
   // count).  The layer-by-layer precision mode sizes its scratch by max_n and
   // gets a true bound.
   const bool strict = cfg && cfg->precision == NIQ_PREC_BF16 && cfg->variant == 3;
+  // 32-wide nets evaluate boxes and points in one launch, unless the caller chose
+  // another classify tile
+  const bool fused = (!cfg || (cfg->precision == NIQ_PREC_FP32 && cfg->variant == 0)) &&
+                     (mode == NIQ_MODE_INTERVAL || mode == NIQ_MODE_AFFINE_FIXED);
   FrustCount h[kGroup + 2];
   int hfin = 0;
   bool done = st != NIQ_OK, growing = true;
@@ -131,8 +148,20 @@ extern "C" niq_status niq_cast_rays_frustum(const niq_model* const* models, int 
           ClassifyArgs a{};
           a.center = W.center; a.vecs = W.vecs; a.vin = 3; a.d = 3; a.n_dev = n_live; a.offset = 0.f;
           a.codes = W.codes + (size_t)f * cap;
+          float* fvals = W.vals + (size_t)f * 2 * cap;
+          if (fused && models[f]->wt == 32) {
+            const niq_model* m = models[f];
+            if (mode == NIQ_MODE_INTERVAL)
+              st = m->relu_only ? launch_frust_forward<0, ACTS_RELU>(m, a, W.pts, fvals, est, s)
+                                : launch_frust_forward<0, ACTS_ALL>(m, a, W.pts, fvals, est, s);
+            else
+              st = m->relu_only ? launch_frust_forward<3, ACTS_RELU>(m, a, W.pts, fvals, est, s)
+                                : launch_frust_forward<3, ACTS_ALL>(m, a, W.pts, fvals, est, s);
+            if (st) break;
+            continue;
+          }
           if ((st = classify_dispatch(models[f], cfg, mode == NIQ_MODE_INTERVAL ? 0 : 3, a, est, s))) break;
-          st = points_dev(models[f], W.pts, n_live, 2, 2 * est, W.vals + (size_t)f * 2 * cap, s);
+          st = points_dev(models[f], W.pts, n_live, 2, 2 * est, fvals, s);
         }
         if (st) break;
         const int first = sub == 0 ? 1 : 0;
