@@ -31,6 +31,11 @@ niq_status launch_rows_w(const niq_model* m, const niq_eval_cfg* cfg, const Clas
   // reference's) may carry a negative error term into err and then is no bound.
   const bool signs = a.list && a.lower && a.d == 3 && !a.bounds && m->bounded &&
                      (m->relu_only || m->tanh_only || m->elu_only) && max_n >= kRowsSignsMin;
+  // A tree's top levels in passes, where a box costs far more than a pass's latency:
+  // depth-18 affine_all tree of the 128x8 TanH net 24.0 -> 17.9 ms (3 passes 21.0,
+  // 8 passes 19.6), but the affine_all tree of a 32x4 net 0.99 -> 1.04, the
+  // affine_truncate tree of the 32x8 fox net 8.1 -> 8.9.
+  const bool heap = signs && a.heap && MODE == ROWS_ALL && W >= 128;
   void* scratch = nullptr;
   HIPCHK(hipMallocAsync(&scratch, per_wg * g, s));
   RowsArgs ra{};
@@ -39,7 +44,7 @@ niq_status launch_rows_w(const niq_model* m, const niq_eval_cfg* cfg, const Clas
     constexpr int NW_S = W <= 64 ? 4 : 8;
     auto ks = k_rows_signs<16, NW_S, W>;
     hipLaunchKernelGGL(ks, dim3(tile_grid((max_n + 15) / 16, persistent_blocks(ks, NW_S * 64))), dim3(NW_S * 64), 0, s,
-                       m->dev, a);
+                       m->dev, a, heap);
   } else {
     ra.c.list = nullptr;
   }
@@ -47,7 +52,13 @@ niq_status launch_rows_w(const niq_model* m, const niq_eval_cfg* cfg, const Clas
   ra.max_rows = max_rows;
   ra.n_keep = n_keep;
   ra.n_append = n_append;
-  hipLaunchKernelGGL(k, dim3((unsigned)g), dim3(NW * 64), 0, s, m->dev, ra);
+  for (int pass = 0; pass < (heap ? kRowsHeapPasses : 1); ++pass) {
+    if (heap) {
+      hipLaunchKernelGGL(k_rows_heap_list, dim3(1), dim3(1024), 0, s, a.codes, (int)max_n,
+                         pass == kRowsHeapPasses - 1, a.list, a.list_n);
+    }
+    hipLaunchKernelGGL(k, dim3((unsigned)g), dim3(NW * 64), 0, s, m->dev, ra);
+  }
   const hipError_t e = hipGetLastError();
   HIPCHK(hipFreeAsync(scratch, s));
   if (e != hipSuccess) return fail(NIQ_ERR_HIP, std::string("k_classify_rows: ") + hipGetErrorString(e));

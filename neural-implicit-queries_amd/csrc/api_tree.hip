@@ -431,6 +431,7 @@ niq_status tree_enqueue(const niq_model* m, const niq_eval_cfg* cfg, const niq_t
     ClassifyArgs a{};
     a.lower = top_lo; a.upper = top_up; a.d = 3; a.n = n_top; a.offset = p->offset;
     a.codes = top_codes;
+    a.heap = true;
     if (L.lw_bytes) { a.lw_buf = base + L.off_lw; a.lw_bytes = L.lw_bytes; }
     if (niq_status st = classify(a, n_top, T - 1)) return st;
     TreeTopArgs ta{};

@@ -110,6 +110,7 @@ struct ClassifyArgs {
   int* list;               // boxes left by a first look (split contraction, corner signs),
   int* list_n;             //   their count (zero on entry) and capacity
   int list_cap;
+  bool heap;               // the boxes are a tree's top levels, by heap index
   float lipschitz;         // weak-SDF test: Lipschitz bound of f
   float* gx;               // forms too large for LDS: activation planes in global
                            //   memory, R * NB * WMAX floats per workgroup

@@ -41,6 +41,9 @@ struct RowsArgs {
 // compute unit the boxes run side by side, and leaving some out saves no time.
 constexpr int kRowsSignsMin = 256;
 
+// Code of a heap box that its corners leave open.
+constexpr int kRowsPending = -1;
+
 // The boxes whose code the signs of f at their corners decide.  A bound contains
 // f's values in the box, so with one value below the offset and one above its
 // negative the code is UNKNOWN, whatever the mode; only the other boxes, listed for
@@ -53,7 +56,7 @@ constexpr int kRowsSignsMin = 256;
 // the depth-15 one of a 32x4 TanH net 1.25 -> 0.95 ms.
 template <int NB, int NW, int WMAX>
 __global__ void __launch_bounds__(NW * 64)
-k_rows_signs(const DevModel* __restrict__ Mp, ClassifyArgs a) {
+k_rows_signs(const DevModel* __restrict__ Mp, ClassifyArgs a, bool heap) {
   constexpr int P = WMAX <= 256 ? 8 : 4;
   constexpr int NT = NW * 64;
   using PL = Planes<2, 0, P>;
@@ -93,11 +96,36 @@ k_rows_signs(const DevModel* __restrict__ Mp, ClassifyArgs a) {
       const float m = 0.02f * big;
       const bool unknown = finite && far <= 1e6f && half >= far * 0x1p-11f && mn < a.offset - m && mx > m - a.offset;
       if (unknown) a.codes[i] = CODE_UNKNOWN;
+      else if (heap) a.codes[i] = kRowsPending;
       else {
         const int at = atomicAdd(a.list_n, 1);
         if (at < a.list_cap) a.list[at] = (int)i;
       }
     });
+  }
+}
+
+// The pending boxes of a tree's top levels (heap index h - 1 of node h) that need
+// their bound, in kRowsHeapPasses passes, each with the codes of those before.  Most
+// nodes of the heap are never reached: an ancestor is certified.  A pass lists the nodes
+// whose ancestors are all UNKNOWN, reached for certain; the last one those
+// without a certified ancestor (one still pending itself may cost a bound that
+// nobody reads).  The rest are not reached, and their codes not read.  One
+// workgroup.  128x8 TanH net, 8191 nodes: 9.8 -> 3.8 ms.
+constexpr int kRowsHeapPasses = 5;
+static __global__ void __launch_bounds__(1024) k_rows_heap_list(const int* codes, int n, bool last, int* list,
+                                                               int* list_n) {
+  if (threadIdx.x == 0) *list_n = 0;
+  __syncthreads();
+  for (int i = threadIdx.x; i < n; i += 1024) {
+    if (codes[i] != kRowsPending) continue;
+    bool open = false, certified = false;
+    for (int h = (i + 1) >> 1; h > 0; h >>= 1) {
+      const int c = codes[h - 1];
+      open = open || c == kRowsPending;
+      certified = certified || c > CODE_UNKNOWN;
+    }
+    if (!certified && (last || !open)) list[atomicAdd(list_n, 1)] = i;
   }
 }
 
