@@ -396,13 +396,13 @@ niq_status niq_shade_image(const niq_shade_opts* opts, const float* ray_dirs, co
  * priority.  Requests queue in arrival order; a worker takes the oldest one as
  * soon as its device memory fits under mem_cap_bytes beside the work in
  * flight.  Ray requests waiting in the queue with the same eval config and
- * template width are merged into the cast of the request taken (up to 64
+ * template width (widths up to 64 count as one) are merged into the cast of the request taken (up to 64
  * requests and max_merge_rays rays): each request is a group of rays with its
  * own models, options, inputs and outputs inside one persistent kernel, and
  * every ray is independent, so merged results (N_evals included) equal lone
  * ones bit for bit.  Tree builds in the fused-kernel FP32 modes with a
  * split_depth that wait in the queue with the same eval config, build params
- * (root boxes aside) and template width are merged too (up to 64): one build
+ * (root boxes aside) and template width (as above) are merged too (up to 64): one build
  * runs every level of all of them in shared launches, each tree's level as
  * its lone build runs it, so the outputs are a lone build's bit for bit.  A
  * tree build taken alone replays a hipGraph captured once per (model,
