@@ -28,9 +28,10 @@ niq_status launch_rows_w(const niq_model* m, const niq_eval_cfg* cfg, const Clas
   g = std::max<long long>(1, std::min<long long>(g, (long long)((16ull << 30) / per_wg)));
   // Boxes that their corners decide (k_rows_signs): in a tree's levels, which give
   // room for a list of the others.  Not with Sin layers, whose affine rule (the
-  // reference's) may carry a negative error term into err and then is no bound.
+  // reference's) may carry a negative error term into err and then is no bound (and
+  // whose rounding is not known).
   const bool signs = a.list && a.lower && a.d == 3 && !a.bounds && m->bounded &&
-                     (m->relu_only || m->tanh_only || m->elu_only) && max_n >= kRowsSignsMin;
+                     std::isfinite(m->round_rel) && max_n >= kRowsSignsMin;
   // A tree's top levels in passes, where a box costs far more than a pass's latency:
   // depth-18 affine_all tree of the 128x8 TanH net 24.0 -> 17.9 ms (3 passes 21.0,
   // 8 passes 19.6), but the affine_all tree of a 32x4 net 0.99 -> 1.04, the
@@ -41,10 +42,11 @@ niq_status launch_rows_w(const niq_model* m, const niq_eval_cfg* cfg, const Clas
   RowsArgs ra{};
   ra.c = a;
   if (signs) {
+    ra.c.noise = kNoiseRoom * m->round_out;
     constexpr int NW_S = W <= 64 ? 4 : 8;
     auto ks = k_rows_signs<16, NW_S, W>;
     hipLaunchKernelGGL(ks, dim3(tile_grid((max_n + 15) / 16, persistent_blocks(ks, NW_S * 64))), dim3(NW_S * 64), 0, s,
-                       m->dev, a, heap);
+                       m->dev, ra.c, heap);
   } else {
     ra.c.list = nullptr;
   }

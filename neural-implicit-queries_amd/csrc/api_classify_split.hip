@@ -69,10 +69,14 @@ bool niqi::split_eligible(const niq_model* m, const niq_eval_cfg* cfg) {
   if (cfg && (cfg->mode != NIQ_MODE_AFFINE_FIXED || cfg->precision != NIQ_PREC_FP32 || cfg->recheck_tol > 0.f ||
               cfg->variant > 1))
     return false;
-  return split_shape(m) && m->relu_only && m->bias_small && m->in_dim == 3;
+  return split_shape(m) && m->relu_only && m->in_dim == 3 && std::isfinite(m->round_rel);
 }
 
-niq_status niqi::classify_split(const niq_model* m, const ClassifyArgs& a, long long max_n, hipStream_t s) {
+float niqi::split_min_half(const niq_model* m) { return m->round_rel / kSplitRound; }
+
+niq_status niqi::classify_split(const niq_model* m, ClassifyArgs a, long long max_n, hipStream_t s) {
+  a.min_half = split_min_half(m);
+  a.noise = kNoiseRoom * m->round_out;
   switch (m->wt) {
     case 256: return launch_split_w<256>(m, a, max_n, s);
     case 512: return launch_split_w<512>(m, a, max_n, s);

@@ -278,6 +278,7 @@ niq_status cast_run_groups(CastGroupReq* reqs, int ng, const niq_eval_cfg* cfg, 
     G.iter_hist = reinterpret_cast<int*>(base + L.hist[g]);
     G.lipschitz = cfg ? cfg->sdf_lipschitz : 1.f;
     G.stride = claim_stride(r.n, wt);
+    G.noise = kNoiseRoom * r.models[0]->round_out;
     hg[g] = G;
     m0 += r.n_models;
     n_rays += r.n;
@@ -305,7 +306,7 @@ niq_status cast_run_groups(CastGroupReq* reqs, int ng, const niq_eval_cfg* cfg, 
     // Lipschitz constant is the caller's word, nor with Sin layers, whose affine rule
     // (the reference's) may carry a negative error term and then is no bound.
     bool pool = !bf16 && mode != NIQ_MODE_SDF && acts != ACTS_ALL;
-    for (int g = 0; g < ng; ++g) pool = pool && reqs[g].n_models == 1 && reqs[g].models[0]->bounded;
+    for (int g = 0; g < ng; ++g) pool = pool && reqs[g].n_models == 1 && std::isfinite(reqs[g].models[0]->round_rel);
     if (pool) st = cast_pool(mode, wt, rv, acts, table, a, n_rays, &pool, s);
     if (pool) {}   // launched, or failed
     else if (bf16) st = mode == NIQ_MODE_AFFINE_FIXED ? launch_rays_bf16<1>(wt16, relu, table16, a, n_rays, s)

@@ -11,7 +11,7 @@ niq_status launch_pool_w(const DevModel* models, const RayArgs& a, long long n_r
   constexpr int R = Planes<KIND, V, 1>::R;
   constexpr int LDSOCC = LdsOcc<R, NB, NW, W>::value;
   constexpr int OCC = RayTile<W, VAR>::OCC ? std::min(RayTile<W, VAR>::OCC, LDSOCC) : LDSOCC;
-  static_assert(R * NB * W * 4 + sizeof(RayPool) + 4 * (2 * NB + 1) <= kLdsLimit, "LDS");
+  static_assert(R * NB * W * 4 + sizeof(RayPool) + 4 * (3 * NB + 1) <= kLdsLimit, "LDS");
   auto k = k_cast_rays_pool<KIND, V, NB, NW, W, OCC, AS>;
   // Few rays are spread over as many workgroups as there are, down to the NB/2
   // whose tests fit into the pass of their bounds.

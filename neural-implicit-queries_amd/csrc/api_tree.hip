@@ -399,7 +399,7 @@ niq_status tree_enqueue(const niq_model* m, const niq_eval_cfg* cfg, const niq_t
   const int n_levels = p->split_depth >= 0 ? p->split_depth + 1 : 64;
   int level = 0;
   // Levels whose boxes are large enough, beside the root's distance from the
-  // origin, take the split contraction where the net is eligible (smaller boxes
+  // origin and the net's rounding, take the split contraction where the net is eligible (smaller boxes
   // would all be listed for the plain one).
   int split_levels = 0;
   if (split_eligible(m, cfg)) {
@@ -409,7 +409,8 @@ niq_status tree_enqueue(const niq_model* m, const niq_eval_cfg* cfg, const niq_t
       far = std::max(far, std::max(std::fabs(p->lower[k]), std::fabs(p->upper[k])));
     }
     while (split_levels <= kSplitMaxLevel &&
-           0.5f * std::ldexp(ext, -(split_levels + 2) / 3) >= far * kSplitMinSize)
+           0.5f * std::ldexp(ext, -(split_levels + 2) / 3) >=
+               std::max(far * kSplitMinSize, std::max(far, 1.f) * split_min_half(m)))
       ++split_levels;
   }
   auto classify = [&](ClassifyArgs a, long long max_n, int lv) -> niq_status {

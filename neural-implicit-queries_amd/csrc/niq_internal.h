@@ -135,7 +135,8 @@ struct niq_model {
   bool tanh_only = false;      // every hidden activation is TanH
   bool elu_only = false;       // every hidden activation is ELU
   bool bounded = false;        // activations below 1e30 on inputs up to 1e6 (split contraction)
-  bool bias_small = false;     // first-layer biases are small beside the weights (split contraction)
+  float round_rel = INFINITY;  // float32 rounding of bounds beside a unit of box width, and of f, over the
+  float round_out = INFINITY;  //   unit cube (net_rounding; infinite where it is not known)
   DevModelBf16 host16;         // precision-mode copy (bf16 hi/lo/|W| weights)
   DevModelBf16* dev16 = nullptr;
   void* weights16 = nullptr;
@@ -147,6 +148,14 @@ struct niq_model {
 };
 
 namespace niqi {
+
+// Rounding that a first look (the split contraction, a box's corners, a ray's certified
+// segment) keeps clear of, in units of niq_model::round_out, at coordinates up to 1 (in
+// proportion beyond).  Emulated float32 sums of ReLU nets 32x3, 64x6, 256x1, 256x3,
+// 256x6, 256x4 and 512x3, with hidden biases of 10, 1e3 and 1e5 among them (round_out 8e-8
+// to 0.12): the error of f is at most 3.1 units, and f leaves a float32 bound of a box
+// or segment (half-widths 1e-3 and 1e-4) by at most 2.8.
+constexpr float kNoiseRoom = 8.f;
 
 inline niq_status check_model(const niq_model* m, int d) {
   if (!m) return fail(NIQ_ERR_INVALID, "null model");
@@ -189,7 +198,9 @@ niq_status classify_rows(const niq_model* m, const niq_eval_cfg* cfg, const Clas
 // the codes of classify_dispatch, faster on wide ReLU nets.  Needs
 // split_eligible(m, cfg).  Defined in api_classify_split.hip.
 bool split_eligible(const niq_model* m, const niq_eval_cfg* cfg);
-niq_status classify_split(const niq_model* m, const ClassifyArgs& a, long long max_n, hipStream_t s);
+niq_status classify_split(const niq_model* m, ClassifyArgs a, long long max_n, hipStream_t s);
+// The smallest half-width of a box, at coordinates up to 1, that it judges by.
+float split_min_half(const niq_model* m);
 // Point values by the FP32 matrix instructions (api_classify.hip).  Marching
 // cubes samples with these: its cells' signs, and so its triangles, are theirs.
 niq_status points_plain(const niq_model* m, const float* x, int d, long long n, float* out, hipStream_t s);

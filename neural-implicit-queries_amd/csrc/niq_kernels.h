@@ -111,6 +111,8 @@ struct ClassifyArgs {
   int* list_n;             //   their count (zero on entry) and capacity
   int list_cap;
   bool heap;               // the boxes are a tree's top levels, by heap index
+  float noise;             // rounding that a first look keeps clear of, at coordinates up to 1
+  float min_half;          // split contraction: smallest half-width judged, likewise
   float lipschitz;         // weak-SDF test: Lipschitz bound of f
   float* gx;               // forms too large for LDS: activation planes in global
                            //   memory, R * NB * WMAX floats per workgroup
@@ -794,6 +796,8 @@ struct RayGroup {
   unsigned long long* next_ray;  // work counter, zero on entry
   int* iter_hist;          // (n_max_step + 2,) rays by iterations lived, nullable
   float lipschitz;         // weak-SDF form (KIND 2): Lipschitz bound of f
+  float noise;             // pooled caster: least distance of a bound from zero that excludes a
+                           //   hit without a test, at coordinates up to 1
   long long stride;        // claim k is ray k * stride mod n (coprime with n; pooled caster)
 };
 

@@ -28,8 +28,8 @@ __device__ __forceinline__ int turn_rank(unsigned long long want, int rot, int l
 // Persistent certified-step ray caster (src/queries.py:39-175) for one function.
 // A ray's step bounds the segment ahead of it and compares the signs of f at its
 // start and hit_eps further on.  Where the bound certifies the segment with room
-// (its nearer end 2 % of its scale from zero, a segment long enough that the
-// points' FP32 rounding is far below that), both points have the certified sign,
+// (its nearer end 2 % of its scale and the rounding of this net from zero, see
+// kNoiseRoom, a segment long beside its distance), both points have the certified sign,
 // so the test cannot report a hit and is not evaluated; nor is it where both
 // points lie in an earlier segment certified so.  About 60 % of the steps of a
 // 256x6 random net, 85 % of a trained 32x8 net's.
@@ -56,7 +56,7 @@ k_cast_rays_pool(const DevModel* __restrict__ models, RayArgs a, int cap) {
   __shared__ float X[R * NB * WMAX];
   __shared__ RayPool S;
   __shared__ int s_code[NB];
-  __shared__ float s_val[NB];
+  __shared__ float s_val[NB], s_near[NB];
   __shared__ int s_model;
   const int lane = threadIdx.x & 63;
   const bool first_wave = NW == 1 || __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == 0;
@@ -90,9 +90,11 @@ k_cast_rays_pool(const DevModel* __restrict__ models, RayArgs a, int cap) {
             d2 = d2 + di[k] * di[k];
           }
           // the segment is no shorter than 2^-12 of its start's distance from the
-          // origin, holds both points, and lies where the network cannot overflow
+          // origin, holds both points, lies where the network cannot overflow, and its
+          // bound ends further from zero than bound and points round
           const float l2 = step * step * d2;
-          if (!(l2 >= 0x1p-24f * p2 && l2 <= 1e11f && p2 <= 1e11f && G.hit_eps >= 0.f && G.hit_eps <= step))
+          if (!(l2 >= 0x1p-24f * p2 && l2 <= 1e11f && p2 <= 1e11f && G.hit_eps >= 0.f && G.hit_eps <= step &&
+                s_near[pa] >= G.noise * fmaxf(1.f, sqrtf(p2) + sqrtf(l2))))
             phase &= ~kRaySure;
         }
       }
@@ -196,6 +198,7 @@ k_cast_rays_pool(const DevModel* __restrict__ models, RayArgs a, int cap) {
       const bool sure = code != CODE_UNKNOWN && scale <= 3.4028234663852886e38f &&
                         fminf(fabsf(lo), fabsf(hi)) >= 0.02f * scale;
       s_code[b] = code | (sure ? kRaySure : 0);
+      s_near[b] = fminf(fabsf(lo), fabsf(hi));
       s_val[b] = v[PT];
     });
     __syncthreads();

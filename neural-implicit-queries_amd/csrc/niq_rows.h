@@ -48,8 +48,8 @@ constexpr int kRowsPending = -1;
 // f's values in the box, so with one value below the offset and one above its
 // negative the code is UNKNOWN, whatever the mode; only the other boxes, listed for
 // k_classify_rows, need the bound.  The values must clear the thresholds by 2 % of
-// the largest and the box be no smaller than 2^-11 of its distance from the
-// origin, where float32 rounding of values and bound is far below that.  A box
+// the largest and by the rounding of this net (a.noise, see kNoiseRoom), and the box
+// be no smaller than 2^-11 of its distance from the origin.  A box
 // costs 8 points here (4, every other corner, at width 512, for LDS), about 1/50 of
 // its growing error terms, and in the trees of random nets two thirds of all boxes
 // are decided: the depth-18 affine_all tree of a 128x8 TanH net 54 -> 24 ms,
@@ -93,7 +93,7 @@ k_rows_signs(const DevModel* __restrict__ Mp, ClassifyArgs a, bool heap) {
         half = fmaxf(half, 0.5f * (up - lo));
         far = fmaxf(far, fmaxf(fabsf(lo), fabsf(up)));
       }
-      const float m = 0.02f * big;
+      const float m = fmaxf(0.02f * big, a.noise * fmaxf(1.f, far));
       const bool unknown = finite && far <= 1e6f && half >= far * 0x1p-11f && mn < a.offset - m && mx > m - a.offset;
       if (unknown) a.codes[i] = CODE_UNKNOWN;
       else if (heap) a.codes[i] = kRowsPending;

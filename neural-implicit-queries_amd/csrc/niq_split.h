@@ -2,7 +2,8 @@
 // instructions, for launches that ask for sign codes only.
 //
 // Every activation and weight is split into three bf16 terms that add up to it
-// exactly (x = x1 + x2 + x3: 8 bits of significand each, 24 in all), and a
+// exactly (x = x1 + x2 + x3: 8 bits of significand each, 24 in all; above 1e-33, below
+// which the third term leaves the range of normal numbers), and a
 // dense layer sums the six products down to 2^-18 of the largest,
 //     x3 w1 + x2 w2 + x1 w3 + x2 w1 + x1 w2 + x1 w1
 // (the three dropped ones are below 2^-26 |x w|, a quarter of half an ulp),
@@ -194,18 +195,24 @@ __device__ __forceinline__ void mlp_forward_split(const DevModelBf16& M, float* 
 
 // Classify axis-aligned boxes by the split contraction.  A box goes to the list
 // that k_classify then classifies when its bound lies within kSplitNear * (|base|
-// + radius) of the threshold, is not a number or is too small to judge by, or
-// when the box is smaller than 1/200 of its distance from the origin.
+// + radius) of the threshold or within the rounding of f (a.noise), is not a number
+// or is too small to judge by, or when the box is smaller than 1/200 of its
+// distance from the origin or than a.min_half = round_rel / kSplitRound.
 //
-// The band: the two forms' bounds differ by their rounding alone, which the
-// ReLU crossings amplify by (rounding of a pre-activation) / (its radius), the
-// more the smaller the box.  Largest difference over 131,072 random boxes each
-// of ReLU nets 256x3, 256x6 (He and Xavier) and 512x8, relative to |base| +
-// radius: 1e-6 at half-width 1/16, 1.3e-4 at 1/64, 5e-4 at 1/128; at 1/1000 it
-// reaches 0.2, so boxes that small take the plain kernel.  At 1/128 the band
-// holds 40 times that difference, and 1 % of the boxes of a shallow net (none of
-// a deep one's, whose bounds all span the threshold widely).
+// The band: the two forms' bounds differ by their rounding alone.  The rounding D of
+// a pre-activation moves its ReLU's chord, so the difference of two bounds relative to
+// |base| + radius is some D / r, r the pre-activation's radius over the box, and
+// round_rel / (half-width) estimates the largest D / r of the net's layers.
+// Measured with emulated float32 sums, 2,500 boxes each of 20 nets (He and Xavier,
+// 256x1 to 512x8, hidden biases up to 1e3 among them) at half-widths 1/16 to 1/200: the
+// largest difference is at most 5.6 times that estimate, and kSplitRound = 5e-4 keeps
+// it below 2.8e-3, a seventh of the band.  (On the card, 131,072 boxes each of He and
+// Xavier nets: 1.3e-4 at half-width 1/64, 5e-4 at 1/128.)  Nets without large biases have
+// round_rel below 2e-6 and reach the 1/200 first.  The band holds 1 % of the boxes of a
+// shallow net at half-width 1/128, none of a deep one's, whose bounds all span the
+// threshold widely.
 constexpr float kSplitNear = 2e-2f;
+constexpr float kSplitRound = 5e-4f;
 
 template <int V, int NB, int NW, int WMAX, int AS>
 __global__ void __launch_bounds__(NW * 64, 2)
@@ -232,9 +239,10 @@ k_classify_split(const DevModelBf16* __restrict__ Mp, ClassifyArgs a) {
       float lo, hi, scale;
       final_bounds<0, V>(v, lo, hi, scale);
       a.codes[i] = sign_code(lo, hi, a.offset);
-      const float tol = kSplitNear * scale;
+      const float far = fmaxf(1.f, cmax);
+      const float tol = fmaxf(kSplitNear * scale, a.noise * far);
       const bool clear = fabsf(lo - a.offset) > tol && fabsf(hi + a.offset) > tol && scale > 1e-20f &&
-                         scale < 1e30f && hmin >= kSplitMinSize * cmax;
+                         scale < 1e30f && hmin >= kSplitMinSize * cmax && hmin >= a.min_half * far;
       if (!clear) {
         const int slot = atomicAdd(a.list_n, 1);
         if (slot < a.list_cap) a.list[slot] = (int)i;
