@@ -222,10 +222,11 @@ niq_status cast_check(const niq_model* const* models, int n_models, const niq_ev
                       const int32_t* out_hit_id, const int32_t* out_count, int* wt, int* wt16,
                       bool allow_rows = true);
 // The pooled caster over groups of one model each (modes with a range form);
-// acts as in launch_rays.  *launched is false, and nothing was launched, where
-// k_cast_rays suits the cast better.  Defined in api_rays_pool.hip.
+// acts as in launch_rays.  loose: the nets' bounds exclude few tests.  *launched is
+// false, and nothing was launched, where k_cast_rays suits the cast better.  Defined
+// in api_rays_pool.hip.
 niq_status cast_pool(int mode, int wt, int variant, int acts, const DevModel* models, const RayArgs& a,
-                     long long n_rays, bool* launched, hipStream_t s);
+                     long long n_rays, bool loose, bool* launched, hipStream_t s);
 niq_status cast_run(const niq_model* const* models, int n_models, const niq_eval_cfg* cfg, const float* roots,
                     const float* dirs, int64_t n, const niq_cast_opts* o, float* out_t, int32_t* out_hit_id,
                     int32_t* out_count, unsigned char* base, int wt, int wt16, int64_t* n_evals, hipStream_t s);
