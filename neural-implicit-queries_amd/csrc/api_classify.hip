@@ -124,6 +124,13 @@ niq_status launch_classify(const niq_model* m, const ClassifyArgs& a, long long 
     if (m->tanh_only) return launch_classify_acts<KIND, V, ACTS_TANH>(m, a, max_n, s);
     if (m->elu_only) return launch_classify_acts<KIND, V, ACTS_ELU>(m, a, max_n, s);
   }
+  // Every rule in one kernel spills at width 256, and the spills' traffic evicts the weights
+  // that the re-test is about to read: there the tile of 16 waves, without spills (9,000 and
+  // 40,000 boxes of a 256x3 Sin net with the re-test 454 -> 350 and 926 -> 852 us; without
+  // it 248 and 243, 714 and 742).
+  if constexpr (KIND == 0 && V == 3)
+    if (variant == 0 && m->wt == 256 && a.recheck_tol > 0.f)
+      return launch_classify_w<KIND, V, 256, TileCfgWide<256>>(m, a, max_n, s);
   return launch_classify_acts<KIND, V, ACTS_ALL>(m, a, max_n, s);
 }
 

@@ -227,8 +227,10 @@ __device__ __forceinline__ void tanh_rule(T lo, T hi, T& a, T& b, T& d) {
   al = (hi > lo) ? al : dl;
   al = clip_t(nan_to_num_t(al), T(0), T(1));
   T xs = Fm<T>::atanh(Fm<T>::sqrt(T(1) - al));
-  // Each location clamps to itself, lo or hi, whose tanh is known (tanh is odd
-  // bit for bit), so the four values take one more tanh instead of four.
+  // Each location clamps to itself, lo or hi, whose tanh is known (tanhf is odd
+  // bit for bit), so the four values take one more tanh instead of four.  In double,
+  // where that was not checked, the FP64 re-test evaluates all four (and keeps the
+  // registers of three waves a SIMD).
   const T ts = Fm<T>::tanh(xs);
   const T locs[4] = {lo, hi, xs, -xs};
   const T tans[4] = {tl, tu, ts, -ts};
@@ -236,7 +238,9 @@ __device__ __forceinline__ void tanh_rule(T lo, T hi, T& a, T& b, T& d) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const T x = Fm<T>::min(Fm<T>::max(locs[i], lo), hi);
-    const T t = x == locs[i] ? tans[i] : (x == lo ? tl : tu);
+    T t;
+    if constexpr (sizeof(T) == 8) t = Fm<T>::tanh(x);
+    else t = x == locs[i] ? tans[i] : (x == lo ? tl : tu);
     const T v = t - al * x;
     rl = Fm<T>::min(rl, v); ru = Fm<T>::max(ru, v);
   }
