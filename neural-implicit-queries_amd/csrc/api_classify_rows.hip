@@ -32,11 +32,15 @@ niq_status launch_rows_w(const niq_model* m, const niq_eval_cfg* cfg, const Clas
   // whose rounding is not known).
   const bool signs = a.list && a.lower && a.d == 3 && !a.bounds && m->bounded &&
                      std::isfinite(m->round_rel) && max_n >= kRowsSignsMin;
-  // A tree's top levels in passes, where a box costs far more than a pass's latency:
-  // depth-18 affine_all tree of the 128x8 TanH net 24.0 -> 17.9 ms (3 passes 21.0,
-  // 8 passes 19.6), but the affine_all tree of a 32x4 net 0.99 -> 1.04, the
-  // affine_truncate tree of the 32x8 fox net 8.1 -> 8.9.
-  const bool heap = signs && a.heap && MODE == ROWS_ALL && W >= 128;
+  // A tree's top levels in passes, where a box costs far more than a pass's latency and
+  // the heap is many rounds of the resident workgroups: depth-18 affine_all tree of
+  // the 128x8 TanH net 24.0 -> 17.9 ms (3 passes 21.0, 8 passes 19.6), depth 11 (4,095
+  // nodes) of 256x4 TanH 7.7 -> 4.6, of 512x3 33 -> 14.7, of 256x6 ReLU, whose boxes are
+  // hardly ever certified, 13.7 -> 18.5 (22.3 without k_rows_signs).  With fewer nodes the
+  // passes' latency is the larger: depth 9 of 256x4 TanH 2.5 -> 4.4, of 256x6 ReLU
+  // 3.2 -> 9.5.  Nor at widths below 128 (affine_all tree of a 32x4 net 0.99 -> 1.04) or
+  // in the other modes (affine_truncate tree of the 32x8 fox net 8.1 -> 8.9).
+  const bool heap = signs && a.heap && MODE == ROWS_ALL && W >= 128 && max_n >= kRowsHeapMin;
   void* scratch = nullptr;
   HIPCHK(hipMallocAsync(&scratch, per_wg * g, s));
   RowsArgs ra{};

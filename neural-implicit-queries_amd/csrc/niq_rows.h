@@ -113,6 +113,7 @@ k_rows_signs(const DevModel* __restrict__ Mp, ClassifyArgs a, bool heap) {
 // nobody reads).  The rest are not reached, and their codes not read.  One
 // workgroup.  128x8 TanH net, 8191 nodes: 9.8 -> 3.8 ms.
 constexpr int kRowsHeapPasses = 5;
+constexpr int kRowsHeapMin = 4095;   // nodes of the heap from which the passes pay
 static __global__ void __launch_bounds__(1024) k_rows_heap_list(const int* codes, int n, bool last, int* list,
                                                                int* list_n) {
   if (threadIdx.x == 0) *list_n = 0;
