@@ -19,3 +19,33 @@ def pytest_configure(config):
 @pytest.fixture(scope="session")
 def golden_dir():
     return GOLDEN
+
+
+# Tests of the serving loop that need requests to wait in the queue together while
+# the only worker is busy.  The tree build that they keep it busy with takes a fraction
+# of a millisecond, less than a slow host needs for the next submits.
+HELD = {"test_merged_rays_equal_lone_casts", "test_rays_of_different_models_and_options_share_a_cast",
+        "test_tree_requests_merge_into_one_build", "test_batched_tree_overflow_fails_only_its_tree",
+        "test_casts_merge_however_slow_the_submits", "test_wide_trees_merge"}
+
+
+@pytest.fixture(autouse=True)
+def held_worker(request, monkeypatch):
+    """In these tests the first tree of a server is queued behind a closest-point
+    request of about a quarter of a second (some 10,000 dependent rounds)."""
+    if getattr(request.node, "originalname", None) not in HELD:
+        return
+    import numpy as np
+    from niq import implicit_mlp_utils, mlp, serve
+
+    submit_tree = serve.Server.submit_tree
+    params = mlp.load(os.path.join(GOLDEN, "fox.npz"))
+    func, _ = implicit_mlp_utils.implicit_from_params(params, "affine_fixed")
+    q = np.random.default_rng(3).uniform(-1, 1, size=(500, 3)).astype(np.float32)
+
+    def behind_a_long_request(self, *args, **kw):
+        if not hasattr(self, "_holding"):
+            self._holding = self.submit_closest_point(func, params, [-1.] * 3, [1.] * 3, q, eps=0.1)
+        return submit_tree(self, *args, **kw)
+
+    monkeypatch.setattr(serve.Server, "submit_tree", behind_a_long_request)
