@@ -79,8 +79,8 @@ bool same_cast(const Request& a, const Request& b) {
 
 // Tree requests that can share one batched build: the same eval config (its
 // tile variants aside: they change no result, and a batch runs the default
-// tile) and build params (root boxes aside), one width class, a batchable
-// form.
+// tile) and build params (root boxes aside), one width class, the same levels by
+// the split contraction, a batchable form.
 bool same_tree_batch(const Request& a, const Request& b) {
   if (a.kind != REQ_TREE || b.kind != REQ_TREE) return false;
   niq_eval_cfg ca = a.cfg, cb = b.cfg;
@@ -93,6 +93,7 @@ bool same_tree_batch(const Request& a, const Request& b) {
   return p.split_depth == q.split_depth && p.node_terminate_thresh == q.node_terminate_thresh &&
          p.batch_process_size == q.batch_process_size && p.with_interior_nodes == q.with_interior_nodes &&
          p.with_exterior_nodes == q.with_exterior_nodes && p.offset == q.offset &&
+         tree_split_levels(a.model, &a.cfg, &p) == tree_split_levels(b.model, &b.cfg, &q) &&
          tree_batchable(b.model, &b.cfg, &b.tp);
 }
 

@@ -1,5 +1,6 @@
 // Device-resident level-set tree build.
 #include "niq_internal.h"
+#include "niq_split.h"
 
 extern "C" {
 
@@ -26,10 +27,6 @@ int top_levels_for(const niq_eval_cfg* cfg, const niq_tree_params* p) {
   const int t = std::min(n_levels, kTopLevels);
   return t >= 3 ? t : 0;
 }
-
-// The deepest level whose boxes (1/128 of the root's sides) the split
-// contraction takes.
-constexpr int kSplitMaxLevel = 21;
 
 // Boxes per chunk of the layer-by-layer precision mode inside a tree build.
 constexpr long long kTreeLwChunk = 32768;
@@ -149,6 +146,8 @@ extern "C++" {   // templates below; the file's outer block has C linkage
 // tree of the batch shares, at its own base), root box and output lists.
 struct TreeItem {
   const DevModel* m;
+  const DevModelBf16* m16;      // split contraction: its weights, smallest box and noise (ClassifyArgs)
+  float min_half, noise;
   unsigned char* ws;
   float root[6];
   float* unk_lo; float* unk_up; long long cap_unk;
@@ -158,8 +157,9 @@ struct TreeItem {
 
 // Offsets of the shared layout, for the device.
 struct TreeOffs {
-  size_t counters, codes, bcnt, boff, lvl[2], top_box, top_codes;
+  size_t counters, codes, bcnt, boff, lvl[2], top_box, top_codes, list;
   long long cap;
+  int list_cap;
   int n_top, top_levels, with_int, with_ext;
 };
 
@@ -179,6 +179,7 @@ __global__ void k_tree_init_b(const TreeItem* __restrict__ items, TreeOffs o) {
 
 __global__ void k_top_boxes_b(const TreeItem* __restrict__ items, TreeOffs o) {
   const TreeItem& it = items[blockIdx.y];
+  if (blockIdx.x == 0 && threadIdx.x == 0) item_counters(it, o)->near_cnt = 0;
   float* lo = reinterpret_cast<float*>(it.ws + o.top_box);
   top_box_body(it.root, o.n_top, lo, lo + 3 * (size_t)o.n_top, blockIdx.x * blockDim.x + threadIdx.x + 1);
 }
@@ -237,25 +238,62 @@ __global__ void __launch_bounds__(256) k_tree_scatter_b(const TreeItem* __restri
 }
 
 // Tile offsets of one level over the trees of a batch: pref[g] = tiles (of nb
-// boxes) of the trees before g, pref[ng] = all.  level -1: the top launch.
+// boxes) of the trees before g, pref[ng] = all.  level -1: the top launch.  listed:
+// of the boxes that the split contraction left.
 __global__ void k_items_prefix(const TreeItem* __restrict__ items, int ng, TreeOffs o, int level, int nb,
-                               int* __restrict__ pref) {
+                               bool listed, int* __restrict__ pref) {
   if (threadIdx.x != 0) return;
   int acc = 0;
   for (int g = 0; g < ng; ++g) {
     pref[g] = acc;
-    const int n = level < 0 ? o.n_top : item_counters(items[g], o)->n[level & 1];
+    const TreeCounters* C = item_counters(items[g], o);
+    const int n = listed ? min(C->near_cnt, o.list_cap) : (level < 0 ? o.n_top : C->n[level & 1]);
     acc += (n + nb - 1) / nb;
   }
   pref[ng] = acc;
+}
+
+// Item g whose tiles hold tile t: the last one whose first tile is at or before t.
+__device__ __forceinline__ int item_of_tile(const int* __restrict__ pref, int ng, int t) {
+  int g = 0, hi = ng - 1;
+  while (g < hi) {
+    const int mid = (g + hi + 1) >> 1;
+    if (pref[mid] <= t) g = mid; else hi = mid - 1;
+  }
+  return g;
+}
+
+// The boxes of an item's level and where their codes go.
+__device__ __forceinline__ ClassifyArgs item_args(const TreeItem& it, const TreeOffs& o, int level, float offset) {
+  ClassifyArgs a{};
+  if (level < 0) {
+    a.lower = reinterpret_cast<const float*>(it.ws + o.top_box);
+    a.upper = a.lower + 3 * (size_t)o.n_top;
+    a.n = o.n_top;
+    a.codes = reinterpret_cast<int*>(it.ws + o.top_codes);
+  } else {
+    a.lower = item_lvl(it, o, level);
+    a.upper = a.lower + 3 * o.cap;
+    a.n = item_counters(it, o)->n[level & 1];
+    a.codes = reinterpret_cast<int*>(it.ws + o.codes);
+  }
+  a.d = 3;
+  a.offset = offset;
+  a.list = reinterpret_cast<int*>(it.ws + o.list);
+  a.list_n = &item_counters(it, o)->near_cnt;
+  a.list_cap = o.list_cap;
+  a.min_half = it.min_half;
+  a.noise = it.noise;
+  return a;
 }
 
 // The classify pass of one level of every tree of a batch in one launch: the
 // trees' tiles of NB boxes are numbered one tree after another (pref) and
 // workgroups walk them; each tile runs its own tree's model.  level -1 is the
 // launch over the top of the trees.  Every (box, feature) sums as in
-// k_classify: the codes are a lone build's bit for bit.
-template <int KIND, int V, int NB, int NW, int WMAX>
+// k_classify: the codes are a lone build's bit for bit.  LIST: only the boxes that
+// the split contraction left.
+template <int KIND, int V, int NB, int NW, int WMAX, bool LIST = false, int AS = ACTS_ALL>
 __global__ void __launch_bounds__(NW * 64, (LdsOcc<Planes<KIND, V, 0>::R, NB, NW, WMAX>::value))
 k_classify_items(const TreeItem* __restrict__ items, int ng, TreeOffs o, int level, float offset,
                  const int* __restrict__ pref) {
@@ -264,36 +302,34 @@ k_classify_items(const TreeItem* __restrict__ items, int ng, TreeOffs o, int lev
   __shared__ float X[PL::R * NB * WMAX];
   const int total = pref[ng];
   for (int t = blockIdx.x; t < total; t += gridDim.x) {
-    int g = 0, hi = ng - 1;   // the last tree whose first tile is at or before t
-    while (g < hi) {
-      const int mid = (g + hi + 1) >> 1;
-      if (pref[mid] <= t) g = mid; else hi = mid - 1;
-    }
-    const int first = pref[g];
+    const int g = item_of_tile(pref, ng, t);
     const TreeItem& it = items[g];
-    ClassifyArgs a{};
-    int* codes;
-    if (level < 0) {
-      a.lower = reinterpret_cast<const float*>(it.ws + o.top_box);
-      a.upper = a.lower + 3 * (size_t)o.n_top;
-      a.n = o.n_top;
-      codes = reinterpret_cast<int*>(it.ws + o.top_codes);
-    } else {
-      a.lower = item_lvl(it, o, level);
-      a.upper = a.lower + 3 * o.cap;
-      a.n = item_counters(it, o)->n[level & 1];
-      codes = reinterpret_cast<int*>(it.ws + o.codes);
-    }
-    a.d = 3;
-    const long long i0 = (long long)(t - first) * NB, n = a.n;
-    fill_box_inputs<KIND, V, NB, NT, WMAX>(X, a, i0, n);
-    mlp_forward<PL, KIND, V, NB, NW, WMAX>(*it.m, X, [&](const float* v, int b) {
-      const long long i = i0 + b;
+    const ClassifyArgs a = item_args(it, o, level, offset);
+    const long long i0 = (long long)(t - pref[g]) * NB, n = LIST ? (long long)min(*a.list_n, a.list_cap) : a.n;
+    fill_box_inputs<KIND, V, NB, NT, WMAX, LIST>(X, a, i0, n);
+    mlp_forward<PL, KIND, V, NB, NW, WMAX, AS>(*it.m, X, [&](const float* v, int b) {
+      long long i = i0 + b;
       if (i >= n) return;
+      if constexpr (LIST) i = a.list[i];
       float lo, hi2, scale;
       final_bounds<KIND, V>(v, lo, hi2, scale);
-      codes[i] = sign_code(lo, hi2, offset);
+      a.codes[i] = sign_code(lo, hi2, offset);
     });
+  }
+}
+
+// The same by the split contraction (k_classify_split's tiles).
+template <int NB, int NW, int WMAX>
+__global__ void __launch_bounds__(NW * 64, 2)
+k_classify_split_items(const TreeItem* __restrict__ items, int ng, TreeOffs o, int level, float offset,
+                       const int* __restrict__ pref) {
+  __shared__ float X[Planes<0, 3, 0>::R * NB * WMAX];
+  const int total = pref[ng];
+  for (int t = blockIdx.x; t < total; t += gridDim.x) {
+    const int g = item_of_tile(pref, ng, t);
+    const TreeItem& it = items[g];
+    const ClassifyArgs a = item_args(it, o, level, offset);
+    classify_split_tile<3, NB, NW, WMAX, ACTS_RELU>(*it.m16, a, X, (long long)(t - pref[g]) * NB, a.n);
   }
 }
 
@@ -304,7 +340,7 @@ niq_status launch_classify_items_w(const TreeItem* items, int ng, const TreeOffs
     return fail(NIQ_ERR_UNSUPPORTED, "batched tree build: planes above LDS");
   } else {
     constexpr int NB = TileCfg<W>::NB, NW = TileCfg<W>::NW;
-    hipLaunchKernelGGL(k_items_prefix, dim3(1), dim3(64), 0, s, items, ng, o, level, NB, pref);
+    hipLaunchKernelGGL(k_items_prefix, dim3(1), dim3(64), 0, s, items, ng, o, level, NB, false, pref);
     auto k = k_classify_items<KIND, V, NB, NW, W>;
     const long long max_tiles = (long long)ng * ((max_n + NB - 1) / NB);
     const unsigned g = tile_grid(max_tiles, persistent_blocks(k, NW * 64));
@@ -312,6 +348,26 @@ niq_status launch_classify_items_w(const TreeItem* items, int ng, const TreeOffs
     HIPCHK(hipGetLastError());
     return NIQ_OK;
   }
+}
+
+// A level of trees of wide ReLU nets by the split contraction, the boxes it leaves by
+// k_classify's forward, as classify_split.
+template <int W>
+niq_status launch_split_items(const TreeItem* items, int ng, const TreeOffs& o, int level, float offset,
+                              long long max_n, int* pref, hipStream_t s) {
+  constexpr int NB = SplitTile<W>::NB, NW = SplitTile<W>::NW, NWL = BoxTile<W>::NW;
+  static_assert(BoxTile<W>::NB == NB, "both passes number tiles of NB boxes");
+  const long long max_tiles = (long long)ng * ((max_n + NB - 1) / NB);
+  auto k = k_classify_split_items<NB, NW, W>;
+  auto kl = k_classify_items<0, 3, NB, NWL, W, true, ACTS_RELU>;
+  hipLaunchKernelGGL(k_items_prefix, dim3(1), dim3(64), 0, s, items, ng, o, level, NB, false, pref);
+  hipLaunchKernelGGL(k, dim3(tile_grid(max_tiles, persistent_blocks(k, NW * 64))), dim3(NW * 64), 0, s, items, ng, o,
+                     level, offset, pref);
+  hipLaunchKernelGGL(k_items_prefix, dim3(1), dim3(64), 0, s, items, ng, o, level, NB, true, pref);
+  hipLaunchKernelGGL(kl, dim3(grid_for(max_tiles, persistent_blocks(kl, NWL * 64))), dim3(NWL * 64), 0, s, items, ng, o,
+                     level, offset, pref);
+  HIPCHK(hipGetLastError());
+  return NIQ_OK;
 }
 
 // (KIND, V) of the fused classify of a config: 0 interval, 1 affine_fixed
@@ -398,21 +454,7 @@ niq_status tree_enqueue(const niq_model* m, const niq_eval_cfg* cfg, const niq_t
   int* top_codes = reinterpret_cast<int*>(base + L.off_top_codes);
   const int n_levels = p->split_depth >= 0 ? p->split_depth + 1 : 64;
   int level = 0;
-  // Levels whose boxes are large enough, beside the root's distance from the
-  // origin and the net's rounding, take the split contraction where the net is eligible (smaller boxes
-  // would all be listed for the plain one).
-  int split_levels = 0;
-  if (split_eligible(m, cfg)) {
-    float ext = INFINITY, far = 0.f;
-    for (int k = 0; k < 3; ++k) {
-      ext = std::min(ext, p->upper[k] - p->lower[k]);
-      far = std::max(far, std::max(std::fabs(p->lower[k]), std::fabs(p->upper[k])));
-    }
-    while (split_levels <= kSplitMaxLevel &&
-           0.5f * std::ldexp(ext, -(split_levels + 2) / 3) >=
-               std::max(far * kSplitMinSize, std::max(far, 1.f) * split_min_half(m)))
-      ++split_levels;
-  }
+  const int split_levels = tree_split_levels(m, cfg, p);
   auto classify = [&](ClassifyArgs a, long long max_n, int lv) -> niq_status {
     // room for the boxes that a first look leaves (the split contraction, or the
     // growing-row modes' corners); the FP64 re-test's, which neither path has
@@ -580,6 +622,23 @@ niq_status niq_tree_decode(const void* host_counters, const niq_tree_params* p, 
 
 namespace niqi {
 
+// The deepest level whose boxes (1/128 of the root's sides) the split
+// contraction takes.
+constexpr int kSplitMaxLevel = 21;
+
+int tree_split_levels(const niq_model* m, const niq_eval_cfg* cfg, const niq_tree_params* p) {
+  if (!m || !split_eligible(m, cfg)) return 0;
+  float ext = INFINITY, far = 0.f;
+  for (int k = 0; k < 3; ++k) {
+    ext = std::min(ext, p->upper[k] - p->lower[k]);
+    far = std::max(far, std::max(std::fabs(p->lower[k]), std::fabs(p->upper[k])));
+  }
+  const float half = std::max(far * kSplitMinSize, std::max(far, 1.f) * split_min_half(m));
+  int levels = 0;
+  while (levels <= kSplitMaxLevel && 0.5f * std::ldexp(ext, -(levels + 2) / 3) >= half) ++levels;
+  return p->split_depth >= 0 ? std::min(levels, p->split_depth + 1) : levels;
+}
+
 niq_status tree_enqueue_async(const niq_model* m, const niq_eval_cfg* cfg, const niq_tree_params* p, void* ws,
                               size_t ws_bytes, niq_tree_result* res, size_t* counters_offset, const float* root_dev,
                               void* stream) {
@@ -633,6 +692,13 @@ niq_status tree_batch_build(const niq_model* const* models, int ng, const niq_ev
       return fail(NIQ_ERR_INVALID, "exterior output buffers are required");
   }
   const int form = batch_form(cfg);
+  // levels by the split contraction: those that every tree's lone build runs so
+  int split_levels = INT_MAX;
+  for (int g = 0; g < ng; ++g) {
+    niq_tree_params pg = *p;
+    for (int k = 0; k < 3; ++k) { pg.lower[k] = roots[6 * g + k]; pg.upper[k] = roots[6 * g + 3 + k]; }
+    split_levels = std::min(split_levels, tree_split_levels(models[g], cfg, &pg));
+  }
   TreeLayout L;
   if (niq_status st = tree_layout(models[0], cfg, p, &L)) return st;
   size_t need = 0;
@@ -647,6 +713,9 @@ niq_status tree_batch_build(const niq_model* const* models, int ng, const niq_ev
     TreeItem& it = items[g];
     const niq_tree_result* r = res[g];
     it.m = models[g]->dev;
+    it.m16 = models[g]->dev16;
+    it.min_half = split_min_half(models[g]);
+    it.noise = kNoiseRoom * models[g]->round_out;
     it.ws = trees + L.total * (size_t)g;
     for (int k = 0; k < 6; ++k) it.root[k] = roots[6 * g + k];
     it.unk_lo = static_cast<float*>(r->unknown_lower); it.unk_up = static_cast<float*>(r->unknown_upper);
@@ -659,9 +728,11 @@ niq_status tree_batch_build(const niq_model* const* models, int ng, const niq_ev
   TreeOffs o{};
   o.counters = L.off_counters; o.codes = L.off_codes; o.bcnt = L.off_bcnt; o.boff = L.off_boff;
   o.lvl[0] = L.off_lvl[0]; o.lvl[1] = L.off_lvl[1]; o.top_box = L.off_top_box; o.top_codes = L.off_top_codes;
+  o.list = L.off_recheck;
   o.cap = L.cap;
   o.top_levels = L.top_levels;
   o.n_top = L.top_levels ? (1 << L.top_levels) - 1 : 0;
+  o.list_cap = (int)std::min<long long>(std::max<long long>(L.cap, o.n_top), INT_MAX);
   o.with_int = p->with_interior_nodes ? 1 : 0; o.with_ext = p->with_exterior_nodes ? 1 : 0;
   const int B = p->batch_process_size;
   const int n_levels = p->split_depth + 1;
@@ -672,6 +743,11 @@ niq_status tree_batch_build(const niq_model* const* models, int ng, const niq_ev
   };
   auto classify = [&](int level, long long max_n) {
     if (st != NIQ_OK) return;
+    if ((level < 0 ? o.top_levels - 1 : level) < split_levels) {   // (every model's width is 256, or 512)
+      st = wt == 256 ? launch_split_items<256>(d_items, ng, o, level, p->offset, max_n, d_pref, s)
+                     : launch_split_items<512>(d_items, ng, o, level, p->offset, max_n, d_pref, s);
+      return;
+    }
     switch (wt) {
       case 32: st = launch_classify_items<32>(form, d_items, ng, o, level, p->offset, max_n, d_pref, s); break;
       case 64: st = launch_classify_items<64>(form, d_items, ng, o, level, p->offset, max_n, d_pref, s); break;

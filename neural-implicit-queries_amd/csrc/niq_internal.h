@@ -174,6 +174,10 @@ niq_status rows_tile_shape(int variant, int wt, int* ch, int* nw, int* occ);
 // launches.  Each tree's outputs and counts equal its lone build's.
 constexpr int kMaxTreeBatch = 64;
 bool tree_batchable(const niq_model* m, const niq_eval_cfg* cfg, const niq_tree_params* p);
+// Levels of a build, from the top, whose boxes take the split contraction (smaller boxes
+// would all be listed for the plain one): large enough beside the root's distance from
+// the origin and the net's rounding.  0: none.
+int tree_split_levels(const niq_model* m, const niq_eval_cfg* cfg, const niq_tree_params* p);
 niq_status tree_batch_bytes(const niq_model* m, const niq_eval_cfg* cfg, const niq_tree_params* p, int ng,
                             size_t* bytes);
 // roots: 6 floats per tree (lower then upper); tree_status (nullable): each

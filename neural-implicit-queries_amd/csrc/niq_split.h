@@ -214,41 +214,46 @@ __device__ __forceinline__ void mlp_forward_split(const DevModelBf16& M, float* 
 constexpr float kSplitNear = 2e-2f;
 constexpr float kSplitRound = 5e-4f;
 
+// The tile of boxes i0 .. i0 + NB - 1 of n.
+template <int V, int NB, int NW, int WMAX, int AS>
+__device__ __forceinline__ void classify_split_tile(const DevModelBf16& M, const ClassifyArgs& a, float* X,
+                                                    long long i0, long long n) {
+  using PL = Planes<0, V, 0>;
+  constexpr int NT = NW * 64, R = PL::R;
+  fill_box_inputs<0, V, NB, NT, WMAX>(X, a, i0, n);
+  for (int e = threadIdx.x; e < R * NB * 16; e += NT)   // the chunk's upper half
+    X[xoff<NB, WMAX>(e / (NB * 16), (e / 16) % NB, 16 + (e & 15))] = 0.f;
+  mlp_forward_split<PL, 0, V, NB, NW, WMAX, AS>(M, X, [&](const float* v, int b) {
+    const long long i = i0 + b;
+    if (i >= n) return;
+    float hmin = INFINITY, cmax = 0.f;
+    for (int k = 0; k < a.d; ++k) {
+      const float l = a.lower[i * a.d + k], u = a.upper[i * a.d + k];
+      hmin = fminf(hmin, 0.5f * (u - l));
+      cmax = fmaxf(cmax, fmaxf(fabsf(l), fabsf(u)));
+    }
+    float lo, hi, scale;
+    final_bounds<0, V>(v, lo, hi, scale);
+    a.codes[i] = sign_code(lo, hi, a.offset);
+    const float far = fmaxf(1.f, cmax);
+    const float tol = fmaxf(kSplitNear * scale, a.noise * far);
+    const bool clear = fabsf(lo - a.offset) > tol && fabsf(hi + a.offset) > tol && scale > 1e-20f && scale < 1e30f &&
+                       hmin >= kSplitMinSize * cmax && hmin >= a.min_half * far;
+    if (!clear) {
+      const int slot = atomicAdd(a.list_n, 1);
+      if (slot < a.list_cap) a.list[slot] = (int)i;
+    }
+  });
+}
+
 template <int V, int NB, int NW, int WMAX, int AS>
 __global__ void __launch_bounds__(NW * 64, 2)
 k_classify_split(const DevModelBf16* __restrict__ Mp, ClassifyArgs a) {
-  using PL = Planes<0, V, 0>;
-  constexpr int NT = NW * 64, R = PL::R;
-  __shared__ float X[R * NB * WMAX];
+  __shared__ float X[Planes<0, V, 0>::R * NB * WMAX];
   const long long n = a.n_dev ? (long long)(*a.n_dev) : a.n;
   const long long ntiles = (n + NB - 1) / NB;
-  for (long long tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const long long i0 = tile * NB;
-    fill_box_inputs<0, V, NB, NT, WMAX>(X, a, i0, n);
-    for (int e = threadIdx.x; e < R * NB * 16; e += NT)   // the chunk's upper half
-      X[xoff<NB, WMAX>(e / (NB * 16), (e / 16) % NB, 16 + (e & 15))] = 0.f;
-    mlp_forward_split<PL, 0, V, NB, NW, WMAX, AS>(*Mp, X, [&](const float* v, int b) {
-      const long long i = i0 + b;
-      if (i >= n) return;
-      float hmin = INFINITY, cmax = 0.f;
-      for (int k = 0; k < a.d; ++k) {
-        const float l = a.lower[i * a.d + k], u = a.upper[i * a.d + k];
-        hmin = fminf(hmin, 0.5f * (u - l));
-        cmax = fmaxf(cmax, fmaxf(fabsf(l), fabsf(u)));
-      }
-      float lo, hi, scale;
-      final_bounds<0, V>(v, lo, hi, scale);
-      a.codes[i] = sign_code(lo, hi, a.offset);
-      const float far = fmaxf(1.f, cmax);
-      const float tol = fmaxf(kSplitNear * scale, a.noise * far);
-      const bool clear = fabsf(lo - a.offset) > tol && fabsf(hi + a.offset) > tol && scale > 1e-20f &&
-                         scale < 1e30f && hmin >= kSplitMinSize * cmax && hmin >= a.min_half * far;
-      if (!clear) {
-        const int slot = atomicAdd(a.list_n, 1);
-        if (slot < a.list_cap) a.list[slot] = (int)i;
-      }
-    });
-  }
+  for (long long tile = blockIdx.x; tile < ntiles; tile += gridDim.x)
+    classify_split_tile<V, NB, NW, WMAX, AS>(*Mp, a, X, tile * NB, n);
 }
 
 // Point values by the split contraction, for nets whose activations stay far
