@@ -106,6 +106,7 @@ struct TreeGraph {
   uint64_t model_serial = 0;
   niq_eval_cfg cfg{};
   int split_depth = 0, B = 0, with_int = 0, with_ext = 0;
+  int split_levels = 0;    // depends on the root box, which a replay may change
   float offset = 0.f;
   int64_t cap_unk = 0, cap_int = 0, cap_ext = 0;
   void* ws = nullptr;
@@ -119,7 +120,7 @@ struct TreeGraph {
 
   bool matches(const Request& r) const {
     return model_serial == r.model->serial && std::memcmp(&cfg, &r.cfg, sizeof(cfg)) == 0 && split_depth == r.tp.split_depth &&
-           B == r.tp.batch_process_size && with_int == r.tp.with_interior_nodes &&
+           split_levels == tree_split_levels(r.model, &r.cfg, &r.tp) && B == r.tp.batch_process_size && with_int == r.tp.with_interior_nodes &&
            with_ext == r.tp.with_exterior_nodes && offset == r.tp.offset && cap_unk == r.tres.unknown_capacity &&
            cap_int == (r.tp.with_interior_nodes ? r.tres.interior_capacity : 0) &&
            cap_ext == (r.tp.with_exterior_nodes ? r.tres.exterior_capacity : 0);
@@ -230,6 +231,7 @@ TreeGraph* Worker::graph_for(Request* r, bool* reused) {
   if (niq_tree_workspace_bytes(r->model, &r->cfg, &r->tp, &ws_bytes) != NIQ_OK) return nullptr;
   TreeGraph g;
   g.model_serial = r->model->serial; g.cfg = r->cfg; g.split_depth = r->tp.split_depth; g.B = r->tp.batch_process_size;
+  g.split_levels = tree_split_levels(r->model, &r->cfg, &r->tp);
   g.with_int = r->tp.with_interior_nodes; g.with_ext = r->tp.with_exterior_nodes; g.offset = r->tp.offset;
   g.cap_unk = r->tres.unknown_capacity;
   g.cap_int = g.with_int ? r->tres.interior_capacity : 0;

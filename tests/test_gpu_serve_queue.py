@@ -1,7 +1,7 @@
 """The serving loop's merging does not depend on how fast requests are submitted or
 how long a build takes, as long as they wait in the queue together; and merged builds
 of wide ReLU nets, whose levels run by the split contraction, equal lone builds bit for
-bit."""
+bit, also where a captured graph was first built for another root box."""
 import time
 
 import numpy as np
@@ -62,3 +62,23 @@ def test_wide_512_trees_merge():
         got = [r.result() for r in reqs]
     for a, g in zip(alone * 4, got):
         assert base.same_tree(a, g)
+
+
+@pytest.mark.parametrize("first", ["near", "far"])
+def test_graph_of_a_near_root_is_not_a_far_roots(first):
+    """A cached graph holds the levels that take the split contraction, which the root
+    box decides: near and far roots keep a graph each, and both are lone builds."""
+    p = models.random_mlp([256, 256], seed=1)
+    f, _ = implicit_mlp_utils.implicit_from_params(p, "affine_fixed")
+    kw = dict(split_depth=13, with_interior_nodes=True, with_exterior_nodes=True)
+    roots = {"near": (LO, UP), "far": FAR, "half": (LO, 0.5 * UP)}
+    alone = {k: kd_tree.construct_uniform_unknown_levelset_tree(f, p, *r, **kw) for k, r in roots.items()}
+    order = ["near", "far"] if first == "near" else ["far", "near"]
+    reused = {}
+    with serve.Server(n_streams=1) as srv:
+        for k in order + ["half", "far", "near"]:
+            r = srv.submit_tree(f, p, *roots[k], **kw)   # one at a time: never merged
+            assert base.same_tree(alone[k], r.result()), k
+            reused.setdefault(k, []).append(r.info["graph_reused"])
+    # the second of near and far is captured anew; near's graph serves another near root
+    assert reused["near"] == [False, True] and reused["far"] == [False, True] and reused["half"] == [True]
