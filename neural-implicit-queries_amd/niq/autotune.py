@@ -3,8 +3,11 @@
 The search space is the kernels' tile shapes, each a compiled variant:
 
 * plain FP32 classify (interval and affine_fixed over 3 box vectors),
-  ``EvalCfg.variant``: 1 the default tile (``BoxTile``: 16 boxes, 64 at
-  width 32, 4-8 waves, the register budget LDS occupancy allows), 2 twice
+  ``EvalCfg.variant``: 0 the default, with the forms that only it takes (the
+  narrowest width tile for small launches, the split contraction of wide ReLU
+  nets' trees, the fused frustum and closest-point rounds), 1 its tile
+  (``BoxTile``: 16 boxes, 64 at width 32, 4-8 waves, the register budget LDS
+  occupancy allows) for every launch, 2 twice
   the boxes per workgroup where LDS allows (fewer waves at width 512), 3 the
   default tile with a 256-register budget (no spills, fewer resident
   workgroups), 4 16 boxes with the most waves (the narrowest width tile: the
@@ -29,7 +32,9 @@ chunks and the ray tiles sum every (box, feature) in the same order
 same splits (the e-plane bound differs by at most 2^-15 relative) and
 variant 3 repeats variant 2's arithmetic exactly.  ``tune`` times the
 classify variants on boxes of the size of the finest tree cells of
-``split_depth``; ``tune_rays`` times the ray variants on a camera's rays.
+``split_depth``, and leaves a plain FP32 form on variant 0 unless the fastest
+one also builds a tree in less time; ``tune_rays`` times the ray variants on a
+camera's rays.
 Both keep the fastest in the function's config and cache the choice per
 (layer widths, activations, mode, precision).
 """
@@ -41,7 +46,7 @@ import torch
 from . import _lib
 from . import mlp as _mlp
 
-VARIANTS = (1, 2, 3, 4)
+VARIANTS = (0, 1, 2, 3, 4)
 VARIANTS_ROWS = (1, 2, 3)
 VARIANTS_BF16 = (1, 2, 3)
 RAY_VARIANTS = (0, 1, 2)
@@ -87,10 +92,30 @@ def _time(fn, reps):
     return e0.elapsed_time(e1) / reps
 
 
+def _against_default(func, params, best, times, depth, reps, res):
+    """``best`` where it is 2 % faster than variant 0 on the boxes and faster in a
+    tree build, else 0: boxes alone do not show what only variant 0 runs (a depth-18
+    tree of a 256x6 ReLU net takes 8.7 ms by the split contraction, 14.2 without).
+    Nets of width 32 keep 0, whose frustum casts take one launch an iteration (a 768^2
+    image of a 32x8 net 23.6 ms, 27.1 otherwise)."""
+    from . import kd_tree
+    width = max(_mlp.device_model(params).dims)
+    if times[best] > 0.98 * times[0] or width <= 32:
+        return 0
+    lo, up = np.full(3, -1.0, np.float32), np.full(3, 1.0, np.float32)
+    ms = {}
+    for v in (0, best):
+        func.cfg.variant = v
+        ms[v] = _time(lambda: kd_tree.build_tree(func, params, lo, up, split_depth=depth), reps)
+    res["tree_ms"] = ms
+    return best if ms[best] < ms[0] else 0
+
+
 def tune(func, params, split_depth=18, n_boxes=1 << 17, reps=3, seed=0):
     """Time every classify variant of ``func`` on ``n_boxes`` random cells of
     half-width 2^-(split_depth/3) in [-1, 1]^3; set the fastest and return
-    {"best", "ms": {variant: ms}, "shape"}."""
+    {"best", "ms": {variant: ms}, "shape"}.  Variant 0 stays where no other is
+    2 % faster on the boxes and faster in a tree build (``"tree_ms"``)."""
     key = _key(func, params)
     if key in _cache:
         func.cfg.variant = _cache[key]["best"]
@@ -101,14 +126,15 @@ def tune(func, params, split_depth=18, n_boxes=1 << 17, reps=3, seed=0):
     lo = torch.as_tensor((c - h).astype(np.float32), device="cuda")
     up = torch.as_tensor((c + h).astype(np.float32), device="cuda")
     times = {}
-    saved = func.cfg.variant
     for v in variants_of(func):
         func.cfg.variant = v
         times[v] = _time(lambda: func.classify_box(params, lo, up), reps)
-    func.cfg.variant = saved
     best = min(times, key=times.get)
+    res = {"ms": times, "n_boxes": n_boxes}
+    if 0 in times and best != 0:
+        best = _against_default(func, params, best, times, min(split_depth, 18), reps, res)
     func.cfg.variant = best
-    res = {"best": best, "ms": times, "n_boxes": n_boxes}
+    res["best"] = best
     if int(func.cfg.precision) == 0:
         kernel = "rows" if int(func.cfg.mode) in ROWS_MODES else "classify"
         res["shape"] = tile_shape(kernel, best, max(_mlp.device_model(params).dims))
