@@ -284,7 +284,8 @@ niq_status cast_run_groups(CastGroupReq* reqs, int ng, const niq_eval_cfg* cfg, 
     G.iter_hist = reinterpret_cast<int*>(base + L.hist[g]);
     G.lipschitz = cfg ? cfg->sdf_lipschitz : 1.f;
     G.stride = claim_stride(r.n, wt);
-    G.noise = kNoiseRoom * r.models[0]->round_out;
+    const float noise = kNoiseRoom * r.models[0]->round_out;
+    G.noise2 = noise * noise;
     hg[g] = G;
     m0 += r.n_models;
     n_rays += r.n;

@@ -796,8 +796,8 @@ struct RayGroup {
   unsigned long long* next_ray;  // work counter, zero on entry
   int* iter_hist;          // (n_max_step + 2,) rays by iterations lived, nullable
   float lipschitz;         // weak-SDF form (KIND 2): Lipschitz bound of f
-  float noise;             // pooled caster: least distance of a bound from zero that excludes a
-                           //   hit without a test, at coordinates up to 1
+  float noise2;            // pooled caster: square of the least distance of a bound from zero that
+                           //   excludes a hit without a test, at coordinates up to 1
   long long stride;        // claim k is ray k * stride mod n (coprime with n; pooled caster)
 };
 

@@ -91,10 +91,11 @@ k_cast_rays_pool(const DevModel* __restrict__ models, RayArgs a, int cap) {
           }
           // the segment is no shorter than 2^-12 of its start's distance from the
           // origin, holds both points, lies where the network cannot overflow, and its
-          // bound ends further from zero than bound and points round
-          const float l2 = step * step * d2;
+          // bound ends further from zero than bound and points round ((|p| + l)^2 is at
+          // most 2 (p2 + l2))
+          const float l2 = step * step * d2, near = s_near[pa];
           if (!(l2 >= 0x1p-24f * p2 && l2 <= 1e11f && p2 <= 1e11f && G.hit_eps >= 0.f && G.hit_eps <= step &&
-                s_near[pa] >= G.noise * fmaxf(1.f, sqrtf(p2) + sqrtf(l2))))
+                near * near >= G.noise2 * fmaxf(1.f, 2.f * (p2 + l2))))
             phase &= ~kRaySure;
         }
       }
