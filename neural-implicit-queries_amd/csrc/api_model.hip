@@ -183,13 +183,16 @@ niq_status niq_model_create(int n_layers, const int* dims, const int* acts, cons
   }
   // largest magnitude a layer's sum can take on inputs up to 1e6
   double mag = 1e6;
+  std::vector<double> sums;
   for (int i = 0; i < n_layers; ++i) {
+    const int nf = dims[i + 1];
+    sums.assign(nf, 0.0);
+    for (int f = 0; f < nf; ++f)
+      if (b && b[i]) sums[f] = std::fabs((double)b[i][f]);
+    for (int k = 0; k < dims[i]; ++k)
+      for (int f = 0; f < nf; ++f) sums[f] += mag * std::fabs((double)W[i][(size_t)k * nf + f]);
     double next = 0.0;
-    for (int f = 0; f < dims[i + 1]; ++f) {
-      double sum = (b && b[i]) ? std::fabs((double)b[i][f]) : 0.0;
-      for (int k = 0; k < dims[i]; ++k) sum += mag * std::fabs((double)W[i][(size_t)k * dims[i + 1] + f]);
-      next = std::isnan(sum) ? INFINITY : std::max(next, sum);
-    }
+    for (double sum : sums) next = std::isnan(sum) ? INFINITY : std::max(next, sum);
     mag = std::max(next, 1.0);   // (and activations of magnitude 1)
   }
   m->bounded = mag < 1e30;
