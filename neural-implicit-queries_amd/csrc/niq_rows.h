@@ -130,8 +130,10 @@ static __global__ void __launch_bounds__(1024) k_rows_heap_list(const int* codes
   }
 }
 
-// Block-wide argmax over n values (largest first, lowest index on ties);
-// every thread gets the result.  `sv`/`si` are 2 * NT scratch entries.
+// Block-wide argmax over n values (largest first, lowest index on ties), at least one
+// of them not taken; every thread gets the result.  `sv`/`si` are 2 * NT scratch entries.
+// NaN ranks last: the result indexes weights, so a box whose values are all NaN gets one
+// of them too.
 template <int NT>
 __device__ __forceinline__ int block_argmax(const float* vals, const unsigned char* taken, int n, float* sv, int* si,
                                             float& best) {
@@ -139,7 +141,7 @@ __device__ __forceinline__ int block_argmax(const float* vals, const unsigned ch
   int bi = 0x7fffffff;
   for (int k = threadIdx.x; k < n; k += NT) {
     if (taken[k]) continue;
-    const float v = vals[k];
+    const float v = vals[k] == vals[k] ? vals[k] : -INFINITY;
     if (v > bv || (v == bv && k < bi)) { bv = v; bi = k; }
   }
   sv[threadIdx.x] = bv; si[threadIdx.x] = bi;
