@@ -191,7 +191,7 @@ k_classify_rows(const DevModel* __restrict__ Mp, RowsArgs ra) {
   __shared__ float s_rv[NT];
   __shared__ float s_pe[NT];
   __shared__ int s_ri[NT];
-  __shared__ int s_keep[64];
+  __shared__ int s_keep[MODE == ROWS_APPEND ? WMAX : 64];   // at most n_append or n_keep
   const ClassifyArgs& a = ra.c;
   const DevModel& M = *Mp;
   const int lane = threadIdx.x & 63;
@@ -479,10 +479,10 @@ k_classify_rows(const DevModel* __restrict__ Mp, RowsArgs ra) {
         const float extra = s_rv[0];
         for (int f = threadIdx.x; f < Ly.out_pad; f += NT) s_err[f] = s_err[f] + extra;
         __syncthreads();
-        if (threadIdx.x < na) {
-          const int k = s_keep[threadIdx.x];
-          s_idx[threadIdx.x] = k;
-          s_scale[threadIdx.x] = s_mag[k];
+        for (int r = threadIdx.x; r < na; r += NT) {
+          const int k = s_keep[r];
+          s_idx[r] = k;
+          s_scale[r] = s_mag[k];
         }
         n_new = na;
         cur ^= 1;
