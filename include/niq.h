@@ -75,7 +75,12 @@ typedef struct niq_eval_cfg {
                           registers where a layer does not fill the
                           template (the default), 3 layer by layer; closest
                           point runs its round as one forward launch only at
-                          variant 0.  Every variant gives the same results. */
+                          variant 0, frustum casts of 32-wide nets an iteration.
+                          Every variant gives the same results.  (Trees of wide
+                          ReLU nets run another contraction at variants 0 and 1,
+                          and again by the plain one the boxes whose bound lies
+                          within several times its rounding, as estimated for
+                          the net, of the threshold.) */
   float sdf_lipschitz; /* NIQ_MODE_SDF: Lipschitz bound of f (sdf_lipschitz kwarg) */
   int ray_variant;     /* cast_rays tile shape, 0 = default; 1 and 2 are the
                           alternatives the autotuner times (same results) */
@@ -402,11 +407,12 @@ niq_status niq_shade_image(const niq_shade_opts* opts, const float* ray_dirs, co
  * every ray is independent, so merged results (N_evals included) equal lone
  * ones bit for bit.  Tree builds in the fused-kernel FP32 modes with a
  * split_depth that wait in the queue with the same eval config, build params
- * (root boxes aside) and template width (as above) are merged too (up to 64): one build
+ * (root boxes aside), template width (as above) and levels on the wide ReLU
+ * nets' contraction are merged too (up to 64): one build
  * runs every level of all of them in shared launches, each tree's level as
  * its lone build runs it, so the outputs are a lone build's bit for bit.  A
  * tree build taken alone replays a hipGraph captured once per (model,
- * config, depth, capacities) and shared by the workers (a graph replays on
+ * config, depth, levels on that contraction, capacities) and shared by the workers (a graph replays on
  * one stream at a time).  Closest-point batches run as they are.
  *
  * Buffers: inputs must be complete on the device when submitted and stay

@@ -170,8 +170,8 @@ inline niq_status check_model(const niq_model* m, int d) {
 niq_status rows_tile_shape(int variant, int wt, int* ch, int* nw, int* occ);
 // Batched level-set trees (the serving loop's merged builds): up to
 // kMaxTreeBatch trees with one eval config, one set of params (their root
-// boxes aside) and one template width, built level by level in shared
-// launches.  Each tree's outputs and counts equal its lone build's.
+// boxes aside), one template width and the same levels on the split contraction
+// (tree_split_levels), built level by level in shared launches.  Each tree's outputs and counts equal its lone build's.
 constexpr int kMaxTreeBatch = 64;
 bool tree_batchable(const niq_model* m, const niq_eval_cfg* cfg, const niq_tree_params* p);
 // Levels of a build, from the top, whose boxes take the split contraction (smaller boxes
@@ -199,7 +199,8 @@ niq_status classify_rows(const niq_model* m, const niq_eval_cfg* cfg, const Clas
                          hipStream_t s);
 // Sign codes of axis-aligned boxes (a.list, a.list_n set; no bounds, no FP64
 // re-test) by the split contraction, the boxes near the threshold by k_classify:
-// the codes of classify_dispatch, faster on wide ReLU nets.  Needs
+// the codes of classify_dispatch where the two forwards differ by less than that band
+// (kSplitNear), faster on wide ReLU nets.  Needs
 // split_eligible(m, cfg).  Defined in api_classify_split.hip.
 bool split_eligible(const niq_model* m, const niq_eval_cfg* cfg);
 niq_status classify_split(const niq_model* m, ClassifyArgs a, long long max_n, hipStream_t s);

@@ -15,7 +15,8 @@
 //
 // The sums round differently from k_classify's, so a box whose bound lies near
 // the threshold is listed and classified again by k_classify's own forward:
-// the codes are the plain kernel's.
+// the codes are the plain kernel's where the difference stays within that band, whose
+// width and limits are measured (kSplitNear).
 #pragma once
 #include "niq_bf16.h"
 

@@ -10,10 +10,10 @@ inside the library, each with its own HIP stream:
 * continuous batching: ray requests waiting with the same models, config and
   cast options are merged into the cast of the request taken;
 * tree builds with a ``split_depth`` in the fused-kernel modes that wait in the
-  queue together (same config, depth and template width, any models) run as
-  one batched build, every level of all of them in shared launches; a lone
-  one replays a hipGraph captured once per (model, config, depth,
-  capacities), shared by the workers;
+  queue together (same config, depth, template width and levels on the wide ReLU
+  nets' contraction, any models) run as one batched build, every level of all of
+  them in shared launches; a lone one replays a hipGraph captured once per (model,
+  config, depth, those levels, capacities), shared by the workers;
 * every request reports its queueing time and latency.
 
 Each result equals the result of the matching standalone call
